@@ -808,6 +808,39 @@ __global__ __launch_bounds__(64 * KW, (MI * NI == 1 && KW == 8 && DEPTH == 0) ? 
     else conv_tile<MI, NI, KW, TAP_MAJOR, kPreNone, DEPTH>(p, blockIdx.x);
 }
 
+#include "conv_small.h"
+
+constexpr int kSmallWaves = 8;  // sixteen: 1 % less over the layers with 16 parts, 20 % more over those with 8
+
+template <int MI>
+__global__ __launch_bounds__(64 * kSmallWaves) void conv_small_kernel(SmallArgs args) {
+    int idx = 0;  // see conv_mfma_kernel
+    asm volatile("" : "+s"(idx));
+    const SmallArgs& p = (&args)[idx];
+    if (p.pointwise) conv_small_tile<MI, kSmallWaves, true>(p, blockIdx.x);
+    else conv_small_tile<MI, kSmallWaves, false>(p, blockIdx.x);
+}
+
+struct SmallPreArgs {
+    SmallArgs conv;
+    PreOp pre;
+};
+
+template <int MI>
+__global__ __launch_bounds__(64 * kSmallWaves) void conv_small_pre_kernel(SmallPreArgs args) {
+    int idx = 0;  // see conv_mfma_kernel
+    asm volatile("" : "+s"(idx));
+    const SmallPreArgs& a = (&args)[idx];
+    const bool bounded = a.pre.lo > -__builtin_inff();
+    if (a.conv.pointwise) {
+        if (bounded) conv_small_tile<MI, kSmallWaves, true, kPreBounded>(a.conv, blockIdx.x, a.pre);
+        else conv_small_tile<MI, kSmallWaves, true, kPreUnbounded>(a.conv, blockIdx.x, a.pre);
+    } else {
+        if (bounded) conv_small_tile<MI, kSmallWaves, false, kPreBounded>(a.conv, blockIdx.x, a.pre);
+        else conv_small_tile<MI, kSmallWaves, false, kPreUnbounded>(a.conv, blockIdx.x, a.pre);
+    }
+}
+
 // A conv that applies a per-channel transform to its input on the way (smallest tile, tap-major order).
 struct ConvPreArgs {
     ConvArgs conv;
@@ -916,6 +949,34 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_group_kern
 }
 
 constexpr int kMaxGroupWithPool = 3;  // convs of one call that also carries a pooling operator
+
+// Independent convs of one call on 16-row tiles, and the pooling operator that may ride with them.
+struct SmallGroupArgs {
+    unsigned start[kMaxGroup];  // first workgroup id of each conv, multiples of eight; 0xFFFFFFFF for unused entries
+    unsigned pool_start;        // 0xFFFFFFFF without a pool
+    SmallArgs m[kMaxGroup];
+    paella::PoolArgs pool;
+};
+
+template <int MI>
+__global__ __launch_bounds__(64 * kSmallWaves) void conv_small_group_kernel(SmallGroupArgs g) {
+    if (blockIdx.x >= g.pool_start) {
+        paella::pool_element(g.pool, (int)((blockIdx.x - g.pool_start) * (64 * kSmallWaves) + threadIdx.x));
+        return;
+    }
+    int idx = 0;
+    unsigned first = g.start[0];
+#pragma unroll
+    for (int i = 1; i < kMaxGroup; ++i)
+        if (blockIdx.x >= g.start[i]) {
+            idx = i;
+            first = g.start[i];
+        }
+    const SmallArgs& p = g.m[idx];
+    const unsigned bid = blockIdx.x - first;
+    if (p.pointwise) conv_small_tile<MI, kSmallWaves, true>(p, bid);
+    else conv_small_tile<MI, kSmallWaves, false>(p, bid);
+}
 
 // ---------------------------------------------------------------------------------------------------
 // Depthwise conv (groups == C == K): HBM-bound, one thread per output pixel, taps from L1/L2.
@@ -1186,6 +1247,35 @@ ConvKernel pick_kernel(int mi, int ni, int kw, int k_order = 0, int depth = 0) {
 
 constexpr size_t kMaxSplitTiles = 16384;  // counters at the head of a split-k workspace
 
+// Which form a launch without a notifier takes when it is not packed with others (conv_small.h), for the convs of one call: tiles
+// of 16 channels x 16 pixels where that makes at most one workgroup per compute unit, else 32 x 16 where that does, else (0) the
+// plan's own kernel.  Measured over the 251 different conv layers of the zoo, one launch at a time with weights and input not in
+// the L2 (sum of their times, each as often as it occurs): 3507 us with the 32 x 32 kernel, 3265 us with this rule, 3262 us with
+// the fastest form picked for each layer.  Pointwise 768->192 on 17x17 6.1 -> 4.6 us, 512->128 with input transform on 14x14
+// 5.7 -> 4.4, 1x7 160->192 on 17x17 8.3 -> 5.9.
+// Where the lines lie: a second workgroup on a compute unit shares its vector cache, which already delivers twice the bytes per
+// matrix instruction that it does for a 32 x 32 tile (64->64 3x3 on 56x56, 784 workgroups: 5.8 -> 8.5 us); beyond 16 parts (8 of
+// the larger tile) the waves' turns from part to part cost more than the exchange through memory (256->256 3x3 on 14x14, 32
+// parts: 8.1 -> 10.6 us); long reductions are bound by the same vector cache; and the larger tile does not pay for a
+// reduction of one chunk per wave (64->384 pointwise on 14x14: 3.0 -> 3.2 us).
+int choose_small(const paella_conv_plan* const* plans, int n) {
+    long tiles1 = 0, tiles2 = 0, chunks = 0;
+    int parts = 0, shortest = 1 << 30;
+    for (int i = 0; i < n; ++i) {
+        const paella_conv_plan& p = *plans[i];
+        if (p.kind != 0 || p.mi != 1 || p.ni != 1 || p.k_order != 1 || p.depth != 0) return 0;
+        const long tiles_n = ((long)p.P * p.Q + 15) / 16, t1 = tiles_n * ((p.d.K + 15) / 16);
+        tiles1 += t1;
+        tiles2 += tiles_n * ((p.d.K + 31) / 32);
+        chunks += t1 * (p.k_pad / 8);  // what the compute units' vector caches have to deliver, in units of 1 KB
+        parts = std::max(parts, p.splits * p.kw);
+        shortest = std::min(shortest, p.k_pad / 8);
+    }
+    if (tiles1 <= 256 && parts <= 16 && chunks <= 150 * 256) return 1;
+    if (tiles2 <= 256 && parts <= 8 && chunks <= 300 * 256 && shortest >= 16) return 2;
+    return 0;
+}
+
 int conv_out(int in, int k, int stride, int pad, int dil) { return (in + 2 * pad - dil * (k - 1) - 1) / stride + 1; }
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
@@ -1321,6 +1411,7 @@ extern "C" int paella_conv2d_plan(const paella_conv_desc* d, int has_residual, i
             if (plan->dims.lds_bytes > 160 * 1024) return PAELLA_ENOSUP;  // table does not fit the CU's LDS
         }
         plan->dims.vgprs = 128;
+        if (tile_hint == 0 || (tile_hint >> 20 & 1)) plan->small = 1;
         return 0;
     }
     if (d->groups == d->C && d->K == d->C) {
@@ -1423,6 +1514,46 @@ int fill_args(const paella_conv_plan* plan, const float* x, const void* blob_dev
     a.pair_s0 = plan->pair_taps - 1;
     return 0;
 }
+
+// The form (rows of 16 channels per tile) that a launch of these convs takes on 16-row tiles, or 0: one that reports to a notifier
+// counts the plan's workgroups, and divisions there is no shortcut for are left to the other kernel.
+int small_form(const paella_conv_plan* const* plans, const ConvArgs* const* args, int n) {
+    for (int i = 0; i < n; ++i)
+        if (!plans[i]->small || args[i]->notifier || !args[i]->fast_div) return 0;
+    if (n == 1 && plans[0]->small > 1) return plans[0]->small - 1;
+    return choose_small(plans, n);
+}
+
+unsigned small_lds(const paella_conv_plan* plan, int mi) { return (unsigned)(plan->splits * plan->kw * mi * 4 * 256); }
+
+// Kernel arguments of that form, from those of the plan's own kernel; false where its divisions have no shortcut.
+bool fill_small(const paella_conv_plan* plan, const ConvArgs& a, int mi, SmallArgs& s, unsigned* grid) {
+    s.x = a.x; s.wpk = a.wpk; s.bias = a.bias; s.residual = a.residual; s.slope = a.act == PAELLA_ACT_PRELU ? a.slope : nullptr; s.y = a.y;
+    s.H = a.H; s.W = a.W; s.Q = a.Q; s.PQ = a.PQ; s.sh = a.sh; s.sw = a.sw; s.ph = a.ph; s.pw = a.pw;
+    s.K = a.K; s.m_pad = a.m_pad; s.nchunks = a.nchunks; s.S = a.S; s.dh = a.dh; s.dw = a.dw; s.CB = a.CB;
+    s.x_bytes = a.x_bytes; s.w_bytes = a.w_bytes;
+    s.n_tiles_n = (a.PQ + 15) / 16;
+    s.n_tiles_m = (a.K + 16 * mi - 1) / (16 * mi);
+    s.slab_major = a.slab_major; s.pointwise = a.pointwise; s.pair_s0 = a.pair_s0;
+    s.parts = plan->splits * plan->kw;
+    s.kw_log = 0;
+    while ((1 << s.kw_log) < plan->kw) ++s.kw_log;
+    s.chunks_per_split = a.chunks_per_split;
+    s.act = a.act; s.lo = a.lo; s.hi = a.hi;
+    const unsigned d_w = s.slab_major ? (unsigned)s.n_tiles_n : (unsigned)s.n_tiles_m;
+    const uint64_t total = (uint64_t)s.n_tiles_n * s.n_tiles_m;
+    if (total * d_w >= ((uint64_t)1 << 32) || (uint64_t)s.n_tiles_n * 16 * s.Q >= ((uint64_t)1 << 32)) return false;
+    s.div_w = fast_div(d_w);
+    s.div_q = a.div_q; s.div_cb = a.div_cb; s.div_s = a.div_s;
+    *grid = (unsigned)total;
+    return true;
+}
+
+typedef void (*ConvSmallKernel)(SmallArgs);
+typedef void (*ConvSmallPreKernel)(SmallPreArgs);
+
+ConvSmallKernel pick_small(int mi) { return mi == 1 ? conv_small_kernel<1> : mi == 2 ? conv_small_kernel<2> : nullptr; }
+ConvSmallPreKernel pick_small_pre(int mi) { return mi == 1 ? conv_small_pre_kernel<1> : mi == 2 ? conv_small_pre_kernel<2> : nullptr; }
 
 int allow_lds(const void* kern, unsigned lds_bytes) {
     if (lds_bytes <= 65536) return 0;
@@ -1960,6 +2091,41 @@ extern "C" int paella_pack_stats(uint64_t* launches, uint64_t* members) {
     return g_pack.held;
 }
 
+namespace {
+
+// The members of a group call on 16-row tiles, if all of them have that form.  Returns 1 when launched, 0 when not, else an error.
+int launch_small_group(const paella_conv_plan* const* plans, const ConvArgs* args, int n, const paella::PoolArgs* pool, void* stream) {
+    const ConvArgs* each[kMaxGroup];
+    for (int i = 0; i < n; ++i) each[i] = args + i;
+    const int mi = small_form(plans, each, n);
+    if (!mi) return 0;
+    SmallGroupArgs g;
+    unsigned next = 0, lds = 0;
+    for (int i = 0; i < n; ++i) {
+        unsigned grid = 0;
+        if (!fill_small(plans[i], args[i], mi, g.m[i], &grid)) return 0;
+        next = align_start(next);
+        g.start[i] = next;
+        next += grid;
+        lds = std::max(lds, small_lds(plans[i], mi));
+    }
+    for (int i = n; i < kMaxGroup; ++i) g.start[i] = 0xFFFFFFFFu;
+    g.pool_start = 0xFFFFFFFFu;
+    if (pool) {
+        constexpr unsigned block = 64u * kSmallWaves;
+        g.pool = *pool;
+        g.pool_start = next;
+        next += (unsigned)(((size_t)pool->C * pool->P * pool->Q + block - 1) / block);
+    }
+    auto kern = mi == 1 ? conv_small_group_kernel<1> : conv_small_group_kernel<2>;
+    if (int rc = allow_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
+    paella::launch(kern, dim3(next), dim3(64u * kSmallWaves), lds, reinterpret_cast<hipStream_t>(stream), g);
+    const int rc = (int)hipGetLastError();
+    return rc ? rc : 1;
+}
+
+}  // namespace
+
 extern "C" int paella_conv2d_launch_group(const paella_conv_operands* members, int n, void* stream, uint32_t job_id, void* notifier) {
     if (!members || n < 2 || n > kMaxGroup) return PAELLA_EINVAL;
     const paella_conv_plan* plans[kMaxGroup];
@@ -1979,6 +2145,7 @@ extern "C" int paella_conv2d_launch_group(const paella_conv_operands* members, i
         dyn_lds = std::max(dyn_lds, m.plan->dims.lds_bytes);
     }
     if (pack_hold(plans, args, n, stream)) return 0;
+    if (const int rc = launch_small_group(plans, args, n, nullptr, stream)) return rc == 1 ? 0 : rc;
     for (int i = 0; i < n; ++i) {
         next = align_start(next);
         g.m[i].conv = args[i];
@@ -2038,6 +2205,7 @@ extern "C" int paella_conv2d_launch_group_pool(const paella_conv_operands* membe
     if (!paella::pool_fill_args(pool, pool_x, pool_y, job_id, notifier, &pa)) return PAELLA_EINVAL;
     const unsigned pool_grid = dims.grid - next;
     if (pack_hold(plans, args, n, stream, &pa, pool_grid)) return 0;
+    if (const int rc = launch_small_group(plans, args, n, &pa, stream)) return rc == 1 ? 0 : rc;
     next = 0;
     for (int i = 0; i < n; ++i) {
         next = align_start(next);
@@ -2080,6 +2248,17 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         ConvArgs a;
         if (int rc = fill_args(plan, x, blob_dev, bias, residual, slope, y, workspace, job_id, nf, a)) return rc;
         if (plan->mi == 1 && plan->ni == 1 && !plan->depth && pack_hold(&plan, &a, 1, stream)) return 0;
+        SmallArgs small;
+        unsigned grid = 0;
+        const ConvArgs* one = &a;
+        const int mi = small_form(&plan, &one, 1);
+        if (mi && fill_small(plan, a, mi, small, &grid)) {
+            ConvSmallKernel sk = pick_small(mi);
+            if (!sk) return PAELLA_EINVAL;
+            if (int rc = allow_lds(reinterpret_cast<const void*>(sk), small_lds(plan, mi))) return rc;
+            paella::launch(sk, dim3(grid), dim3(64u * kSmallWaves), small_lds(plan, mi), st, small);
+            return (int)hipGetLastError();
+        }
         if (int rc = allow_lds(reinterpret_cast<const void*>(kern), plan->dims.lds_bytes)) return rc;
         paella::launch(kern, dim3(plan->dims.grid), dim3(plan->dims.block), plan->dims.lds_bytes, st, a);
         return (int)hipGetLastError();
@@ -2324,6 +2503,19 @@ extern "C" int paella_conv2d_launch_transformed(const paella_conv_plan* plan, co
     a.pre.shift = in_shift;
     a.pre.lo = in_act == PAELLA_ACT_RELU ? 0.f : -__builtin_inff();
     if (pack_hold_pre(plan, a, stream)) return 0;
+    SmallPreArgs small;
+    unsigned grid = 0;
+    const ConvArgs* one = &a.conv;
+    const int mi = a.conv.pair_s0 < 0 ? small_form(&plan, &one, 1) : 0;
+    if (mi && fill_small(plan, a.conv, mi, small.conv, &grid)) {
+        small.pre = a.pre;
+        ConvSmallPreKernel sk = pick_small_pre(mi);
+        if (!sk) return PAELLA_EINVAL;
+        const unsigned lds = small_lds(plan, mi) + (unsigned)kPreZeros + 8u * (unsigned)plan->d.C;
+        if (int rc = allow_lds(reinterpret_cast<const void*>(sk), lds)) return rc;
+        paella::launch(sk, dim3(grid), dim3(64u * kSmallWaves), lds, reinterpret_cast<hipStream_t>(stream), small);
+        return (int)hipGetLastError();
+    }
     if (int rc = allow_lds(reinterpret_cast<const void*>(kern), pre_lds_bytes(plan))) return rc;
     paella::launch(kern, dim3(plan->dims.grid), dim3(plan->dims.block), pre_lds_bytes(plan), reinterpret_cast<hipStream_t>(stream), a);
     return (int)hipGetLastError();

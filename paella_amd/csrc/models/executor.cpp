@@ -190,7 +190,7 @@ void pair_up(paella_model* m) {
         *out = m->plans[i];
         if (out->conv.kw == kw) return true;
         const size_t blob = out->conv.blob_bytes;
-        const int hint = log2_ceil(out->conv.splits) << 12 | 1 << 8 | 1 << 4 | log2_ceil(kw);
+        const int hint = 1 << 20 | log2_ceil(out->conv.splits) << 12 | 1 << 8 | 1 << 4 | log2_ceil(kw);
         if (paella_conv2d_plan(&out->node->conv, out->node->x2.buf >= 0, hint, &out->conv) != 0 || out->conv.blob_bytes != blob) return false;
         out->dims = out->conv.dims;
         return true;
