@@ -112,6 +112,11 @@ class Job {
     void set_completes_itself() { completes_itself_ = true; }
     void unset_completes_itself() { completes_itself_ = false; }
 
+    // An instance that keeps nothing of the requests and clients it has served: the server may give it, idle, to another client's
+    // registration of the same definition.  Set by the definition; the default is the reference's, a pool per registration.
+    bool is_shareable() const { return shareable_; }
+    void set_shareable() { shareable_ = true; }
+
     // ---- snapshot of the stage that is currently on the GPU
     unsigned get_cur_num_blocks() const { return cur_.num_blocks; }
     unsigned get_cur_num_threads_per_block() const { return cur_.num_threads_per_block; }
@@ -254,6 +259,7 @@ class Job {
     void* remote_ptr_ = nullptr;
     JobId id_ = 0;
     JobId unique_id_ = 0;
+    bool shareable_ = false;
 };
 
 }  // namespace job

@@ -8,6 +8,7 @@
 #include <llis/job/job.h>
 #include <llis/server/client_connection.h>
 
+#include <map>
 #include <memory>
 #include <string>
 #include <vector>
@@ -19,8 +20,11 @@ class RegisteredJob {
   public:
     using InitJobFn = job::Job* (*)();
 
+    // Idle instances of shareable definitions, by what they were made from (see instance_key_).  One per server, used by its thread.
+    using IdleInstances = std::map<std::string, std::vector<std::unique_ptr<job::Job>>>;
+
     // Reads {job path, pool shm name} from the request ring, loads the definition and answers with the id.
-    RegisteredJob(JobRefId registered_job_id, ipc::ShmChannelCpuReader* c2s_channel, ClientConnection* client_connection);
+    RegisteredJob(JobRefId registered_job_id, ipc::ShmChannelCpuReader* c2s_channel, ClientConnection* client_connection, IdleInstances* idle = nullptr);
     RegisteredJob(RegisteredJob&&) = default;
     RegisteredJob& operator=(RegisteredJob&&) = default;
 
@@ -59,6 +63,9 @@ class RegisteredJob {
     std::vector<void*> mapped_mem_;
 
     std::vector<std::unique_ptr<job::Job>> unused_job_instances_;
+    IdleInstances* idle_ = nullptr;
+    // The definition's path and the settings its instances read when they are made (environment variables of this project).
+    std::string instance_key_;
     std::vector<double> stage_lengths_;
     std::vector<float> stage_resources_;
 };

@@ -69,6 +69,7 @@ class Server {
     // unique_ptr: RegisteredJob keeps pointers to its ClientConnection across growth of these vectors.
     std::vector<std::unique_ptr<ClientConnection>> client_connections_;
     std::vector<ClientId> unused_client_connections_;
+    RegisteredJob::IdleInstances idle_instances_;
     std::vector<std::unique_ptr<RegisteredJob>> registered_jobs_;
     std::vector<JobRefId> unused_registered_jobs_;
 

@@ -49,6 +49,14 @@ class ModelJob : public llis::job::CoroutineJob {
         if (paella_model_io_bytes(name_.c_str(), &in_bytes_, &out_bytes_) != 0) throw std::invalid_argument("cannot load model " + name_);
     }
 
+    // An idle instance's device memory goes back with it; one that is stopped with work in flight keeps it (the kernels of a
+    // direct-dispatch queue are not waited for by the runtime's free).
+    ~ModelJob() override {
+        if (is_running() || has_next()) return;
+        if (exec_) paella_exec_destroy(exec_);
+        if (staging_) llis_hip_host_free(staging_);
+    }
+
     static std::string resolve(const char* model_name, const char* onnx_stem) {
         const char* dir = std::getenv("LLIS_MODELS_DIR");
         if (dir && *dir && onnx_stem) {
@@ -93,6 +101,7 @@ class ModelJob : public llis::job::CoroutineJob {
         // notification ring (fifo2, full3): the queues have no ordering of their own, and fifo relies on the stream.
         const char* resident = std::getenv("PAELLA_INPUT_RESIDENT");
         input_resident_ = resident && std::strcmp(resident, "1") == 0;
+        if (!input_resident_) set_shareable();  // nothing of a request outlives it
         const char* zc = std::getenv("PAELLA_ZERO_COPY_BYTES");
         const size_t zero_copy_limit = zc ? std::strtoull(zc, nullptr, 10) : 65536;
         zero_in_ = !input_resident_ && in_bytes_ <= zero_copy_limit && paella_exec_bind_input(exec_, staging_) == 0;

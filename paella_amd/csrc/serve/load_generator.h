@@ -138,20 +138,26 @@ class LoadGenerator {
             }
         }
         unsigned total = 0;
+        std::vector<std::vector<float>> inputs(variants);  // of the current type: instances that share an input copy it
         for (unsigned t = 0; t < job_refs.size(); ++t) {
+            for (std::vector<float>& in : inputs) in.clear();
             for (unsigned i = 0; i < max_outstanding_[t]; ++i) {
                 llis::client::JobInstanceRef* inst = job_refs[t].create_instance();
                 const size_t in_bytes = job_refs[t].get_job()->get_input_size();
-                std::memset(inst->get_input_ptr(), 0, in_bytes);
                 add_instance(t, inst);
                 if (!variants) {
+                    std::memset(inst->get_input_ptr(), 0, in_bytes);
                     inst->launch();
                     ++total;
                     continue;
                 }
                 const unsigned v = i % variants;
                 variant_of_[inst] = v;
-                verify_input(opt_.seed, t, v, static_cast<float*>(inst->get_input_ptr()), in_bytes / sizeof(float));
+                if (inputs[v].empty()) {
+                    inputs[v].resize((in_bytes + sizeof(float) - 1) / sizeof(float));
+                    verify_input(opt_.seed, t, v, inputs[v].data(), in_bytes / sizeof(float));
+                }
+                std::memcpy(inst->get_input_ptr(), inputs[v].data(), in_bytes);
                 std::memset(inst->get_output_ptr(), 0xFF, out_size_[t]);
                 inst->launch();
                 if (client_->wait() != inst) throw std::runtime_error("verify warm-up: a completion for another instance");

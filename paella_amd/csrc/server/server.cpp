@@ -113,7 +113,7 @@ void Server::handle_register_job() {
     ClientConnection* conn = client_connections_[client_id].get();
     if (unused_registered_jobs_.empty()) {
         const JobRefId id = (JobRefId)registered_jobs_.size();
-        registered_jobs_.push_back(std::make_unique<RegisteredJob>(id, &c2s_channel_, conn));
+        registered_jobs_.push_back(std::make_unique<RegisteredJob>(id, &c2s_channel_, conn, &idle_instances_));
     } else {
         const JobRefId id = unused_registered_jobs_.back();
         unused_registered_jobs_.pop_back();
