@@ -80,6 +80,13 @@ int paella_model_stage_work(const paella_model* m, int stage, const char** op, d
 
 int paella_exec_create(const paella_model* m, paella_exec** out);
 int paella_exec_destroy(paella_exec* e);
+/* For programs that hand inputs over and take outputs back through the two calls below: lets the host address the request's device
+ * memory, so that they need no copy engine (where the platform does not, they copy through the runtime). */
+int paella_exec_host_io(paella_exec* e);
+/* Copies the input from, and the output to, host memory.  Both wait for what a copy on the null stream would wait
+ * for; a pass on a non-blocking stream or a direct-dispatch queue is the caller's to wait for. */
+int paella_exec_set_input(paella_exec* e, const void* src);
+int paella_exec_get_output(paella_exec* e, void* dst);
 /* Device pointers of the request's input and output tensors. */
 void* paella_exec_input(paella_exec* e);
 void* paella_exec_output(paella_exec* e);

@@ -12,6 +12,7 @@
 #include <hsa/hsa.h>
 #include <hsa/hsa_ext_amd.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -342,6 +343,10 @@ void direct_dispatch(DirectQueue* q, const DirectKernel* kernel, dim3 grid, dim3
     hsa_signal_store_screlease(hq->doorbell_signal, (hsa_signal_value_t)index);
 }
 
+bool direct_allow_host_access(void* allocation) {
+    return ensure_runtime() && g_rt.have_device_pool && hsa_amd_agents_allow_access(1, &g_rt.cpu, nullptr, allocation) == HSA_STATUS_SUCCESS;
+}
+
 bool direct_system_clock(uint64_t* now_ticks, uint64_t* ticks_per_second) {
     if (!ensure_runtime()) return false;
     if (now_ticks && hsa_system_get_info(HSA_SYSTEM_INFO_TIMESTAMP, now_ticks) != HSA_STATUS_SUCCESS) return false;
@@ -427,15 +432,20 @@ extern "C" int paella_direct_queue_create(void** out) {
     q->write_index = hsa_queue_load_write_index_relaxed(q->queue);
     {
         std::lock_guard<std::mutex> lock(paella::g_mutex);
-        paella::g_queues.reserve(256);  // lookups iterate without the lock: never reallocate under them
-        if (paella::g_queues.size() >= 256) {
+        // lookups iterate without the lock: the vector never reallocates under them, and a queue keeps its place
+        paella::g_queues.reserve(256);
+        auto place = std::find(paella::g_queues.begin(), paella::g_queues.end(), nullptr);
+        if (place != paella::g_queues.end()) {
+            __atomic_store_n(&*place, q, __ATOMIC_RELEASE);
+        } else if (paella::g_queues.size() < 256) {
+            paella::g_queues.push_back(q);
+        } else {
             hsa_amd_memory_pool_free(ka);
             hsa_queue_destroy(q->queue);
             delete q;
             return PAELLA_ENOSUP;
         }
-        paella::g_queues.push_back(q);
-        __atomic_store_n(&paella::g_direct_queue_count, (int)paella::g_queues.size(), __ATOMIC_RELEASE);
+        __atomic_add_fetch(&paella::g_direct_queue_count, 1, __ATOMIC_RELEASE);
     }
     *out = q;
     return 0;
@@ -526,9 +536,8 @@ extern "C" int paella_direct_queue_destroy(void* queue) {
     {
         std::lock_guard<std::mutex> lock(paella::g_mutex);
         for (auto& slot : paella::g_queues)
-            if (slot == q) slot = paella::g_queues.back();
-        paella::g_queues.pop_back();
-        __atomic_store_n(&paella::g_direct_queue_count, (int)paella::g_queues.size(), __ATOMIC_RELEASE);
+            if (slot == q) __atomic_store_n(&slot, nullptr, __ATOMIC_RELEASE);
+        __atomic_sub_fetch(&paella::g_direct_queue_count, 1, __ATOMIC_RELEASE);
     }
     hsa_queue_destroy(q->queue);
     hsa_amd_memory_pool_free(q->kernargs);

@@ -53,6 +53,9 @@ bool direct_queue_ordered(const DirectQueue* queue);
 // there is no shared set yet.
 uint64_t direct_shared_min_waiting();
 
+// Maps an allocation of device memory (its first address) into the host's address space as well; false where that cannot be.
+bool direct_allow_host_access(void* allocation);
+
 // Kernel-argument packing: every argument at its natural alignment, in order (the kernarg segment layout of
 // by-value arguments).
 inline void pack_args(char*, size_t& offset) { (void)offset; }

@@ -19,6 +19,7 @@ struct TimingEvents {
 };
 
 TimingEvents& timing_events();  // thread-local; defined in ops_misc.hip
+bool timing_armed();
 
 // `used_bytes` (0 = all): how much of the argument block the kernel reads (see direct_dispatch).
 template <typename Kernel, typename... Args>

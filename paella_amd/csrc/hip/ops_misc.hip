@@ -291,6 +291,8 @@ inline void set_dims(paella_launch_dims* d, unsigned grid, unsigned block, unsig
 
 }  // namespace
 
+bool paella::timing_armed() { return timing_events().start != nullptr; }
+
 paella::TimingEvents& paella::timing_events() {
     static thread_local paella::TimingEvents events;
     return events;

@@ -67,6 +67,7 @@ class Exec:
         check(self.lib.paella_model_get(name.encode(), seed, ctypes.byref(self.model)), "paella_model_get")
         self.handle = ctypes.c_void_p()
         check(self.lib.paella_exec_create(self.model, ctypes.byref(self.handle)), "paella_exec_create")
+        check(self.lib.paella_exec_host_io(self.handle), "paella_exec_host_io")
         self.in_bytes, self.out_bytes = io_bytes(name)
         self.num_stages = self.lib.paella_model_num_stages(self.model)
 
@@ -96,11 +97,11 @@ class Exec:
     def set_input(self, x):
         x = np.ascontiguousarray(x, np.float32)
         assert x.nbytes == self.in_bytes
-        check(_abi.hip().llis_hip_memcpy(self.lib.paella_exec_input(self.handle), x.ctypes.data, x.nbytes, 1), "H2D")
+        check(self.lib.paella_exec_set_input(self.handle, x.ctypes.data), "paella_exec_set_input")
 
     def get_output(self):
         out = np.empty(self.out_bytes // 4, np.float32)
-        check(_abi.hip().llis_hip_memcpy(out.ctypes.data, self.lib.paella_exec_output(self.handle), out.nbytes, 2), "D2H")
+        check(self.lib.paella_exec_get_output(self.handle, out.ctypes.data), "paella_exec_get_output")
         return out
 
     def bind_io(self, in_ptr=None, out_ptr=None):
