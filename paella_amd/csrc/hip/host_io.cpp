@@ -49,12 +49,6 @@ bool wide() {
 
 bool host_map_device(void* p) { return __builtin_cpu_supports("sse4.1") && direct_allow_host_access(p); }
 
-void host_touch(void* p, size_t bytes) {
-    volatile char sink = 0;
-    for (size_t off = 0; off < bytes; off += 4096) sink = static_cast<volatile char*>(p)[off];
-    (void)sink;
-}
-
 void host_store(void* dst, const void* src, size_t bytes) {
     char* d = static_cast<char*>(dst);
     const char* s = static_cast<const char*>(src);

@@ -11,8 +11,6 @@ namespace paella {
 
 // Lets the host address `p`, the start of an allocation of device memory; false where the platform does not.
 bool host_map_device(void* p);
-// Takes the page faults of a mapped range now.
-void host_touch(void* p, size_t bytes);
 // Host to mapped device memory; the data is on its way ahead of any doorbell rung afterwards.
 void host_store(void* dst, const void* src, size_t bytes);
 // Mapped device memory to the host, once the kernels that wrote it (through to memory) have finished.  src 64-byte aligned.

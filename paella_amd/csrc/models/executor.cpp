@@ -71,6 +71,7 @@ struct paella_exec {
     float* in_bound = nullptr;   // caller's memory standing for the input / output buffer (paella_exec_bind_*)
     float* out_bound = nullptr;
     bool host_maps = false;      // the host addresses the arena itself (paella_exec_host_io)
+    unsigned inputs = 0;         // handed over by paella_exec_set_input so far
     // The pass as a graph, once it has been asked for often enough; recorded again when the input or output moves.
     void* graph = nullptr;
     std::vector<void*> old_graphs;
@@ -660,9 +661,6 @@ int paella_exec_host_io(paella_exec* e) {
     if (!e) return PAELLA_EINVAL;
     if (e->host_maps || !paella::host_map_device(e->arena)) return 0;
     e->host_maps = true;
-    const Graph& g = e->m->g;
-    paella::host_touch(e->ptr(g.input), g.input.numel() * sizeof(float));
-    if (g.output.numel() * sizeof(float) <= kHostReads) paella::host_touch(e->ptr(g.output), g.output.numel() * sizeof(float));
     return 0;
 }
 
@@ -671,7 +669,9 @@ int paella_exec_set_input(paella_exec* e, const void* src) {
     void* const dst = paella_exec_input(e);
     waited_for(e);
     const size_t bytes = e->m->g.input.numel() * sizeof(float);
-    if (!e->host_maps || e->in_bound) return llis_hip_memcpy(dst, src, bytes, LLIS_HIP_H2D);
+    // The first store to a page of the aperture takes a fault, 200 us for 602 KB: worth it for a request that is used again and again.
+    constexpr unsigned kCopiedInputs = 2;
+    if (!e->host_maps || e->in_bound || (bytes > 4096 && ++e->inputs <= kCopiedInputs)) return llis_hip_memcpy(dst, src, bytes, LLIS_HIP_H2D);
     if (int rc = llis_hip_stream_synchronize(nullptr)) return rc;  // behind everything that a copy would wait for
     paella::host_store(dst, src, bytes);
     return 0;
