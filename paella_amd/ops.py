@@ -5,6 +5,7 @@ on the host with paella_conv2d_pack and uploaded.  Everything runs on the callin
 stream unless a stream handle is given.
 """
 import ctypes
+import functools
 
 import numpy as np
 import torch
@@ -15,15 +16,31 @@ from ._abi import ConvDesc, ConvOperands, ConvPlan, LaunchDims, PoolDesc, check
 ACT_NONE, ACT_RELU, ACT_RELU6, ACT_PRELU, ACT_CLIP = range(5)
 
 
+# A call's time on a small layer is what it costs the calling thread: the launch is 2.7 us of it, an output tensor 1.2, and everything
+# here is meant to stay under 1 (torch.cuda.current_stream alone is 2.6; pointers go to the library as plain integers).
+
 def _ptr(t):
     if t is None:
         return None
     assert t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+def _torch_stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+try:
+    from torch._C import _cuda_getCurrentRawStream, _cuda_getDevice
+
+    def _torch_stream():  # noqa: F811  (the same handle without the stream object around it)
+        return _cuda_getCurrentRawStream(_cuda_getDevice())
+except ImportError:
+    pass
 
 
 def _stream(stream):
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream if stream is None else stream)
+    return _torch_stream() if stream is None else stream
 
 
 def _pair(v):
@@ -53,6 +70,10 @@ class Conv2d:
         self.slope = None if slope is None else torch.tensor(np.asarray(slope, np.float32), device=device)
         self.workspace = torch.zeros(max(self.plan.workspace_bytes, 4) // 4, dtype=torch.int32, device=device) if self.plan.workspace_bytes else None
         self.lib = lib
+        # what every call passes on, looked up once
+        self._plan_ref = ctypes.byref(self.plan)
+        self._launch, self._launch_transformed = lib.paella_conv2d_launch, lib.paella_conv2d_launch_transformed
+        self._in_shape, self._out_shape = (1, self.plan.d.C, self.plan.d.H, self.plan.d.W), (1, self.plan.d.K, self.plan.P, self.plan.Q)
 
     def takes_input_transform(self):
         return bool(self.lib.paella_conv2d_plan_takes_input_transform(ctypes.byref(self.plan)))
@@ -60,30 +81,30 @@ class Conv2d:
     def __call__(self, x, residual=None, out=None, stream=None, job_id=0, notifier=None, in_scale=None, in_shift=None, in_act=ACT_NONE):
         """in_scale / in_shift (per input channel, device tensors): the conv reads in_act(x * in_scale + in_shift), padded
         with zeros after that transform."""
-        p = self.plan
-        assert x.shape == (1, p.d.C, p.d.H, p.d.W), (tuple(x.shape), p.d.C, p.d.H, p.d.W)
-        y = out if out is not None else torch.empty((1, p.d.K, p.P, p.Q), device=x.device, dtype=torch.float32)
+        assert x.shape == self._in_shape, (tuple(x.shape), self._in_shape)
+        y = out if out is not None else x.new_empty(self._out_shape, dtype=torch.float32)
+        workspace = self.workspace
+        if workspace is not None:
+            workspace = workspace.data_ptr()
         if in_scale is not None:
+            p = self.plan
             assert in_scale.numel() == p.d.C and in_shift.numel() == p.d.C
-            check(self.lib.paella_conv2d_launch_transformed(ctypes.byref(p), _ptr(x), _ptr(in_scale), _ptr(in_shift), in_act,
-                                                            ctypes.c_void_p(self.blob.data_ptr()), _ptr(self.bias), _ptr(residual),
-                                                            _ptr(self.slope), _ptr(y),
-                                                            ctypes.c_void_p(self.workspace.data_ptr()) if self.workspace is not None else None,
-                                                            _stream(stream), job_id, notifier), "paella_conv2d_launch_transformed")
+            rc = self._launch_transformed(self._plan_ref, _ptr(x), _ptr(in_scale), _ptr(in_shift), in_act, self.blob.data_ptr(), _ptr(self.bias),
+                                          _ptr(residual), _ptr(self.slope), _ptr(y), workspace, _stream(stream), job_id, notifier)
+            if rc:
+                check(rc, "paella_conv2d_launch_transformed")
             return y
-        check(self.lib.paella_conv2d_launch(ctypes.byref(p), _ptr(x), ctypes.c_void_p(self.blob.data_ptr()),
-                                            _ptr(self.bias), _ptr(residual), _ptr(self.slope), _ptr(y),
-                                            ctypes.c_void_p(self.workspace.data_ptr()) if self.workspace is not None else None,
-                                            _stream(stream), job_id, notifier), "paella_conv2d_launch")
+        rc = self._launch(self._plan_ref, _ptr(x), self.blob.data_ptr(), _ptr(self.bias), _ptr(residual), _ptr(self.slope), _ptr(y), workspace,
+                          _stream(stream), job_id, notifier)
+        if rc:
+            check(rc, "paella_conv2d_launch")
         return y
-
 
     def operands(self, x, residual=None, out=None):
         p = self.plan
         assert x.shape == (1, p.d.C, p.d.H, p.d.W), (tuple(x.shape), p.d.C, p.d.H, p.d.W)
         y = out if out is not None else torch.empty((1, p.d.K, p.P, p.Q), device=x.device, dtype=torch.float32)
-        data = lambda t: None if t is None else _ptr(t).value
-        ops = ConvOperands(ctypes.pointer(p), data(x), self.blob.data_ptr(), data(self.bias), data(residual), data(self.slope), data(y),
+        ops = ConvOperands(ctypes.pointer(p), _ptr(x), self.blob.data_ptr(), _ptr(self.bias), _ptr(residual), _ptr(self.slope), _ptr(y),
                            None if self.workspace is None else self.workspace.data_ptr())
         return ops, y
 
@@ -119,14 +140,8 @@ def conv2d_group_pool(convs, xs, pool_x, k, stride, pad=0, ceil_mode=False, is_a
         members[i], y = c.operands(x, r)
         outs.append(y)
     lib = convs[0].lib
-    _, c, h, w = pool_x.shape
-    r, s = _pair(k)
-    sh, sw = _pair(stride)
-    ph, pw = _pair(pad)
-    d = PoolDesc(c, h, w, r, s, sh, sw, ph, pw, int(ceil_mode), int(is_avg), int(count_include_pad))
-    p = lib.paella_pool_out(h, r, sh, ph, int(ceil_mode))
-    q = lib.paella_pool_out(w, s, sw, pw, int(ceil_mode))
-    pool_y = torch.empty((1, c, p, q), device=pool_x.device, dtype=torch.float32)
+    d, shape = _pool_desc(*pool_x.shape[1:], _pair(k), _pair(stride), _pair(pad), bool(ceil_mode), bool(is_avg), bool(count_include_pad))
+    pool_y = torch.empty(shape, device=pool_x.device, dtype=torch.float32)
     check(lib.paella_conv2d_launch_group_pool(members, len(convs), ctypes.byref(d), _ptr(pool_x), _ptr(pool_y), _stream(stream), job_id,
                                               notifier), "paella_conv2d_launch_group_pool")
     return outs, pool_y
@@ -138,10 +153,18 @@ def pair_dims(first, second):
     return rc, d
 
 
+@functools.lru_cache(maxsize=256)
+def _pool_desc(c, h, w, k, stride, pad, ceil_mode, is_avg, count_include_pad):
+    """The descriptor of a pooling operator and the shape of its output."""
+    lib = _abi.ops()
+    d = PoolDesc(c, h, w, *k, *stride, *pad, int(ceil_mode), int(is_avg), int(count_include_pad))
+    return d, (1, c, lib.paella_pool_out(h, k[0], stride[0], pad[0], int(ceil_mode)), lib.paella_pool_out(w, k[1], stride[1], pad[1], int(ceil_mode)))
+
+
 def dense(x, w, bias=None, act=ACT_NONE, stream=None, job_id=0, notifier=None):
     lib = _abi.ops()
     o, i = w.shape
-    y = torch.empty((1, o), device=x.device, dtype=torch.float32)
+    y = x.new_empty((1, o), dtype=torch.float32)
     check(lib.paella_dense_launch(_ptr(x), _ptr(w), _ptr(bias), _ptr(y), i, o, act, _stream(stream), job_id, notifier),
           "paella_dense_launch")
     return y
@@ -150,14 +173,8 @@ def dense(x, w, bias=None, act=ACT_NONE, stream=None, job_id=0, notifier=None):
 def pool2d(x, k, stride, pad=0, ceil_mode=False, is_avg=False, count_include_pad=True, stream=None, job_id=0,
            notifier=None):
     lib = _abi.ops()
-    _, c, h, w = x.shape
-    r, s = _pair(k)
-    sh, sw = _pair(stride)
-    ph, pw = _pair(pad)
-    d = PoolDesc(c, h, w, r, s, sh, sw, ph, pw, int(ceil_mode), int(is_avg), int(count_include_pad))
-    p = lib.paella_pool_out(h, r, sh, ph, int(ceil_mode))
-    q = lib.paella_pool_out(w, s, sw, pw, int(ceil_mode))
-    y = torch.empty((1, c, p, q), device=x.device, dtype=torch.float32)
+    d, shape = _pool_desc(*x.shape[1:], _pair(k), _pair(stride), _pair(pad), bool(ceil_mode), bool(is_avg), bool(count_include_pad))
+    y = x.new_empty(shape, dtype=torch.float32)
     check(lib.paella_pool2d_launch(ctypes.byref(d), _ptr(x), _ptr(y), _stream(stream), job_id, notifier),
           "paella_pool2d_launch")
     return y
