@@ -71,6 +71,7 @@ class Job {
         is_unfit_ = false;
         deficit_counter_ = 0;
         cur_stage_ = -1;
+        next_span_ = cur_span_ = 1;
     }
 
     void set_id(JobId id) {
@@ -95,6 +96,9 @@ class Job {
     void set_num_threads_per_block(unsigned v) { next_.num_threads_per_block = v; }
     void set_smem_size_per_block(unsigned v) { next_.smem_size_per_block = v; }
     void set_num_registers_per_thread(unsigned v) { next_.num_registers_per_thread = v; }
+    // The declared stage does the work of this many consecutive ones, itself the last of them (1 until said otherwise).
+    void set_stage_span(unsigned v) { next_span_ = v; }
+    unsigned get_stage_span() const { return next_span_; }
 
     bool is_mem() const { return is_mem_; }
     void set_is_mem() { is_mem_ = true; }
@@ -122,6 +126,7 @@ class Job {
     unsigned get_cur_num_threads_per_block() const { return cur_.num_threads_per_block; }
     unsigned get_cur_smem_size_per_block() const { return cur_.smem_size_per_block; }
     unsigned get_cur_num_registers_per_thread() const { return cur_.num_registers_per_thread; }
+    unsigned get_cur_stage_span() const { return cur_span_; }
 
     bool is_running() const { return is_running_; }
     void unset_running() { is_running_ = false; }
@@ -135,7 +140,9 @@ class Job {
         num_pending_blocks_ = next_.num_blocks;
         clear_predicted_smids();
         stage_start_time_ = Clock::now();
-        ++cur_stage_;
+        cur_stage_ += (int)next_span_;
+        cur_span_ = next_span_;
+        next_span_ = 1;
     }
 
     StreamHandle get_cuda_stream() const { return cuda_stream_; }
@@ -217,16 +224,18 @@ class Job {
         stage_resources_ = resources;
     }
     double get_cur_rl() const { return cur_rl_; }
-    // Removes the stage that is about to be queued (cur_stage + 1) from the remaining work.
+    // Removes the stage that is about to be queued (cur_stage + 1, and those it stands for) from the remaining work.
     void dec_cur_rl() {
         // A stage whose length has not been learned yet counts as zero work.
-        const size_t next = (size_t)(cur_stage_ + 1);
-        if (next < stage_lengths_.size() && next < stage_resources_.size()) cur_rl_ -= stage_lengths_[next] * stage_resources_[next];
+        const size_t first = (size_t)(cur_stage_ + 1);
+        for (size_t next = first; next < first + next_span_; ++next)
+            if (next < stage_lengths_.size() && next < stage_resources_.size()) cur_rl_ -= stage_lengths_[next] * stage_resources_[next];
     }
 
   private:
     StageNeeds next_;
     StageNeeds cur_;
+    unsigned next_span_ = 1, cur_span_ = 1;
     bool is_mem_ = false;
     bool is_pre_notify_ = false;
     bool completes_itself_ = false;

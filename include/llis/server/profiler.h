@@ -36,6 +36,9 @@ class Profiler {
 
     bool recording_kernel_info() const { return kernel_info_flag_; }
     bool recording_job_events() const { return job_events_flag_; }
+    bool recording() const {
+        return kernel_info_flag_ || job_events_flag_ || run_next_times_flag_ || resource_events_flag_ || block_exec_times_flag_ || mis_alloc_flag_;
+    }
 
     void record_kernel_info(TimePoint start, TimePoint end, unsigned num_blocks, unsigned num_threads_per_block, unsigned smem_size_per_block,
                             unsigned num_registers_per_thread, double priority, unsigned job_ref_id);

@@ -98,6 +98,7 @@ class SchedulerFull3 : public StreamPoolScheduler {
     void schedule_job();
     void requeue_or_finish(job::Job* job);
     double take_priority(job::Job* job) const;
+    void know_next_stage(job::Job* job);
 
     JobQueue job_queue_;
     SmResources gpu_resources_;

@@ -97,6 +97,12 @@ double SchedulerFull3::take_priority(job::Job* job) const {
     return -remaining;
 }
 
+void SchedulerFull3::know_next_stage(job::Job* job) {
+    const unsigned first = (unsigned)(job->get_cur_stage() + 1);
+    for (unsigned s = first; s < first + job->get_stage_span(); ++s)
+        if (!server_->has_job_stage_resource(job, s)) server_->set_job_stage_resource(job, s, 1);
+}
+
 void SchedulerFull3::handle_new_job(std::unique_ptr<job::Job> owned) {
     if (!owned->has_next()) {
         server_->release_job_instance(std::move(owned));
@@ -107,8 +113,7 @@ void SchedulerFull3::handle_new_job(std::unique_ptr<job::Job> owned) {
     log_->add('J', job->get_id(), job->get_registered_job_id(), job->get_unique_id(), first_is_mem);
     profiler_->record_job_event(job->get_id(), Profiler::JobEvent::JOB_SUBMITTED);
 
-    const unsigned next_stage = (unsigned)(job->get_cur_stage() + 1);
-    if (!server_->has_job_stage_resource(job, next_stage)) server_->set_job_stage_resource(job, next_stage, 1);
+    know_next_stage(job);
     job->set_stage_lengths_resources(server_->get_job_remaining_rl(job, 0), server_->get_job_stage_lengths(job), server_->get_job_stage_resources(job));
     job->set_priority(take_priority(job));
     if (!job->is_mem()) profiler_->record_queued_resource_event(job);
@@ -140,11 +145,11 @@ void SchedulerFull3::requeue_or_finish(job::Job* job) {
     const auto end_time = std::chrono::steady_clock::now();
     const double length = std::chrono::duration<double, std::micro>(end_time - job->get_stage_start_time()).count();
     log_->add('L', job->get_id(), job->get_cur_stage(), 0, 0, 0, length);
-    server_->update_job_stage_length(job, (unsigned)job->get_cur_stage(), length);
+    const unsigned span = job->get_cur_stage_span();
+    for (unsigned k = 0; k < span; ++k) server_->update_job_stage_length(job, (unsigned)job->get_cur_stage() - k, length / span);
 
     if (job->has_next()) {
-        const unsigned next_stage = (unsigned)(job->get_cur_stage() + 1);
-        if (!server_->has_job_stage_resource(job, next_stage)) server_->set_job_stage_resource(job, next_stage, 1);
+        know_next_stage(job);
         job->set_priority(take_priority(job));
         if (!job->is_mem()) profiler_->record_queued_resource_event(job);
         job_queue_.push(job);
@@ -224,6 +229,7 @@ void SchedulerFull3::schedule_job() {
         }
 
         job::Context::set_current_job(job);
+        job::Context::set_alone(num_jobs_ == 1 && !per_cu_ && !log_->enabled() && !profiler_->recording());
         profiler_->record_job_event(job->get_id(), Profiler::JobEvent::KERNEL_SUBMIT_START);
         {
             LLIS_PHASE_IF(is_mem, kLaunchCopy, kLaunch);
