@@ -43,14 +43,15 @@ class Context {
     // jobs always launch on the stream.
     static void set_stage_by_stage(bool v) {
         stage_by_stage_ = v;
-        alone_ = false;
+        uncrowded_ = false;
     }
     static bool is_stage_by_stage() { return stage_by_stage_; }
 
-    // True when the current job is the only one in flight and nobody records its stages: it may then issue several of them at once
-    // (Job::set_stage_span) instead of waiting for the scheduler between any two.  Not in the reference.
-    static void set_alone(bool v) { alone_ = v; }
-    static bool is_alone() { return alone_; }
+    // True when so few jobs are in flight that each may have a hardware queue to itself, and nobody records their stages: a job may
+    // then issue several of them at once (Job::set_stage_span) instead of waiting for the scheduler between any two.  Not in the
+    // reference.
+    static void set_uncrowded(bool v) { uncrowded_ = v; }
+    static bool is_uncrowded() { return uncrowded_; }
 
     // Functions the serving thread calls once per turn of its loop, after it has looked at its rings: for job libraries
     // that hold work back and release it from that thread (a function is added once, however often it is registered).
@@ -66,7 +67,7 @@ class Context {
     static PollHook poll_hooks_[kMaxPollHooks];
     static unsigned num_poll_hooks_;
     static bool stage_by_stage_;
-    static bool alone_;
+    static bool uncrowded_;
     static Job* current_job_;
     static ipc::Gpu2SchedChannel gpu2sched_channel_;
     static ipc::Gpu2SchedChannel gpu2sched_block_time_channel_;

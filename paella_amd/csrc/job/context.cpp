@@ -4,7 +4,7 @@ namespace llis {
 namespace job {
 
 Job* Context::current_job_ = nullptr;
-bool Context::alone_ = false;
+bool Context::uncrowded_ = false;
 bool Context::stage_by_stage_ = false;
 ipc::Gpu2SchedChannel Context::gpu2sched_channel_;
 ipc::Gpu2SchedChannel Context::gpu2sched_block_time_channel_;

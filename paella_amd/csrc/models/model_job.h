@@ -123,8 +123,8 @@ class ModelJob : public llis::job::CoroutineJob {
                 direct_ = whole_job_direct_ = false;
             }
         }
-        // (Eight: a request that arrives in between finds three more queues, and waits for 30 to 70 us at the most.)
-        alone_stages_ = direct_ && !timed_ && group_limit > 0 ? 8 : 1;
+        // (Sixteen at once are another 3 to 5 % for a request alone, but twice as long in a newcomer's way; four lose 10 %.)
+        uncrowded_stages_ = direct_ && !timed_ && group_limit > 0 ? 8 : 1;
         // Conv launches of different requests share launches (paella_pack_enable) unless PAELLA_PACK=0: the serving thread
         // holds them and lets them go from its loop.
         const char* pack = std::getenv("PAELLA_PACK");
@@ -181,18 +181,19 @@ class ModelJob : public llis::job::CoroutineJob {
 
         for (int s = 0; s < num_stages_;) {
             int last = group_end_[(size_t)s];
-            // The only request in flight is not kept waiting for the scheduler after every kernel, which is 4 us of a stage's 8 to 9,
-            // and its kernels but the group's last, which report to nobody, take the tiles of a launch without a server: Inception-v3
-            // alone 801 -> 481 us, DenseNet-121 1404 -> 786, ResNet-18 305 -> 198.
-            const bool alone = alone_stages_ > 1 && last == s && llis::job::Context::is_alone();
-            if (alone) last = std::min(s + alone_stages_, num_stages_) - 1;
+            // One of few requests in flight is not kept waiting for the scheduler after every kernel, which is 4 us of a stage's 8 to 9,
+            // and its kernels but the group's last, which report to nobody, take the tiles of a launch without a server.  Requests/s
+            // with one / two / four in flight: Inception-v3 1250 / 2150 / 3420 -> 2140 / 3480 / 4740, DenseNet-121 710 / 1320 / 2310
+            // -> 1270 / 2370 / 3810, ResNet-18 3280 / 5920 / 9500 -> 5060 / 7960 / 12030.
+            const bool group = uncrowded_stages_ > 1 && last == s && llis::job::Context::is_uncrowded();
+            if (group) last = std::min(s + uncrowded_stages_, num_stages_) - 1;
             paella_launch_dims d;
             paella_model_stage_dims(model_, last, &d);  // the group is admitted and accounted as its last kernel
             set_num_blocks(d.grid);
             set_num_threads_per_block(d.block);
             set_smem_size_per_block(d.lds_bytes);
             set_num_registers_per_thread(d.vgprs);
-            if (alone) set_stage_span((unsigned)(last - s + 1));
+            if (group) set_stage_span((unsigned)(last - s + 1));
             if (zero_out_ && last == num_stages_ - 1) set_pre_notify();
             yield();
             if (zero_in_ && s == 0) std::memcpy(staging_, io_ptr, in_bytes_);
@@ -214,7 +215,7 @@ class ModelJob : public llis::job::CoroutineJob {
             // too, so that it is not held back for packing while the others go out
             if (direct_ && last > s) paella_direct_queue_set_ordered(target, 1);
             // ... and the whole group is recorded, to go out together with the same group of other requests of this model
-            const bool recording = pack_ && last > s && !alone && paella_pack_sequence_begin(model_, target) == 0;
+            const bool recording = pack_ && last > s && !group && paella_pack_sequence_begin(model_, target) == 0;
             for (int k = s; k <= last; ++k) {
                 if (k < last) check(paella_exec_launch_stage(exec_, k, target, 0, nullptr), "stage launch");
                 else check(paella_exec_launch_stage(exec_, k, target, id, get_finished_block_notifier()), "stage launch");
@@ -273,7 +274,7 @@ class ModelJob : public llis::job::CoroutineJob {
     bool pack_ = false;
     bool stage_off_thread_ = false;
     bool timed_ = false;
-    int alone_stages_ = 1;         // kernels issued at once for the only request in flight
+    int uncrowded_stages_ = 1;     // kernels issued at once for a request that shares the device with few others
     bool unfit_starts_ = false;
     bool input_resident_ = false, input_uploaded_ = false;
     bool zero_in_ = false, zero_out_ = false;
