@@ -39,8 +39,16 @@ except ImportError:
     pass
 
 
+_direct_queues = set()
+
+
 def _stream(stream):
-    return _torch_stream() if stream is None else stream
+    if stream is None:
+        return _torch_stream()
+    if stream in _direct_queues:
+        # nothing orders such a queue behind torch's stream, and a call is quick enough to overtake a fill that is still under way there
+        torch.cuda.current_stream().synchronize()
+    return stream
 
 
 def _pair(v):
@@ -233,6 +241,7 @@ class DirectQueue:
         h = ctypes.c_void_p()
         check(self.lib.paella_direct_queue_create(ctypes.byref(h)), "paella_direct_queue_create")
         self.handle = h.value
+        _direct_queues.add(self.handle)
         if ordered:
             check(self.lib.paella_direct_queue_set_ordered(h, 1), "paella_direct_queue_set_ordered")
 
@@ -241,6 +250,7 @@ class DirectQueue:
 
     def close(self):
         if self.handle:
+            _direct_queues.discard(self.handle)
             check(self.lib.paella_direct_queue_destroy(ctypes.c_void_p(self.handle)), "paella_direct_queue_destroy")
             self.handle = None
 
