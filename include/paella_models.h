@@ -87,6 +87,11 @@ int paella_exec_host_io(paella_exec* e);
  * for; a pass on a non-blocking stream or a direct-dispatch queue is the caller's to wait for. */
 int paella_exec_set_input(paella_exec* e, const void* src);
 int paella_exec_get_output(paella_exec* e, void* dst);
+/* The input of a request that nothing on the device is working on, written to its device memory by the library's copy thread or, where
+ * that sleeps, by the call: done(arg) says, from either, that a kernel on a direct-dispatch queue may follow (done NULL: written by the
+ * call).  PAELLA_ENOSUP, with nothing done, where the host does not address that memory (paella_exec_host_io; the first store to each
+ * of its pages is slow). */
+int paella_exec_store_input(paella_exec* e, const void* src, void (*done)(void*), void* arg);
 /* Device pointers of the request's input and output tensors. */
 void* paella_exec_input(paella_exec* e);
 void* paella_exec_output(paella_exec* e);

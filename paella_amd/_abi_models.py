@@ -24,6 +24,7 @@ MODEL_SYMBOLS = {
     "paella_exec_bind_input": (c_int, [c_void_p, c_void_p]),
     "paella_exec_bind_output": (c_int, [c_void_p, c_void_p]),
     "paella_exec_host_io": (c_int, [c_void_p]),
+    "paella_exec_store_input": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "paella_exec_set_input": (c_int, [c_void_p, c_void_p]),
     "paella_exec_get_output": (c_int, [c_void_p, c_void_p]),
     "paella_exec_input": (c_void_p, [c_void_p]),

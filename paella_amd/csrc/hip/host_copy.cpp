@@ -2,8 +2,10 @@
 // shared-memory pool into the pinned staging buffers, so that the serving thread, which must keep reading the
 // notification ring, is not deaf for the 20 to 40 us such a copy takes.  The helper makes no call into the GPU runtime
 // (two threads inside the runtime contend for more than the copy costs); the job issues the host-to-device copy itself
-// once the helper has reported.
+// once the helper has reported.  Where the host addresses the request's device memory itself, the helper writes the input there and
+// no copy follows.
 
+#include "host_io.h"
 #include "paella_ops.h"
 
 #include <atomic>
@@ -25,6 +27,7 @@ struct CopyItem {
     size_t bytes;
     void (*done)(void*);
     void* arg;
+    bool to_device = false;  // dst is mapped device memory (host_io.h)
 };
 
 class CopyWorker {
@@ -88,7 +91,8 @@ class CopyWorker {
                 queue_.pop_front();
             }
             pending_.fetch_sub(1, std::memory_order_acq_rel);
-            std::memcpy(item.dst, item.src, item.bytes);
+            if (item.to_device) paella::host_store(item.dst, item.src, item.bytes);
+            else std::memcpy(item.dst, item.src, item.bytes);
             item.done(item.arg);
         }
     }
@@ -103,10 +107,20 @@ class CopyWorker {
     std::thread thread_;  // last member: the thread starts with everything above constructed
 };
 
+int submit(const CopyItem& item) {
+    static CopyWorker* worker = new CopyWorker();  // lives until the process ends; its thread is never joined
+    return worker->submit(item) ? 0 : PAELLA_EBUSY;
+}
+
 }  // namespace
 
 extern "C" int paella_host_copy_submit(void* dst, const void* src, size_t bytes, void (*done)(void*), void* arg) {
     if (!dst || !src || !done) return PAELLA_EINVAL;
-    static CopyWorker* worker = new CopyWorker();  // lives until the process ends; its thread is never joined
-    return worker->submit(CopyItem{dst, src, bytes, done, arg}) ? 0 : PAELLA_EBUSY;
+    return submit(CopyItem{dst, src, bytes, done, arg});
 }
+
+namespace paella {
+
+int host_store_submit(void* dst, const void* src, size_t bytes, void (*done)(void*), void* arg) { return submit(CopyItem{dst, src, bytes, done, arg, true}); }
+
+}  // namespace paella

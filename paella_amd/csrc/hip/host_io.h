@@ -13,6 +13,8 @@ namespace paella {
 bool host_map_device(void* p);
 // Host to mapped device memory; the data is on its way ahead of any doorbell rung afterwards.
 void host_store(void* dst, const void* src, size_t bytes);
+// The same by the library's copy thread, as paella_host_copy_submit.
+int host_store_submit(void* dst, const void* src, size_t bytes, void (*done)(void*), void* arg);
 // Mapped device memory to the host, once the kernels that wrote it (through to memory) have finished.  src 64-byte aligned.
 void host_load(void* dst, const void* src, size_t bytes);
 

@@ -677,6 +677,18 @@ int paella_exec_set_input(paella_exec* e, const void* src) {
     return 0;
 }
 
+int paella_exec_store_input(paella_exec* e, const void* src, void (*done)(void*), void* arg) {
+    if (!e || !src) return PAELLA_EINVAL;
+    if (!e->host_maps || e->in_bound) return PAELLA_ENOSUP;
+    void* const dst = paella_exec_input(e);
+    const size_t bytes = e->m->g.input.numel() * sizeof(float);
+    if (!done || paella::host_store_submit(dst, src, bytes, done, arg) != 0) {
+        paella::host_store(dst, src, bytes);
+        if (done) done(arg);
+    }
+    return 0;
+}
+
 int paella_exec_get_output(paella_exec* e, void* dst) {
     if (!e || !dst) return PAELLA_EINVAL;
     const void* const src = paella_exec_output(e);
