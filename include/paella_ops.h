@@ -87,7 +87,8 @@ typedef struct paella_conv_plan {
 } paella_conv_plan;
 
 /* Pure host arithmetic: picks the kernel variant and launch shape.  tile_hint = 0 lets the library
- * choose; otherwise log2(splits)<<12 | mi<<8 | ni<<4 | log2(kw) forces a shape (tuning sweeps and tests). */
+ * choose; otherwise log2(splits)<<12 | mi<<8 | ni<<4 | log2(kw) forces a shape (tuning sweeps and tests), with 1<<20 one whose
+ * launches may still take the smaller tiles (`small`). */
 int paella_conv2d_plan(const paella_conv_desc* desc, int has_residual, int tile_hint, paella_conv_plan* plan);
 
 /* Launch shape of paella_conv2d_launch for the scheduler: the plan's, with the register count and the static LDS of the
