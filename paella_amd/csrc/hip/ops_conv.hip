@@ -999,6 +999,9 @@ struct DwArgs {
     FastDiv div_q, div_p;
     int fast;
     unsigned x_bytes, out_bytes;
+    // strips of four outputs (dwconv_strip_kernel): strips per row of outputs and in all; quotient by the former
+    int strips_row, strips;
+    FastDiv div_strip;
 };
 
 // All taps of one output element.  With the filter size known the loads of a window leave back to back (a tap outside the
@@ -1141,6 +1144,66 @@ __device__ __forceinline__ void dw_batch3x3(const DwArgs& p, const int idx, cons
 #pragma unroll
     for (int k = 0; k < K; ++k)  // write-through (sc1), like store_out
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[k]), yr, out_off[k], 0, 16);
+}
+
+// Four neighbouring outputs per thread, along one row of a 3 x 3 depthwise conv with one column of padding and stride SW along the row.  What
+// bounds this operator at batch 1 is not HBM but the number of vector memory instructions per compute unit (one element at a time:
+// 9 taps, 9 weights, bias, residual and slope, 20 per output): here the four outputs share their taps, and all columns but the first
+// and the last are inside the image whatever its width, so a row of taps is one 16-byte load and two or three more (SW = 1: columns
+// 1..4, then 0 and 5; SW = 2: 1..4, 5..7, then 0 and 8), 13 to 16 loads for four outputs.  A row's last strip starts at Q - 4: it
+// computes some outputs of its neighbour once more, to the same bits, instead of testing every column.  Same taps in the same order
+// as dw_element, and so the same bits.
+template <int SW>
+__global__ __launch_bounds__(256) void dwconv_strip_kernel(DwArgs p) {
+    const int idx = (int)(blockIdx.x * 256u + threadIdx.x);
+    if (idx >= p.strips) return;
+    constexpr int kCols = SW == 1 ? 6 : 9;
+    const unsigned pad_off = (unsigned)(p.ph * p.W + 1) * 4u;  // see dw_batch3x3
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const char*>(p.x) - pad_off), 0, p.x_bytes + pad_off, 0x00027000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (unsigned)p.C * 36u, 0x00027000);
+    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc((void*)p.bias, 0, p.bias ? (unsigned)p.C * 4u : 0u, 0x00027000);
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc((void*)p.y, 0, p.out_bytes, 0x00027000);
+    const int row = (int)quot_fast((unsigned)idx, p.div_strip);  // over (channel, output row)
+    const int wo = min((idx - __mul24(row, p.strips_row)) * 4, p.Q - 4);
+    const int c = (int)quot_fast((unsigned)row, p.div_p);
+    const int ho = row - __mul24(c, p.P);
+    const int hs = __mul24(ho, p.sh), ws = wo * SW;
+    const int base = (__mul24(__mul24(c, p.H) + hs, p.W) + ws) * 4;
+    const int first_bad = ws ? 0 : (int)0x80000000u;
+    const int last_bad = ws + kCols - 2 < p.W ? 0 : (int)0x80000000u;
+    auto word = [](const __amdgpu_buffer_rsrc_t r, int voff, int soff) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0)); };
+    float v[3][kCols];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int at = base | ((unsigned)(hs - p.ph + r) < (unsigned)p.H ? 0 : (int)0x80000000u);
+        const int soff = r * p.W * 4;
+        const float4 in = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, at, soff + 4, 0));
+        v[r][1] = in.x; v[r][2] = in.y; v[r][3] = in.z; v[r][4] = in.w;
+        if (SW == 2) {
+            const float2 more = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(xr, at, soff + 20, 0));
+            v[r][5 % kCols] = more.x; v[r][6 % kCols] = more.y;
+            v[r][7 % kCols] = word(xr, at, soff + 28);
+        }
+        v[r][0] = word(xr, at | first_bad, soff);
+        v[r][kCols - 1] = word(xr, at | last_bad, soff + (kCols - 1) * 4);
+    }
+    const int woff = __mul24(c, 36);
+    const float4 wa = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff, 0, 0));
+    const float4 wb = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff, 16, 0));
+    const float wt[9] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w, word(wr, woff, 32)};
+    const float bias = word(br, c * 4, 0);
+    const float slope = p.act == PAELLA_ACT_PRELU ? p.slope[c] : 0.f;
+    float acc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        acc[k] = bias;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[k] = fmaf(v[t / 3][k * SW + t % 3], wt[t], acc[k]);
+        acc[k] = apply_act(acc[k], p.act, slope, p.lo, p.hi);
+    }
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, make_float4(acc[0], acc[1], acc[2], acc[3])), yr,
+                                           (__mul24(row, p.Q) + wo) * 4, 0, 16);  // write-through (sc1), like store_out
 }
 
 // One workgroup's share of a depthwise conv of `grid` workgroups.
@@ -2284,6 +2347,14 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         a.out_bytes = (unsigned)std::min<uint64_t>(elements * 4, 0xFFFFFFFFu);
     }
     if (pack_hold_dw(a, plan->dims.grid, stream)) return 0;
+    // Strips of four outputs: the kernel's window is fixed, and its workgroups are not the plan's, so nobody may count them.
+    if (a.fast && !nf && !residual && d.pad_w == 1 && d.dil_h == 1 && d.dil_w == 1 && d.stride_w <= 2 && plan->Q >= 4) {
+        a.strips_row = (plan->Q + 3) / 4;
+        a.strips = d.C * plan->P * a.strips_row;
+        a.div_strip = fast_div((unsigned)a.strips_row);
+        paella::launch(d.stride_w == 1 ? dwconv_strip_kernel<1> : dwconv_strip_kernel<2>, dim3((unsigned)(a.strips + 255) / 256u), dim3(256), 0, st, a);
+        return (int)hipGetLastError();
+    }
     paella::launch(dwconv_kernel, dim3(plan->dims.grid), dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }

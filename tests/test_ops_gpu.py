@@ -346,6 +346,21 @@ def test_depthwise_conv_parity(cuda, c, h, w, r, stride, pad, dil):
     close(conv(torch.tensor(x, device=cuda)), ref)
 
 
+# the four-outputs-a-thread form: rows of 4 outputs, of a strip and a remainder, odd and even widths under stride 2, strides that differ
+@pytest.mark.parametrize("act", ["ACT_NONE", "ACT_RELU", "ACT_PRELU"])
+@pytest.mark.parametrize("c,h,w,stride,pad_h", [(2, 1, 4, 1, 1), (3, 2, 5, 1, 1), (7, 5, 7, 2, 1), (5, 9, 8, 2, 1), (33, 6, 9, 2, 0), (130, 7, 7, 1, 1), (17, 12, 31, (1, 2), 1),
+                                                (17, 12, 30, (2, 1), 2)])
+def test_depthwise_strips_match_the_oracle(cuda, c, h, w, stride, pad_h, act):
+    from paella_amd import ops
+    x, wt, b, slope = rnd(1, c, h, w), rnd(c, 1, 3, 3, scale=0.3), rnd(c, scale=0.1), rnd(c, scale=0.2)
+    prelu = act == "ACT_PRELU"
+    both = stride if isinstance(stride, tuple) else (stride, stride)
+    ref = orc.conv2d(x, wt, b, stride=both, pad=(pad_h, 1), groups=c, act=getattr(orc, act), slope=slope if prelu else None)
+    conv = ops.Conv2d(wt, b, stride=both, pad=(pad_h, 1), groups=c, act=getattr(ops, act), slope=slope if prelu else None, in_hw=(h, w))
+    assert conv.plan.kind == 1 and conv.plan.Q >= 4
+    close(conv(torch.tensor(x, device=cuda)), ref)
+
+
 @pytest.mark.parametrize("i,o", [(256, 10), (512, 1000), (2048, 1000), (1280, 1000), (25088, 512), (37, 11), (25088, 511), (8192, 3), (8196, 5), (9001, 4),
                                  (16388, 1)])
 def test_dense_parity(cuda, i, o):
