@@ -150,8 +150,9 @@ void SchedulerFull3::requeue_or_finish(job::Job* job) {
     const auto end_time = std::chrono::steady_clock::now();
     const double length = std::chrono::duration<double, std::micro>(end_time - job->get_stage_start_time()).count();
     log_->add('L', job->get_id(), job->get_cur_stage(), 0, 0, 0, length);
+    // first stage first: a type's table of lengths grows at its end
     const unsigned span = job->get_cur_stage_span();
-    for (unsigned k = 0; k < span; ++k) server_->update_job_stage_length(job, (unsigned)job->get_cur_stage() - k, length / span);
+    for (unsigned s = (unsigned)job->get_cur_stage() + 1 - span; s <= (unsigned)job->get_cur_stage(); ++s) server_->update_job_stage_length(job, s, length / span);
 
     if (job->has_next()) {
         know_next_stage(job);

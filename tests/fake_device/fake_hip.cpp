@@ -171,6 +171,7 @@ void maybe_start_autorun() {
 }
 
 void enqueue(void* stream, Op op) {
+    if (!stream) return;  // the null stream's work is over at once
     std::lock_guard<std::mutex> lk(g_mtx);
     op.seq = g_seq++;
     reinterpret_cast<Stream*>(stream)->q.push_back(op);

@@ -5,7 +5,7 @@
 //   sched NAME streams N [extra K] [unfair X] [mem marker|hostfunc] [budget REGS SMEM THREADS BLOCKS] [batch B]
 //         [percu CUS XCDS REGS SMEM THREADS BLOCKS]   full3 with per-compute-unit placement over that topology
 //   client                      register a client                      -> "client ID"
-//   job PATH                    register a job type, grow its pool     -> "job TYPE"
+//   job PATH [SLOT]             register a job type (request slots of SLOT bytes), grow its pool     -> "job TYPE"
 //   launch TYPE [SLOT]          LAUNCH_JOB for slot SLOT of the pool
 //   step [N]                    run the oldest device operation to completion, N times
 //   start STREAM | finish STREAM   advance the head operation of a stream by one phase / to completion
@@ -13,6 +13,12 @@
 //   drain                       step until the device is idle
 //   put TYPE SLOT BYTE          fill the slot's input with BYTE;   get TYPE SLOT -> "out B0 B1 ..." (first 8 output bytes)
 //   log                         print the event log so far (also printed at exit)
+//   recordlog 0|1               stop / resume recording the event log;   profile on|off   switch the profiler's kernel records
+//   lengths TYPE                -> "lengths L0 L1 ...": the type's learned stage lengths, in microseconds
+//   issued                      -> "issued S0 S1* ...": the model stages launched since the last time, * = reports to the scheduler
+//
+// Jobs that run models (libjob_tvm_*.so) issue their launches through the functions at the end of this file instead of the
+// operator library's: a launch that reports becomes a kernel of the scripted device.
 
 #include <llis/job/context.h>
 #include <llis/ipc/name_format.h>
@@ -22,6 +28,11 @@
 #include <llis/server/scheduler_full3.h>
 #include <llis/server/server.h>
 
+#include "paella_hip.h"
+#include "paella_models.h"
+#include "paella_ops.h"
+
+#include <dlfcn.h>
 #include <fcntl.h>
 #include <sys/mman.h>
 #include <sys/socket.h>
@@ -32,6 +43,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <iostream>
+#include <map>
 #include <memory>
 #include <sstream>
 #include <string>
@@ -69,7 +81,8 @@ struct Harness {
 
     void poll(bool drain = true) {
         int idle = 0;
-        while (idle < 4) {
+        const int enough = server->get_event_log()->enabled() ? 4 : 64;  // without a log, turns that did something count as idle too
+        while (idle < enough) {
             const size_t before = server->get_event_log()->events().size();
             server->poll_once();
             ++polls;
@@ -92,6 +105,18 @@ struct Harness {
     }
 };
 
+// Stands for any job of a type where the server is asked about the type.
+struct TypeHandle : job::Job {
+    unsigned type = 0;
+    size_t get_input_size() override { return 0; }
+    size_t get_output_size() override { return 0; }
+    size_t get_param_size() override { return 0; }
+    void full_init(void*) override {}
+    void init(void*) override {}
+    void run_next() override {}
+    bool has_next() const override { return false; }
+};
+
 // Name of the request ring the server creates, kept for the exit paths that run no destructors.
 char g_c2s_object[128];
 
@@ -105,6 +130,8 @@ void on_fatal_signal(int sig) {
 }
 
 }  // namespace
+
+static std::string g_issued;  // reply of the next "issued"
 
 static unsigned long long g_hook_calls = 0;
 static void count_poll_hook() { ++g_hook_calls; }
@@ -196,6 +223,7 @@ int main() {
             shm_unlink(t.shm_name.c_str());
             t.in_size = 100;
             t.slot_size = 208;
+            in >> t.slot_size;
             h.types.push_back(t);
             std::printf("job %u\n", t.id);
         } else if (cmd == "launch") {
@@ -243,6 +271,28 @@ int main() {
             std::printf("out");
             for (int i = 0; i < 8; ++i) std::printf(" %u", out[i]);
             std::printf("\n");
+        } else if (cmd == "recordlog") {
+            int on = 0;
+            in >> on;
+            h.server->get_event_log()->enable(on != 0);
+        } else if (cmd == "profile") {
+            std::string on;
+            in >> on;
+            h.c2s->acquire_writer_lock();
+            h.c2s->write(MsgType::PROFILER_CMD);
+            h.c2s->write(on == "on" ? ProfilerMsgType::SET_RECORD_KERNEL_INFO : ProfilerMsgType::UNSET_RECORD_KERNEL_INFO);
+            h.c2s->release_writer_lock();
+            h.poll();
+        } else if (cmd == "lengths") {
+            TypeHandle of;
+            in >> of.type;
+            of.set_client_details(h.client_id, of.type);
+            std::printf("lengths");
+            for (double l : h.server->get_job_stage_lengths(&of)) std::printf(" %.6f", l);
+            std::printf("\n");
+        } else if (cmd == "issued") {
+            std::printf("issued%s\n", g_issued.c_str());
+            g_issued.clear();
         } else if (cmd == "log") {
             std::fputs(h.server->get_event_log()->to_text().c_str(), stdout);
         } else {
@@ -260,4 +310,41 @@ int main() {
         return 3;
     }
     return 0;
+}
+
+// ---- what the model jobs call (the executable's definitions come before the operator library's)
+namespace {
+
+std::map<paella_exec*, paella_model*> g_model_of;
+void* g_model_stream = nullptr;  // the model jobs' only queue
+
+template <typename F>
+F library(const char* name) {
+    static void* const lib = dlopen("libpaella_ops.so", RTLD_LAZY | RTLD_NOLOAD);  // loaded with the first such job
+    return reinterpret_cast<F>(dlsym(lib, name));
+}
+
+}  // namespace
+
+extern "C" int fake_hip_kernel_launch(void* stream, uint32_t job_id, unsigned nblocks);
+
+extern "C" __attribute__((visibility("default"))) int paella_direct_queue_shared(void** out) {
+    if (!g_model_stream) llis_hip_stream_create(&g_model_stream);
+    *out = g_model_stream;
+    return 0;
+}
+
+extern "C" __attribute__((visibility("default"))) int paella_direct_queue_set_ordered(void*, int) { return 0; }
+
+extern "C" __attribute__((visibility("default"))) int paella_exec_create(const paella_model* m, paella_exec** out) {
+    const int rc = library<int (*)(const paella_model*, paella_exec**)>("paella_exec_create")(m, out);
+    if (rc == 0) g_model_of[*out] = const_cast<paella_model*>(m);
+    return rc;
+}
+
+extern "C" __attribute__((visibility("default"))) int paella_exec_launch_stage(paella_exec* e, int stage, void* stream, uint32_t job_id, void* notifier) {
+    paella_launch_dims d;
+    library<int (*)(const paella_model*, int, paella_launch_dims*)>("paella_model_stage_dims")(g_model_of.at(e), stage, &d);
+    g_issued += " " + std::to_string(stage) + (notifier ? "*" : "");
+    return notifier ? fake_hip_kernel_launch(stream, job_id & ~PAELLA_JOB_ID_FLAGS, d.grid) : 0;
 }

@@ -1,0 +1,27 @@
+"""Stages issued several at a time (Context::is_uncrowded, Job::set_stage_span) on the scripted device: a model job as it is served, whose
+launches the harness takes in the operator library's place, under the real full3 scheduler."""
+import pytest
+
+from _fake import run_harness
+from paella_amd import serve
+
+MODEL, KERNELS = "tvm_mobilenet", 54
+GROUP = 8
+
+
+def serve_alone(body, **env):
+    """`body` with one model type registered, nobody recording stages; the replies of `issued` and `lengths` as lists."""
+    script = "sched full3 streams 8\nrecordlog 0\nclient\njob %s 700000\n" % serve.job_path(MODEL) + body
+    replies, _ = run_harness(script, PAELLA_STAGE_THREAD="0", **env)
+    return [r.split()[1:] for r in replies if r.startswith(("issued", "lengths"))]
+
+
+def test_a_group_fills_the_entries_of_its_own_stages():
+    """From an empty table: one entry per stage after the first request, each an equal share of its group's time."""
+    issued, lengths = serve_alone("launch 0 0\ndrain\nissued\nlengths 0\n")
+    assert [int(s.rstrip("*")) for s in issued] == list(range(KERNELS))
+    ends = [int(s[:-1]) for s in issued if s.endswith("*")]
+    assert ends == list(range(GROUP - 1, KERNELS, GROUP)) + [KERNELS - 1]
+    assert len(lengths) == 1 + KERNELS  # the input's copy, then the kernels
+    for first, last in zip([0] + [e + 1 for e in ends], ends):
+        assert len(set(lengths[1 + first:2 + last])) == 1
