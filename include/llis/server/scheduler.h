@@ -57,6 +57,9 @@ class Scheduler {
         log_ = server->get_event_log();
     }
     virtual void try_handle_block_start_finish() = 0;
+    // A request is about to become a job, which declares its first stage as it is made (what it reads from job::Context for that
+    // has to be of this moment).
+    virtual void before_new_job() {}
     virtual void handle_new_job(std::unique_ptr<job::Job> job) = 0;
     // No job is in flight: every job handed over has had its last stage's completion handled.
     virtual bool idle() const { return true; }

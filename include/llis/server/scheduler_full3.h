@@ -87,6 +87,7 @@ class SchedulerFull3 : public StreamPoolScheduler {
     SchedulerFull3(const SchedulerOptions& options, std::unique_ptr<GpuResources> per_cu);
 
     void set_server(Server* server) override;
+    void before_new_job() override;
     void handle_new_job(std::unique_ptr<job::Job> job) override;
 
   protected:
@@ -96,6 +97,7 @@ class SchedulerFull3 : public StreamPoolScheduler {
 
   private:
     void schedule_job();
+    void tell_jobs_of_company(unsigned num_jobs) const;
     void requeue_or_finish(job::Job* job);
     double take_priority(job::Job* job) const;
     void know_next_stage(job::Job* job);

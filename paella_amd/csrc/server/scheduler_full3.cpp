@@ -108,6 +108,13 @@ void SchedulerFull3::know_next_stage(job::Job* job) {
         if (!server_->has_job_stage_resource(job, s)) server_->set_job_stage_resource(job, s, 1);
 }
 
+// Before each moment at which a job declares a stage: when it is made, and when it is resumed.
+void SchedulerFull3::tell_jobs_of_company(unsigned num_jobs) const {
+    job::Context::set_uncrowded(num_jobs <= kUncrowded && !per_cu_ && !log_->enabled() && !profiler_->recording());
+}
+
+void SchedulerFull3::before_new_job() { tell_jobs_of_company(num_jobs_ + 1); }
+
 void SchedulerFull3::handle_new_job(std::unique_ptr<job::Job> owned) {
     if (!owned->has_next()) {
         server_->release_job_instance(std::move(owned));
@@ -235,7 +242,7 @@ void SchedulerFull3::schedule_job() {
         }
 
         job::Context::set_current_job(job);
-        job::Context::set_uncrowded(num_jobs_ <= kUncrowded && !per_cu_ && !log_->enabled() && !profiler_->recording());
+        tell_jobs_of_company(num_jobs_);
         profiler_->record_job_event(job->get_id(), Profiler::JobEvent::KERNEL_SUBMIT_START);
         {
             LLIS_PHASE_IF(is_mem, kLaunchCopy, kLaunch);

@@ -142,6 +142,7 @@ void Server::handle_launch_job() {
     c2s_channel_.read(&id);
     if (id >= registered_jobs_.size()) throw std::runtime_error("LAUNCH_JOB for an unknown job type");
     LLIS_PHASE_WARMUP_TICK();
+    scheduler_->before_new_job();
     scheduler_->handle_new_job(registered_jobs_[id]->create_instance());
 }
 

@@ -25,3 +25,20 @@ def test_a_group_fills_the_entries_of_its_own_stages():
     assert len(lengths) == 1 + KERNELS  # the input's copy, then the kernels
     for first, last in zip([0] + [e + 1 for e in ends], ends):
         assert len(set(lengths[1 + first:2 + last])) == 1
+
+
+def test_the_first_stage_is_declared_by_what_is_in_flight_now():
+    """A job without an input stage declares kernels as it is made: what an earlier job was told -- few in flight, nobody recording --
+    is not what it goes by."""
+    alone, recorded, unrecorded = serve_alone("launch 0 0\ndrain\nissued\nprofile on\nlaunch 0 0\ndrain\nissued\nprofile off\nlaunch 0 0\ndrain\nissued\n",
+                                              PAELLA_INPUT_RESIDENT="1")
+    assert alone[:GROUP] == [str(k) for k in range(GROUP - 1)] + ["%d*" % (GROUP - 1)]
+    assert recorded == ["%d*" % k for k in range(KERNELS)]
+    assert unrecorded == alone
+
+
+def test_a_fifth_job_declares_single_stages():
+    launches = "".join("launch 0 %d\n" % i for i in range(5))
+    first = serve_alone(launches + "issued\ndrain\n", PAELLA_INPUT_RESIDENT="1")[0]
+    group = [str(k) for k in range(GROUP - 1)] + ["%d*" % (GROUP - 1)]
+    assert first == group * 4 + ["0*"]
