@@ -72,6 +72,7 @@ class Job {
         deficit_counter_ = 0;
         cur_stage_ = -1;
         next_span_ = cur_span_ = 1;
+        next_reporting_ = 0;
     }
 
     void set_id(JobId id) {
@@ -99,6 +100,10 @@ class Job {
     // The declared stage does the work of this many consecutive ones, itself the last of them (1 until said otherwise).
     void set_stage_span(unsigned v) { next_span_ = v; }
     unsigned get_stage_span() const { return next_span_; }
+    // Workgroups whose messages end the declared stage, where those are not the declared ones: a stage that stands for several kernels
+    // declares the needs of the largest, and its last kernel reports.  What it was charged for is then given back when it is over.
+    void set_num_reporting_blocks(unsigned v) { next_reporting_ = v; }
+    unsigned get_num_reporting_blocks() const { return next_reporting_ ? next_reporting_ : next_.num_blocks; }
 
     bool is_mem() const { return is_mem_; }
     void set_is_mem() { is_mem_ = true; }
@@ -127,6 +132,8 @@ class Job {
     unsigned get_cur_smem_size_per_block() const { return cur_.smem_size_per_block; }
     unsigned get_cur_num_registers_per_thread() const { return cur_.num_registers_per_thread; }
     unsigned get_cur_stage_span() const { return cur_span_; }
+    // Each message of the stage stands for workgroups that it was charged for.
+    bool reports_charged_blocks() const { return reports_charged_; }
 
     bool is_running() const { return is_running_; }
     void unset_running() { is_running_ = false; }
@@ -136,8 +143,9 @@ class Job {
         is_running_ = true;
         cuda_stream_ = stream;
         cur_ = next_;
-        num_running_blocks_ = next_.num_blocks;
-        num_pending_blocks_ = next_.num_blocks;
+        num_running_blocks_ = num_pending_blocks_ = get_num_reporting_blocks();
+        reports_charged_ = next_reporting_ == 0;
+        next_reporting_ = 0;
         clear_predicted_smids();
         stage_start_time_ = Clock::now();
         cur_stage_ += (int)next_span_;
@@ -236,6 +244,8 @@ class Job {
     StageNeeds next_;
     StageNeeds cur_;
     unsigned next_span_ = 1, cur_span_ = 1;
+    unsigned next_reporting_ = 0;
+    bool reports_charged_ = true;
     bool is_mem_ = false;
     bool is_pre_notify_ = false;
     bool completes_itself_ = false;

@@ -28,6 +28,7 @@
 
 #include <llis/job/context.h>
 #include <llis/job/coroutine_job.h>
+#include <llis/server/sm_resources.h>
 
 #include "paella_hip.h"
 #include "paella_models.h"
@@ -91,10 +92,11 @@ class ModelJob : public llis::job::CoroutineJob {
         // model (ResNet-18's projections and its global pool) was measured too: 13.9 -> 12.8 k requests/s at saturation,
         // because a member that must wait for its predecessor stalls everything behind it in its queue.
         bool all_small = group_limit > 0;
-        for (int s = 0; s < num_stages_ && all_small; ++s) {
-            paella_launch_dims d;
+        dims_.resize((size_t)num_stages_);
+        for (int s = 0; s < num_stages_; ++s) {
+            paella_launch_dims& d = dims_[(size_t)s];
             paella_model_stage_dims(model_, s, &d);
-            all_small = (unsigned long)d.grid * d.block <= group_limit;
+            all_small = all_small && (unsigned long)d.grid * d.block <= group_limit;
         }
         group_end_.assign((size_t)num_stages_, 0);
         for (int s = 0; s < num_stages_; ++s) group_end_[(size_t)s] = all_small ? num_stages_ - 1 : s;
@@ -208,13 +210,16 @@ class ModelJob : public llis::job::CoroutineJob {
             // -> 1270 / 2370 / 3810, ResNet-18 3280 / 5920 / 9500 -> 5060 / 7960 / 12030.
             const bool group = uncrowded_stages_ > 1 && last == s && llis::job::Context::is_uncrowded();
             if (group) last = std::min(s + uncrowded_stages_, num_stages_) - 1;
-            paella_launch_dims d;
-            paella_model_stage_dims(model_, last, &d);  // the group is admitted and accounted as its last kernel
+            // Admitted and accounted as its last kernel, or, where no limit bounds the others, as the largest.
+            const paella_launch_dims& d = dims_[(size_t)(group ? largest(s, last) : last)];
             set_num_blocks(d.grid);
             set_num_threads_per_block(d.block);
             set_smem_size_per_block(d.lds_bytes);
             set_num_registers_per_thread(d.vgprs);
-            if (group) set_stage_span((unsigned)(last - s + 1));
+            if (group) {
+                set_stage_span((unsigned)(last - s + 1));
+                set_num_reporting_blocks(dims_[(size_t)last].grid);
+            }
             if (zero_out_ && last == num_stages_ - 1) set_pre_notify();
             yield();
             if (zero_in_ && s == 0) stage_small_input(io_ptr);
@@ -276,6 +281,24 @@ class ModelJob : public llis::job::CoroutineJob {
         std::memcpy(staging_, io_ptr, in_bytes_);
     }
 
+    // The kernel of first..last that takes the largest share of the device, by the resource it takes most of.
+    int largest(int first, int last) const {
+        using R = llis::server::SmResources;
+        int at = last;
+        double most = 0;
+        for (int k = first; k <= last; ++k) {
+            const paella_launch_dims& d = dims_[(size_t)k];
+            const double share = d.grid * std::max({(double)R::wg_threads(d.block) / (R::kSimdsPerCu * R::kMaxWavesPerSimd * R::kWaveLanes),
+                                                    (double)R::wg_regs(d.block, d.vgprs) / (R::kSimdsPerCu * R::kVgprsPerSimdLane * R::kWaveLanes),
+                                                    (double)R::wg_lds(d.lds_bytes) / (160 * 1024)});
+            if (share > most) {
+                most = share;
+                at = k;
+            }
+        }
+        return at;
+    }
+
     void* stream() { return reinterpret_cast<void*>(get_cuda_stream()); }
 
     static void staged(void* job) { llis::job::Context::post_mem_completion(static_cast<llis::job::Job*>(job)); }
@@ -303,6 +326,7 @@ class ModelJob : public llis::job::CoroutineJob {
     char* staging_ = nullptr;
     void* io_ptr_ = nullptr;
     int num_stages_ = 0;
+    std::vector<paella_launch_dims> dims_;  // per kernel
     std::vector<int> group_end_;   // per kernel: index of the last kernel of the group it is issued with
     bool direct_ = true;
     bool whole_job_direct_ = false;

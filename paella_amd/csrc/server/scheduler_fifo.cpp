@@ -58,7 +58,7 @@ void SchedulerFifo::schedule_job() {
         int stage = 0;
         while (job->has_next()) {
             const bool is_mem = job->is_mem();
-            const unsigned units = is_mem ? 1u : job->get_num_blocks();
+            const unsigned units = is_mem ? 1u : job->get_num_reporting_blocks();
             pr.remaining_blocks += units;
             if (!saw_pre_notify) {
                 pr.pre_notify_blocks += (int)units;

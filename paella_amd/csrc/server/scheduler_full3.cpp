@@ -190,9 +190,10 @@ void SchedulerFull3::handle_block_finish(job::Job* job, unsigned num) {
         give_stream(job);
         give_notifier(job);
     }
-    if (!per_cu_) gpu_resources_.release(job, (int)num);
+    const unsigned freed = job->reports_charged_blocks() ? num : stage_over ? job->get_cur_num_blocks() : 0;
+    if (!per_cu_) gpu_resources_.release(job, (int)freed);
     else if (job->reports_cu()) per_cu_->observe_block_finish(job, cur_smid_);
-    else per_cu_->release_predicted(job, num);
+    else per_cu_->release_predicted(job, freed);
     if (stage_over && !job->has_next()) retire(job);
     schedule_job();
 }

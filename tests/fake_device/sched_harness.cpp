@@ -15,7 +15,8 @@
 //   log                         print the event log so far (also printed at exit)
 //   recordlog 0|1               stop / resume recording the event log;   profile on|off   switch the profiler's kernel records
 //   lengths TYPE                -> "lengths L0 L1 ...": the type's learned stage lengths, in microseconds
-//   issued                      -> "issued S0 S1* ...": the model stages launched since the last time, * = reports to the scheduler
+//   issued                      -> "issued S0 S1* ...": the model stages launched since the last time, * = reports to the scheduler,
+//                                  and "needs W,T,L,R ...": workgroups, threads, LDS bytes and registers of each
 //
 // Jobs that run models (libjob_tvm_*.so) issue their launches through the functions at the end of this file instead of the
 // operator library's: a launch that reports becomes a kernel of the scripted device.
@@ -131,7 +132,7 @@ void on_fatal_signal(int sig) {
 
 }  // namespace
 
-static std::string g_issued;  // reply of the next "issued"
+static std::string g_issued, g_needs;  // replies of the next "issued"
 
 static unsigned long long g_hook_calls = 0;
 static void count_poll_hook() { ++g_hook_calls; }
@@ -291,8 +292,9 @@ int main() {
             for (double l : h.server->get_job_stage_lengths(&of)) std::printf(" %.6f", l);
             std::printf("\n");
         } else if (cmd == "issued") {
-            std::printf("issued%s\n", g_issued.c_str());
+            std::printf("issued%s\nneeds%s\n", g_issued.c_str(), g_needs.c_str());
             g_issued.clear();
+            g_needs.clear();
         } else if (cmd == "log") {
             std::fputs(h.server->get_event_log()->to_text().c_str(), stdout);
         } else {
@@ -346,5 +348,6 @@ extern "C" __attribute__((visibility("default"))) int paella_exec_launch_stage(p
     paella_launch_dims d;
     library<int (*)(const paella_model*, int, paella_launch_dims*)>("paella_model_stage_dims")(g_model_of.at(e), stage, &d);
     g_issued += " " + std::to_string(stage) + (notifier ? "*" : "");
+    g_needs += " " + std::to_string(d.grid) + "," + std::to_string(d.block) + "," + std::to_string(d.lds_bytes) + "," + std::to_string(d.vgprs);
     return notifier ? fake_hip_kernel_launch(stream, job_id & ~PAELLA_JOB_ID_FLAGS, d.grid) : 0;
 }

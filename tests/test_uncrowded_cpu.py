@@ -1,19 +1,18 @@
 """Stages issued several at a time (Context::is_uncrowded, Job::set_stage_span) on the scripted device: a model job as it is served, whose
 launches the harness takes in the operator library's place, under the real full3 scheduler."""
-import pytest
-
 from _fake import run_harness
+from oracle import sched as oracle_sched
 from paella_amd import serve
 
 MODEL, KERNELS = "tvm_mobilenet", 54
 GROUP = 8
 
 
-def serve_alone(body, **env):
-    """`body` with one model type registered, nobody recording stages; the replies of `issued` and `lengths` as lists."""
-    script = "sched full3 streams 8\nrecordlog 0\nclient\njob %s 700000\n" % serve.job_path(MODEL) + body
+def serve_alone(body, sched="", want=("issued", "lengths"), **env):
+    """`body` with one model type registered, nobody recording stages; the wanted replies as lists."""
+    script = "sched full3 streams 8 %s\nrecordlog 0\nclient\njob %s 700000\n" % (sched, serve.job_path(MODEL)) + body
     replies, _ = run_harness(script, PAELLA_STAGE_THREAD="0", **env)
-    return [r.split()[1:] for r in replies if r.startswith(("issued", "lengths"))]
+    return [r.split()[1:] for r in replies if r.startswith(want)]
 
 
 def test_a_group_fills_the_entries_of_its_own_stages():
@@ -39,6 +38,23 @@ def test_the_first_stage_is_declared_by_what_is_in_flight_now():
 
 def test_a_fifth_job_declares_single_stages():
     launches = "".join("launch 0 %d\n" % i for i in range(5))
-    first = serve_alone(launches + "issued\ndrain\n", PAELLA_INPUT_RESIDENT="1")[0]
+    first = serve_alone(launches + "issued\ndrain\n", "extra 48", PAELLA_INPUT_RESIDENT="1")[0]
     group = [str(k) for k in range(GROUP - 1)] + ["%d*" % (GROUP - 1)]
     assert first == group * 4 + ["0*"]
+
+
+def test_a_group_is_charged_as_its_largest_kernel():
+    """Registers for two of the first group's last kernel, but not for two of its largest: the second job waits for the first one's
+    group, and what that was charged for is given back, so that both are answered (the harness fails otherwise)."""
+    needs = serve_alone("launch 0 0\ndrain\nissued\n", want=("needs",), PAELLA_INPUT_RESIDENT="1")[0]
+    regs = []
+    for need in needs:
+        blocks, threads, lds, vgprs = (int(v) for v in need.split(","))
+        regs.append(blocks * oracle_sched.wg_charge(oracle_sched.Stage(False, blocks, threads, lds, vgprs))[0])
+    largest, last = max(regs[:GROUP]), regs[GROUP - 1]
+    assert 2 * last < largest
+    plenty = 1 << 40
+    first, rest = serve_alone("launch 0 0\nlaunch 0 1\nissued\ndrain\nissued\n", "extra 0 budget %d %d %d %d" % (largest + last, plenty, plenty, plenty),
+                              ("issued",), PAELLA_INPUT_RESIDENT="1")
+    assert first == [str(k) for k in range(GROUP - 1)] + ["%d*" % (GROUP - 1)]
+    assert len(rest) == 2 * KERNELS - GROUP
