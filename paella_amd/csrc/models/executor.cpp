@@ -74,11 +74,13 @@ struct paella_exec {
     unsigned inputs = 0;         // handed over by paella_exec_set_input so far
     // The pass as a graph, once it has been asked for often enough; recorded again when the input or output moves.
     void* graph = nullptr;
+    bool unrecordable = false;   // it was tried, and costs several passes' launches
     std::vector<void*> old_graphs;
     unsigned passes = 0;         // since the buffers last moved
     void buffers_moved() {
         if (graph) old_graphs.push_back(graph);  // it may still be running
         graph = nullptr;
+        unrecordable = false;
         passes = 0;
     }
     float* ptr(const View& v) const {
@@ -764,8 +766,10 @@ int paella_exec_forward(paella_exec* e, void* stream) {
     constexpr unsigned kPlainPasses = 3;
     constexpr size_t kMostGraphs = 8;  // a program that moves the buffers again and again gets plain launches
     if (e->m->stages.size() >= kMinGraph && ++e->passes > kPlainPasses && in_company(e) && paella::forward_graph_allowed(stream)) {
-        if (!e->graph && e->old_graphs.size() < kMostGraphs)
+        if (!e->graph && !e->unrecordable && e->old_graphs.size() < kMostGraphs) {
             e->graph = paella::forward_graph_record([](void* target, void* arg) { return launch_all(static_cast<paella_exec*>(arg), target); }, e);
+            e->unrecordable = !e->graph;
+        }
         replay = e->graph != nullptr;
     }
     const int rc = replay ? paella::forward_graph_replay(e->graph, stream) : launch_all(e, stream);
