@@ -45,6 +45,8 @@ _direct_queues = set()
 def _stream(stream):
     if stream is None:
         return _torch_stream()
+    if isinstance(stream, ctypes.c_void_p):
+        stream = stream.value
     if stream in _direct_queues:
         # nothing orders such a queue behind torch's stream, and a call is quick enough to overtake a fill that is still under way there
         torch.cuda.current_stream().synchronize()
