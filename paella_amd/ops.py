@@ -70,9 +70,9 @@ class Conv2d:
         dh, dw = _pair(dil)
         h, wd = in_hw
         self.desc = ConvDesc(cg * groups, h, wd, k, r, s, sh, sw, ph, pw, dh, dw, groups, act, lo, hi)
-        self.plan = ConvPlan()
-        check(lib.paella_conv2d_plan(ctypes.byref(self.desc), int(has_residual), tile_hint, ctypes.byref(self.plan)),
-              "paella_conv2d_plan")
+        plan = ConvPlan()
+        check(lib.paella_conv2d_plan(ctypes.byref(self.desc), int(has_residual), tile_hint, ctypes.byref(plan)), "paella_conv2d_plan")
+        self.plan = plan
         blob = np.zeros(self.plan.blob_bytes, dtype=np.uint8)
         check(lib.paella_conv2d_pack(ctypes.byref(self.plan), w.ctypes.data, blob.ctypes.data), "paella_conv2d_pack")
         self.blob = torch.from_numpy(blob).to(device)
@@ -80,10 +80,17 @@ class Conv2d:
         self.slope = None if slope is None else torch.tensor(np.asarray(slope, np.float32), device=device)
         self.workspace = torch.zeros(max(self.plan.workspace_bytes, 4) // 4, dtype=torch.int32, device=device) if self.plan.workspace_bytes else None
         self.lib = lib
-        # what every call passes on, looked up once
-        self._plan_ref = ctypes.byref(self.plan)
         self._launch, self._launch_transformed = lib.paella_conv2d_launch, lib.paella_conv2d_launch_transformed
-        self._in_shape, self._out_shape = (1, self.plan.d.C, self.plan.d.H, self.plan.d.W), (1, self.plan.d.K, self.plan.P, self.plan.Q)
+
+    @property
+    def plan(self):
+        return self._plan
+
+    @plan.setter
+    def plan(self, plan):
+        # what every call passes on, looked up once per plan (its extents are not changed in place)
+        self._plan, self._plan_ref = plan, ctypes.byref(plan)
+        self._in_shape, self._out_shape = (1, plan.d.C, plan.d.H, plan.d.W), (1, plan.d.K, plan.P, plan.Q)
 
     def takes_input_transform(self):
         return bool(self.lib.paella_conv2d_plan_takes_input_transform(ctypes.byref(self.plan)))
