@@ -11,7 +11,8 @@ namespace paella {
 
 // Lets the host address `p`, the start of an allocation of device memory; false where the platform does not.
 bool host_map_device(void* p);
-// Host to mapped device memory; the data is on its way ahead of any doorbell rung afterwards.
+// Host to mapped device memory (dst 64-byte aligned); a kernel whose doorbell is rung afterwards, by whatever thread the request is handed
+// to, reads the data.
 void host_store(void* dst, const void* src, size_t bytes);
 // The same by the library's copy thread, as paella_host_copy_submit.
 int host_store_submit(void* dst, const void* src, size_t bytes, void (*done)(void*), void* arg);

@@ -1,11 +1,17 @@
 // The executor (csrc/models/executor.cpp) on the scripted device, launches and graphs taken by the functions below (an executable's
 // definitions come before a library's).  `exec_check refuse|allow`: two requests of one model pass in turn, on buffers that move once;
 // prints how often a recording was tried and how many passes were launched kernel by kernel and replayed.
+// `exec_check copies`: host_store and host_load (csrc/hip/host_io.h) on host memory, up to the last byte in front of a page that may not
+// be touched; prints the number of lengths checked.
 
+#include "../../paella_amd/csrc/hip/host_io.h"
 #include "paella_models.h"
+
+#include <sys/mman.h>
 
 #include <cstdio>
 #include <cstring>
+#include <vector>
 
 namespace {
 bool g_refuse = false;
@@ -30,7 +36,33 @@ extern "C" int paella_exec_launch_stage(paella_exec*, int, void*, uint32_t, void
     return 0;
 }
 
+static int check_copies() {
+    constexpr size_t kRoom = 16384;
+    char* const room = static_cast<char*>(mmap(nullptr, kRoom + 4096, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0));
+    if (room == MAP_FAILED || mprotect(room + kRoom, 4096, PROT_NONE) != 0) return 1;
+    std::vector<char> src(kRoom + 1), back(kRoom);
+    for (size_t i = 0; i < src.size(); ++i) src[i] = (char)(i * 7 + i / 251);
+    int checked = 0;
+    for (size_t n : {0, 1, 4, 15, 16, 17, 63, 64, 65, 127, 784 * 4, 4095, 4096, 4097, 4160, 4161, 12288, 16383, 16384}) {
+        char* const dst = room + (kRoom - n) / 64 * 64;
+        std::memset(room, 0x55, kRoom);
+        paella::host_store(dst, src.data() + 1, n);
+        if (std::memcmp(dst, src.data() + 1, n) != 0) return 1;
+        for (char* p = room; p < room + kRoom; ++p)
+            if ((p < dst || p >= dst + n) && *p != 0x55) return 1;
+        std::fill(back.begin(), back.end(), (char)0x33);
+        paella::host_load(back.data(), dst, n);
+        if (std::memcmp(back.data(), src.data() + 1, n) != 0) return 1;
+        for (size_t i = n; i < kRoom; ++i)
+            if (back[i] != 0x33) return 1;
+        ++checked;
+    }
+    std::printf("%d\n", checked);
+    return 0;
+}
+
 int main(int argc, char** argv) {
+    if (argc > 1 && std::strcmp(argv[1], "copies") == 0) return check_copies();
     g_refuse = argc > 1 && std::strcmp(argv[1], "refuse") == 0;
     paella_model* m = nullptr;
     paella_exec* e[2] = {nullptr, nullptr};

@@ -1,4 +1,4 @@
-"""When the executor records a pass (paella_exec_forward), on the scripted device: tests/fake_device/exec_check.cpp."""
+"""When the executor records a pass (paella_exec_forward), on the scripted device, and the host's copies: tests/fake_device/exec_check.cpp."""
 import os
 import subprocess
 
@@ -21,3 +21,7 @@ def test_the_fourth_pass_in_company_is_recorded():
     """(A pass that this machine holds up for 150 us is not in company and goes out plain.)"""
     for turn, (recorded, plain, replayed) in enumerate(counts("allow"), 1):
         assert recorded == 2 * turn and plain >= 6 * turn and replayed > 0 and plain + replayed == 20 * turn
+
+
+def test_host_copies_touch_their_bytes_and_no_others():
+    assert counts("copies") == [(19,)]
