@@ -96,3 +96,34 @@ def test_inputs_off_the_lines_of_a_streaming_store_and_memory_of_earlier_request
             ex.forward()
             np.testing.assert_array_equal(ex.get_output(), plain(name, np.ascontiguousarray(x)))
             ex.close()
+
+
+@pytest.mark.parametrize("name", ["mnist", "squeezenet1_1"])
+def test_input_and_output_wait_for_passes_on_a_blocking_stream(cuda, name):
+    """Where the host moves them itself they wait for what a copy on the null stream waits for: a pass still queued on a stream that
+    orders with it, behind 20 ms of other work."""
+    from paella_amd import _abi, models
+    hip, rng = _abi.hip(), np.random.default_rng(10)
+    x, y = (rng.standard_normal(models.io_bytes(name)[0] // 4).astype(np.float32) for _ in range(2))
+    want_x, want_y = plain(name, x), plain(name, y)
+    busy, ex = models.Exec("arcfaceresnet100"), models.Exec(name)
+    s = ctypes.c_void_p()
+    _abi.check(hip.hipStreamCreate(ctypes.byref(s)))
+    busy.set_input(np.zeros(busy.in_bytes // 4, np.float32))
+    for _ in range(3):  # past the inputs that the runtime copies
+        ex.set_input(x)
+        ex.forward(s)
+        np.testing.assert_array_equal(ex.get_output(), want_x)
+    for late in (False, True):
+        ex.set_input(y)
+        for _ in range(20):
+            busy.forward(s)
+        ex.forward(s)
+        if late:
+            ex.set_input(x)  # not under the pass that reads y
+        np.testing.assert_array_equal(ex.get_output(), want_y)
+        ex.forward(s)
+        np.testing.assert_array_equal(ex.get_output(), want_x if late else want_y)
+    _abi.check(hip.llis_hip_stream_destroy(s))
+    ex.close()
+    busy.close()
