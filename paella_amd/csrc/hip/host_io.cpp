@@ -46,8 +46,8 @@ void load_lines(char* dst, const char* src, size_t bytes) {
 // that the doorbell announces lies in host memory, and the answer to its fetch comes down the same link, on which completions do not
 // overtake posted writes.  So the packet processor cannot have the packet of a kernel before the device has the kernel's input.
 // Inputs of more than a page do not rest on that: one read goes behind the last store, which no read overtakes on its way to the device,
-// and is waited for.  It costs 1.2 to 1.6 us, nothing beside their 10 to 25 (Inception-v3 alone 405 -> 403 us), but 5 % of a request of the
-// small CNN (4 KB: 27.6 -> 29.3 us without a server, 25.3 -> 26.5 us through one).
+// and is waited for.  It costs 1.2 to 2 us: under 1 % of a request without a server (ResNet-18 166.5 -> 168, Inception-v3 403 -> 405), nothing
+// on the copy thread, but 5 % of a request of the small CNN (4 KB: 27.6 -> 29.3 us without a server, 25.3 -> 26.5 us through one).
 constexpr size_t kPostedOnly = 4096;
 
 bool wide() {
