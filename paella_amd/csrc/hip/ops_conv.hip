@@ -1489,6 +1489,7 @@ extern "C" int paella_conv2d_plan(const paella_conv_desc* d, int has_residual, i
         plan->dims.block = 256;
         plan->dims.lds_bytes = 0;
         plan->dims.vgprs = 32;
+        plan->small = 1;
         return 0;
     }
     return PAELLA_ENOSUP;
@@ -2347,8 +2348,15 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         a.out_bytes = (unsigned)std::min<uint64_t>(elements * 4, 0xFFFFFFFFu);
     }
     if (pack_hold_dw(a, plan->dims.grid, stream)) return 0;
-    // Strips of four outputs: the kernel's window is fixed, and its workgroups are not the plan's, so nobody may count them.
-    if (a.fast && !nf && !residual && d.pad_w == 1 && d.dil_h == 1 && d.dil_w == 1 && d.stride_w <= 2 && plan->Q >= 4) {
+    // Strips of four outputs: the kernel's window is fixed, and its workgroups are not the plan's, so nobody may count them.  Only where the
+    // plan gives a thread several outputs too (from kDwWideFrom on): a smaller layer is over in one trip to memory, and a quarter of the
+    // workgroups, each longer, takes more time, not less.  One launch behind the other, one output per thread -> strips, over 140 shapes of
+    // 16 to 960 channels: 0.1 to 0.9 us more below the line (960 x 7 x 7 2.12 -> 2.44 us, 576 x 14 x 14 with stride 2 2.15 -> 2.79, 16 x 112 x 112
+    // with stride 2, 50 176 outputs, 2.15 -> 3.06); and above it, where the plain form has four outputs per thread a grid stride apart, 0.2 to 5 us
+    // less (384 x 14 x 14 3.15 -> 2.43, 16 x 80 x 80 2.95 -> 2.56, 96 x 112 x 112 with stride 2 4.86 -> 4.35, 192 x 150 x 150 15.6 -> 10.5).
+    const bool wide = (uint64_t)plan->dims.grid * 256 < (uint64_t)d.C * plan->P * plan->Q;
+    if ((plan->small > 1 || (plan->small == 1 && wide)) && a.fast && !nf && !residual && d.pad_w == 1 && d.dil_h == 1 && d.dil_w == 1 &&
+        d.stride_w <= 2 && plan->Q >= 4) {
         a.strips_row = (plan->Q + 3) / 4;
         a.strips = d.C * plan->P * a.strips_row;
         a.div_strip = fast_div((unsigned)a.strips_row);

@@ -357,8 +357,26 @@ def test_depthwise_strips_match_the_oracle(cuda, c, h, w, stride, pad_h, act):
     both = stride if isinstance(stride, tuple) else (stride, stride)
     ref = orc.conv2d(x, wt, b, stride=both, pad=(pad_h, 1), groups=c, act=getattr(orc, act), slope=slope if prelu else None)
     conv = ops.Conv2d(wt, b, stride=both, pad=(pad_h, 1), groups=c, act=getattr(ops, act), slope=slope if prelu else None, in_hw=(h, w))
-    assert conv.plan.kind == 1 and conv.plan.Q >= 4
-    close(conv(torch.tensor(x, device=cuda)), ref)
+    assert conv.plan.kind == 1 and conv.plan.Q >= 4 and conv.plan.small == 1
+    xd = torch.tensor(x, device=cuda)
+    plain = conv(xd)  # too few outputs for strips, unless they are asked for
+    conv.plan.small = 2
+    strips = torch.full_like(plain, float("nan"))
+    conv(xd, out=strips)
+    close(strips, ref)
+    assert torch.equal(strips, plain)
+
+
+@pytest.mark.parametrize("c,h,w,stride", [(335, 14, 14, 1), (1311, 10, 5, 1), (335, 28, 28, 2), (2, 512, 64, 1)])
+def test_depthwise_strips_from_65536_outputs_on(cuda, c, h, w, stride):
+    """Around the line from which strips are taken (the first channel or row past it, and whole): the bits of the plain kernel."""
+    from paella_amd import ops
+    conv = ops.Conv2d(rnd(c, 1, 3, 3, scale=0.3), rnd(c, scale=0.1), stride=stride, pad=1, groups=c, act=ops.ACT_RELU6, in_hw=(h, w))
+    assert 65536 <= c * conv.plan.P * conv.plan.Q < 65536 + 1000 and conv.plan.dims.grid == -(-c * conv.plan.P * conv.plan.Q // 1024)
+    x = torch.tensor(rnd(1, c, h, w), device=cuda)
+    strips = conv(x)
+    conv.plan.small = 0
+    assert torch.equal(strips, conv(x))
 
 
 @pytest.mark.parametrize("i,o", [(256, 10), (512, 1000), (2048, 1000), (1280, 1000), (25088, 512), (37, 11), (25088, 511), (8192, 3), (8196, 5), (9001, 4),
