@@ -105,7 +105,6 @@ class ModelJob : public llis::job::CoroutineJob {
         // notification ring (fifo2, full3): the queues have no ordering of their own, and fifo relies on the stream.
         const char* resident = std::getenv("PAELLA_INPUT_RESIDENT");
         input_resident_ = resident && std::strcmp(resident, "1") == 0;
-        if (!input_resident_) set_shareable();  // nothing of a request outlives it
         const char* zc = std::getenv("PAELLA_ZERO_COPY_BYTES");
         const size_t zero_copy_limit = zc ? std::strtoull(zc, nullptr, 10) : 65536;
         zero_in_ = !input_resident_ && in_bytes_ <= zero_copy_limit && paella_exec_bind_input(exec_, staging_) == 0;
@@ -126,6 +125,11 @@ class ModelJob : public llis::job::CoroutineJob {
                 direct_ = whole_job_direct_ = false;
             }
         }
+        // Nothing of a request outlives it.  Only with direct dispatch, where instances that outlive their client spare the next one's first
+        // requests 0.1 to 0.3 ms each (2 to 3 ms of p99 in every third run of 10 000 requests at 48 k/s).  With HIP launches they cost the
+        // small CNN's p99 in the 9 : 1 mix 10 to 25 % at 17 k requests/s, and the rate at a p99 of 260 us and 7.93 ms falls from 16.7 to
+        // 14.5 k (medians of 12 searches each; the saturation rate stays); what the runtime does with the older allocations is not known.
+        if (!input_resident_ && direct_) set_shareable();
         // (Sixteen at once are another 3 to 5 % for a request alone, but twice as long in a newcomer's way; four lose 10 %.)
         uncrowded_stages_ = direct_ && !timed_ && group_limit > 0 ? 8 : 1;
         // Conv launches of different requests share launches (paella_pack_enable) unless PAELLA_PACK=0: the serving thread

@@ -17,6 +17,7 @@
 //   lengths TYPE                -> "lengths L0 L1 ...": the type's learned stage lengths, in microseconds
 //   issued                      -> "issued S0 S1* ...": the model stages launched since the last time, * = reports to the scheduler,
 //                                  and "needs W,T,L,R ...": workgroups, threads, LDS bytes and registers of each
+//   instances                   -> "instances N": model job instances made so far
 //
 // Jobs that run models (libjob_tvm_*.so) issue their launches through the functions at the end of this file instead of the
 // operator library's: a launch that reports becomes a kernel of the scripted device.
@@ -132,6 +133,7 @@ void on_fatal_signal(int sig) {
 
 }  // namespace
 
+static unsigned g_instances = 0;
 static std::string g_issued, g_needs;  // replies of the next "issued"
 
 static unsigned long long g_hook_calls = 0;
@@ -291,6 +293,8 @@ int main() {
             std::printf("lengths");
             for (double l : h.server->get_job_stage_lengths(&of)) std::printf(" %.6f", l);
             std::printf("\n");
+        } else if (cmd == "instances") {
+            std::printf("instances %u\n", g_instances);
         } else if (cmd == "issued") {
             std::printf("issued%s\nneeds%s\n", g_issued.c_str(), g_needs.c_str());
             g_issued.clear();
@@ -340,6 +344,7 @@ extern "C" __attribute__((visibility("default"))) int paella_direct_queue_set_or
 
 extern "C" __attribute__((visibility("default"))) int paella_exec_create(const paella_model* m, paella_exec** out) {
     const int rc = library<int (*)(const paella_model*, paella_exec**)>("paella_exec_create")(m, out);
+    ++g_instances;
     if (rc == 0) g_model_of[*out] = const_cast<paella_model*>(m);
     return rc;
 }

@@ -1,5 +1,5 @@
-"""Stages issued several at a time (Context::is_uncrowded, Job::set_stage_span) on the scripted device: a model job as it is served, whose
-launches the harness takes in the operator library's place, under the real full3 scheduler."""
+"""Model jobs as they are served, under the real full3 scheduler on the scripted device (the harness takes their launches in the operator
+library's place): stages issued several at a time (Context::is_uncrowded, Job::set_stage_span), and instances shared by registrations."""
 from _fake import run_harness
 from oracle import sched as oracle_sched
 from paella_amd import serve
@@ -58,3 +58,10 @@ def test_a_group_is_charged_as_its_largest_kernel():
                               ("issued",), PAELLA_INPUT_RESIDENT="1")
     assert first == [str(k) for k in range(GROUP - 1)] + ["%d*" % (GROUP - 1)]
     assert len(rest) == 2 * KERNELS - GROUP
+
+
+def test_idle_instances_are_shared_with_direct_dispatch_only():
+    """A second registration of the same library finds the first one's instance; with HIP launches it makes its own."""
+    second = "job %s 700000\nlaunch 0 0\ndrain\nlaunch 1 0\ndrain\nlaunch 1 0\ndrain\ninstances\n" % serve.job_path(MODEL)
+    assert serve_alone(second, want=("instances",)) == [["1"]]
+    assert serve_alone(second, want=("instances",), PAELLA_DISPATCH="hip") == [["2"]]
