@@ -59,7 +59,7 @@ def log(*a):
 # HBM-side bytes per conv launch (mean over the conv launches of one forward pass), from FETCH_SIZE / WRITE_SIZE
 # counter passes of `bench.py --counter-pass MODEL` scaled by the copy-kernel calibration (FETCH_SIZE x 2.0,
 # WRITE_SIZE x 1.0); counters cannot be collected from inside this process, so the figures are carried here.
-CONV_TRAFFIC_BYTES_PER_LAUNCH = {"inception_v3": 8.63e6, "resnet18": 6.97e6, "resnet50": 7.06e6, "mobilenetv2": 1.84e6}
+CONV_TRAFFIC_BYTES_PER_LAUNCH = {"inception_v3": 8.53e6, "resnet18": 6.99e6, "resnet50": 7.10e6, "mobilenetv2": 1.84e6}
 
 
 def under_counter_collection():
@@ -430,7 +430,7 @@ def roofline_of(rl, model):
     achieved = rl["conv_flops"] / (rl["conv_us"] * 1e-6) / 1e12
     return {"bound": "mfma", "achieved": achieved, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / FP32_MFMA_PEAK_TFLOPS,
             "traffic": CONV_TRAFFIC_BYTES_PER_LAUNCH.get(model),
-            "kernel": "conv_mfma_kernel and its grouped forms (all %d conv launches of one %s forward pass, one at a time on an idle device)" % (rl["conv_launches"], model),
+            "kernel": "conv_mfma_kernel, conv_small_kernel and their grouped forms (all %d conv launches of one %s forward pass, one at a time on an idle device)" % (rl["conv_launches"], model),
             "flops_per_launch_avg": rl["conv_flops"] / rl["conv_launches"], "us_per_launch_avg": rl["conv_us"] / rl["conv_launches"],
             "algorithmic_bytes_per_launch_avg": rl["by_op"]["conv"]["bytes"] / rl["conv_launches"]}
 
@@ -951,7 +951,7 @@ def headline(out):
         if k in out:
             line[k] = out[k]
     r = {k: rf.get(k) for k in ("bound", "achieved", "peak", "unit", "frac", "traffic") if k in rf}
-    r["kernel"] = "conv_mfma_kernel (+ grouped forms), Inception-v3's conv launches one at a time"
+    r["kernel"] = "conv_mfma_kernel, conv_small_kernel (+ grouped forms), Inception-v3's conv launches one at a time"
     for k in ("flops_per_launch_avg", "us_per_launch_avg", "algorithmic_bytes_per_launch_avg", "peak_measured", "empty_kernel_us"):
         if k in rf:
             r[k] = rf[k]
