@@ -7,7 +7,9 @@
 // memory and a read back, 2 to 3 us of the launch's 5 to 8.  Here a tile is (16 * MI) channels x 16 pixels
 // (v_mfma_f32_16x16x4_f32, the same rate per cycle), four or two times as many of them, the whole reduction stays in one
 // workgroup and its partial tiles, 1 KB each, meet in LDS.  Each wave loads twice the operands per matrix instruction, which a
-// launch that fills the device several times over pays for and a lone small layer does not.
+// launch that fills the device several times over pays for and a lone small layer does not.  By counters, 256->256 3x3 on 14x14: twice the
+// look-ups of a compute unit's vector cache (11 600 against 5600), whose data unit is busy for 6.9 of 11.0 us (4.3 of 8.1); 768->192 on 17x17:
+// half of them (1900 against 3800), since four times as many compute units have work, and 2.3 of 4.9 us (4.0 of 6.2).
 //
 // The result has the bits of the 32 x 32 kernel.  The fp32 matrix instructions add their products one after the other, each
 // with one rounding, in ascending order of the reduction index they are given; v_mfma_f32_32x32x2 is given the pairs (k, k + 4),

@@ -1321,6 +1321,11 @@ constexpr size_t kMaxSplitTiles = 16384;  // counters at the head of a split-k w
 // the larger tile) the waves' turns from part to part cost more than the exchange through memory (256->256 3x3 on 14x14, 32
 // parts: 8.1 -> 10.6 us); long reductions are bound by the same vector cache; and the larger tile does not pay for a
 // reduction of one chunk per wave (64->384 pointwise on 14x14: 3.0 -> 3.2 us).
+// Launches that few others accompany take the same form: passes replayed as graphs on two / four / eight streams, 32 x 32 throughout -> this
+// rule, Inception-v3 696 / 1032 / 1827 -> 630 / 956 / 1814 us, ResNet-50 581 / 869 / 1539 -> 534 / 800 / 1436, DenseNet-121 1179 / 1482 / 2550
+// -> 1122 / 1405 / 2390, MobileNetV2 432 / 683 / 920 -> 417 / 657 / 890; groups of a server's requests with one / two / four in flight, in
+// requests/s, Inception-v3 2209 / 3620 / 5250 -> 2338 / 3830 / 5318, DenseNet-121 1244 / 2268 / 3950 -> 1330 / 2480 / 4287, ResNet-50 2667 /
+// 4475 / 6330 -> 2754 / 4673 / 6514.  ResNet-18, GoogLeNet and ArcFace-R100 within 1 % either way.
 int choose_small(const paella_conv_plan* const* plans, int n) {
     long tiles1 = 0, tiles2 = 0, chunks = 0;
     int parts = 0, shortest = 1 << 30;
