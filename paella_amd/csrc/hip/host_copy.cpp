@@ -91,8 +91,12 @@ class CopyWorker {
                 queue_.pop_front();
             }
             pending_.fetch_sub(1, std::memory_order_acq_rel);
-            if (item.to_device) paella::host_store(item.dst, item.src, item.bytes);
-            else std::memcpy(item.dst, item.src, item.bytes);
+            if (item.to_device) {
+                paella::host_store(item.dst, item.src, item.bytes);
+                paella::host_settle(item.dst, item.bytes);  // another thread launches
+            } else {
+                std::memcpy(item.dst, item.src, item.bytes);
+            }
             item.done(item.arg);
         }
     }

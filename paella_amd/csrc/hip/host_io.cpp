@@ -40,16 +40,6 @@ void load_lines(char* dst, const char* src, size_t bytes) {
     }
 }
 
-// When is the data there?  Stores through the aperture are posted: the core is done with them before they are in memory.  The fence keeps
-// them ahead of everything this core, or one that it hands the request to, stores to the device later; on the link, posted writes keep
-// their order, so they arrive ahead of the doorbell, and ahead of a direct-dispatch kernel's arguments, which take the same way.  The packet
-// that the doorbell announces lies in host memory, and the answer to its fetch comes down the same link, on which completions do not
-// overtake posted writes.  So the packet processor cannot have the packet of a kernel before the device has the kernel's input.
-// Inputs of more than a page do not rest on that: one read goes behind the last store, which no read overtakes on its way to the device,
-// and is waited for.  It costs 1.2 to 2 us: under 1 % of a request without a server (ResNet-18 166.5 -> 168, Inception-v3 403 -> 405), nothing
-// on the copy thread, but 5 % of a request of the small CNN (4 KB: 27.6 -> 29.3 us without a server, 25.3 -> 26.5 us through one).
-constexpr size_t kPostedOnly = 4096;
-
 bool wide() {
     static const bool has = __builtin_cpu_supports("avx512f");
     return has;
@@ -65,9 +55,11 @@ void host_store(void* dst, const void* src, size_t bytes) {
     const size_t done = wide() ? store_512(d, s, bytes) : store_128(d, s, bytes);
     std::memcpy(d + done, s + done, bytes - done);
     _mm_sfence();
-    if (bytes <= kPostedOnly) return;
+}
+
+void host_settle(const void* dst, size_t bytes) {
     _mm_mfence();
-    (void)*static_cast<const volatile char*>(d + bytes - 1);
+    if (bytes) (void)*(static_cast<const volatile char*>(dst) + bytes - 1);
     _mm_lfence();
 }
 

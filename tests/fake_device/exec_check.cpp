@@ -1,7 +1,7 @@
 // The executor (csrc/models/executor.cpp) on the scripted device, launches and graphs taken by the functions below (an executable's
 // definitions come before a library's).  `exec_check refuse|allow`: two requests of one model pass in turn, on buffers that move once;
 // prints how often a recording was tried and how many passes were launched kernel by kernel and replayed.
-// `exec_check copies`: host_store and host_load (csrc/hip/host_io.h) on host memory, up to the last byte in front of a page that may not
+// `exec_check copies`: host_store, host_settle and host_load (csrc/hip/host_io.h) on host memory, up to the last byte in front of a page that may not
 // be touched; prints the number of lengths checked.
 
 #include "../../paella_amd/csrc/hip/host_io.h"
@@ -47,6 +47,7 @@ static int check_copies() {
         char* const dst = room + (kRoom - n) / 64 * 64;
         std::memset(room, 0x55, kRoom);
         paella::host_store(dst, src.data() + 1, n);
+        paella::host_settle(dst, n);
         if (std::memcmp(dst, src.data() + 1, n) != 0) return 1;
         for (char* p = room; p < room + kRoom; ++p)
             if ((p < dst || p >= dst + n) && *p != 0x55) return 1;
