@@ -2355,10 +2355,11 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
     if (pack_hold_dw(a, plan->dims.grid, stream)) return 0;
     // Strips of four outputs: the kernel's window is fixed, and its workgroups are not the plan's, so nobody may count them.  Only where the
     // plan gives a thread several outputs too (from kDwWideFrom on): a smaller layer is over in one trip to memory, and a quarter of the
-    // workgroups, each longer, takes more time, not less.  One launch behind the other, one output per thread -> strips, over 140 shapes of
-    // 16 to 960 channels: 0.1 to 0.9 us more below the line (960 x 7 x 7 2.12 -> 2.44 us, 576 x 14 x 14 with stride 2 2.15 -> 2.79, 16 x 112 x 112
-    // with stride 2, 50 176 outputs, 2.15 -> 3.06); and above it, where the plain form has four outputs per thread a grid stride apart, 0.2 to 5 us
-    // less (384 x 14 x 14 3.15 -> 2.43, 16 x 80 x 80 2.95 -> 2.56, 96 x 112 x 112 with stride 2 4.86 -> 4.35, 192 x 150 x 150 15.6 -> 10.5).
+    // workgroups, each longer, takes more time, not less.  One launch behind the other, one output per thread -> strips, over 200 shapes of
+    // 16 to 8192 channels and rows of 4 to 150 outputs: 0.1 to 1 us more below the line (960 x 7 x 7 2.12 -> 2.44 us, 576 x 14 x 14 with stride 2
+    // 2.15 -> 2.79, 18 x 118 x 119 with stride 2, 63 720 outputs, 2.12 -> 3.08); and above it, where the plain form has four outputs per thread a
+    // grid stride apart, 0.1 to 5 us less (4096 x 4 x 4 3.11 -> 2.41, 16 x 80 x 80 2.95 -> 2.56, 96 x 112 x 112 with stride 2 4.86 -> 4.35, 192 x
+    // 150 x 150 15.6 -> 10.5) but for one (923 x 11 x 91 with stride 2 3.62 -> 3.81).
     const bool wide = (uint64_t)plan->dims.grid * 256 < (uint64_t)d.C * plan->P * plan->Q;
     if ((plan->small > 1 || (plan->small == 1 && wide)) && a.fast && !nf && !residual && d.pad_w == 1 && d.dil_h == 1 && d.dil_w == 1 &&
         d.stride_w <= 2 && plan->Q >= 4) {
