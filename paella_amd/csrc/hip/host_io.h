@@ -20,8 +20,8 @@ bool host_map_device(void* p);
 void host_store(void* dst, const void* src, size_t bytes);
 // Waits until what host_store wrote is in memory: a read does not overtake the stores on its way to the device.  For a thread whose
 // stores another core may follow with a doorbell within a microsecond, so that nothing rests on the order between two cores' stores.
-// 1.2 to 2 us, nothing measurable on the copy thread (ResNet-18 under load 216.1 -> 216.0 ms for 4096 requests); the calling thread's own
-// launches do without (a small CNN's request 27.6 -> 29.3 us with it, ResNet-18's 166.5 -> 168, Inception-v3's 403 -> 405).
+// 1.2 to 2 us on the copy thread: a lone served request of ResNet-18 163 -> 164.5 us, nothing under load (4096 of them 216.1 -> 216.0 ms).  The
+// calling thread's own launches do without (a small CNN's request 27.6 -> 29.3 us with it, ResNet-18's 166.5 -> 168, Inception-v3's 403 -> 405).
 void host_settle(const void* dst, size_t bytes);
 // The same by the library's copy thread, as paella_host_copy_submit.
 int host_store_submit(void* dst, const void* src, size_t bytes, void (*done)(void*), void* arg);
