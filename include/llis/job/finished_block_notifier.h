@@ -121,6 +121,30 @@ class FinishedBlockNotifier {
         if (timed && timing_is_on()) send_block_time_first();
         announce<false>(&agg_counter_end_, 0, job_id, num_blocks);
     }
+
+    // For a workgroup that does the work of `count` of the num_blocks workgroups the scheduler counts (not under per-workgroup
+    // timing): the messages are those that `count` calls of end_from_one_lane would send.
+    __device__ __forceinline__ void end_many_from_one_lane(JobId job_id, unsigned num_blocks, unsigned count) {
+        if (count == 0) return;
+        const unsigned batch = batch_mask_ + 1;
+        const unsigned before = atomicAdd(&agg_counter_end_, count), total = before + count;
+        // the last one leaves the counter at zero, ahead of the message that lets the next kernel start
+        if (total == num_blocks) {
+            atomicExch(&agg_counter_end_, 0u);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        InstrumentInfo info;
+        info.is_start = 0;
+        info.job_id = job_id;
+        for (unsigned at = (before & ~batch_mask_) + batch; at <= total; at += batch) {
+            info.num = (uint8_t)batch;
+            gpu2sched_channel_.write_relaxed(info);
+        }
+        if (total == num_blocks && (total & batch_mask_) != 0) {
+            info.num = (uint8_t)(total & batch_mask_);
+            gpu2sched_channel_.write_relaxed(info);
+        }
+    }
 #endif
 
     // Allocates `num` notifiers in device memory, all bound to the given ring (and, when given, to the ring

@@ -83,7 +83,8 @@ typedef struct paella_conv_plan {
                                     3-wide filter reads them as neighbouring input pixels (see the kernel's operand fetch) */
     int small;                   /* 1: a launch without a notifier that is not packed with others may take tiles of 16 or 32 channels
                                     x 16 pixels where those are faster (same bits, set for tile_hint = 0 or with 1<<20 in it); 2, 3:
-                                    it takes the former / the latter (tuning sweeps and tests, reductions of at most 64 parts); 0: never.
+                                    it takes the former / the latter (tuning sweeps and tests, reductions of at most 64 parts), 4: workgroups of two
+                                    32 x 32 tiles, which 1 takes in launches that fill the device (same bits); 0: never.
                                     Depthwise: 1: strips of four outputs per thread where those are faster (same bits); 2: wherever the
                                     kernel for them applies; 0: never */
 } paella_conv_plan;

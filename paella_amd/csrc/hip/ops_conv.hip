@@ -138,9 +138,14 @@ struct PreOp {
 // PRE: kPreBounded with a lower bound (ReLU), kPreUnbounded without (a batch-norm alone: the four maxima per chunk are not
 // computed at all -- a vector instruction costs a sixteenth of a matrix instruction of pipe time).
 constexpr int kPreNone = 0, kPreBounded = 1, kPreUnbounded = 2;
-template <int MI, int NI, int KW, bool TAP_MAJOR, int PRE = kPreNone, int DEPTH = 0, bool PW = false>
-__device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid, const PreOp pre = PreOp{nullptr, nullptr, 0.f}) {
+// TALL: one of the tiles that conv_tall_tile has worked out, 64 rows high (MI 2, or 1 where the last rows are a single tile).
+struct Tile {
+    int n, m, split;
+};
+template <int MI, int NI, int KW, bool TAP_MAJOR, int PRE = kPreNone, int DEPTH = 0, bool PW = false, bool TALL = false>
+__device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid, const PreOp pre = PreOp{nullptr, nullptr, 0.f}, const Tile given = Tile{0, 0, 0}) {
     static_assert(!PRE || (TAP_MAJOR && MI * NI == 1), "the input transform is built for the smallest tile in tap-major order");
+    static_assert(!TALL || NI == 1, "a tall workgroup's tiles lie one under the other");
     static_assert(!PW || TAP_MAJOR, "the pointwise shortcut belongs to the tap-major order");
     // A grouped launch starts every conv at a multiple of eight workgroups (see align_start): the ids between the end of one
     // problem and the start of the next belong to no tile and report to nobody.
@@ -168,7 +173,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
                      "+s"(a.div_tm.mul), "+s"(a.div_tm.one));
     }
     TL_STAMP(8);
-    if (bid >= (unsigned)(a.n_tiles_n * a.n_tiles_m * a.splits)) return;
+    if (!TALL && bid >= (unsigned)(a.n_tiles_n * a.n_tiles_m * a.splits)) return;
     const unsigned hook_blocks = p.hook_blocks ? p.hook_blocks : gridDim.x;
     paella::hook_entry(p.notifier, p.job_id, hook_blocks);
     // Waves of this workgroup whose result stores have been acknowledged (see the end of this function); cleared here, and
@@ -181,7 +186,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
     float* red = reinterpret_cast<float*>(smem);
     // With a fused input transform, behind the partial tiles' region (waves leave the loop at different times): 64 bytes of zeros,
     // then per four input channels their four scales and their four shifts, 32 bytes.
-    char* const ptab = smem + (KW > 1 ? KW * MI * NI * 16 * 64 * 4 : 0);
+    char* const ptab = smem + (KW > 1 ? KW * (TALL ? 1 : MI) * NI * 16 * 64 * 4 : 0);
     // A thread's first two entries of that table are requested here, so that they travel while the tile is decoded (entries
     // past the last channel read as zero and are not written).
     constexpr int kPreEarly = 2;
@@ -218,8 +223,8 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
     // XCDs, each with its own L2; the ids that land on one XCD are given a contiguous run of the work list, and
     // the list is ordered so that a run shares what the layer reads most of: the same slab of weights (layers
     // with small feature maps) or neighbouring pixel tiles, whose 3x3 halos overlap (layers with large ones).
-    int tile_n, tile_m, split;
-    {
+    int tile_n = given.n, tile_m = given.m, split = given.split;
+    if (!TALL) {
         const unsigned total = (unsigned)(a.n_tiles_n * a.n_tiles_m * a.splits);
         const unsigned xcd = bid & 7u, j = bid >> 3;
         const unsigned q = total >> 3, r = total & 7u;
@@ -240,7 +245,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
         if (__builtin_amdgcn_readfirstlane(a.fast_div)) decode([](unsigned x, unsigned, const FastDiv& f) { return quot_fast(x, f); });
         else decode([](unsigned x, unsigned d, const FastDiv&) { return x / d; });
     }
-    const int m0 = tile_m * (32 * MI);
+    const int m0 = tile_m * (TALL ? 64 : 32 * MI);
     const int n0 = tile_n * (32 * NI);
     TL_STAMP(9);
 
@@ -319,7 +324,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
     // columns.  The host packs the weights to match: per filter row, CB chunks of the unpaired column (eight channels each), then
     // 2 CB chunks of the pair (four channels of both columns each), so a row is 3 CB chunks either way and chunk c is still
     // (unit c / CB, block c % CB).  The host has checked that both columns lie inside the image for every output pixel.
-    const int pair_s0 = (TAP_MAJOR && !PW && MI * NI == 1) ? p.pair_s0 : -1;
+    const int pair_s0 = (TAP_MAJOR && !PW && NI == 1) ? p.pair_s0 : -1;
     const int pair_delta = (negkk & (p.dw * 4)) - kk4hw;  // from the lane's offset for a plain chunk to that for a paired one
     int seg_chan0 = 0, seg_chans = 8;  // first channel of the current unit's chunks, channels per chunk; wave-uniform
     bool seg_pair = false;
@@ -455,6 +460,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
 
     constexpr int NACC = MI * NI * 16;
     constexpr int RPW = NACC / KW;
+    constexpr int RPT = TALL ? RPW / MI : RPW;  // of each tile where the tiles are summed one after the other
     // (a variant with a deeper operand pipeline keeps its registers for the chunks in flight)
     // (nor does the variant with an input transform: its scale and shift operands take the registers, and with the epilogue's
     // operands requested after the loop it fits the 64 registers of eight waves per SIMD)
@@ -468,11 +474,11 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
     // pixels past P*Q read as zero and their stores are dropped, without a compare on the vector unit.
     // (K * P * Q * 4 < 2^31 is a condition of the plan.)
     auto row_of = [&](int w, int rr) {
-        const int r = w * RPW + rr;
+        const int r = (rr / RPT) * 16 + w * RPT + rr % RPT;
         const int e = r & 15;
         return ((r >> 4) / NI) * 32 + (e >> 2) * 8 + (e & 3);
     };
-    auto lane_off = [&](int rr) { return lane_offs[((wave * RPW + rr) >> 4) % NI]; };
+    auto lane_off = [&](int rr) { return lane_offs[NI == 1 ? 0 : ((wave * RPW + rr) >> 4) % NI]; };
     const int rows_tile = max(p.K - m0, 0);  // channels from this tile's first one to the last that exists (may exceed the tile)
     const float* const res_tile = p.residual ? p.residual + (size_t)m0 * p.PQ : nullptr;
     float* const y_tile = p.y + (size_t)m0 * p.PQ;
@@ -531,7 +537,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
     // 44 registers, so that depth 3 and 4 fit eight waves per SIMD at 52 and 60: 76.8 and 76.4 against 78.1 TFLOP/s with the
     // device full.  Requesting one input dword per chunk instead of four -- wrong results, timing only -- gives 84 against 77:
     // the load path is worth at most 9 % here, and half again on the stride-2 layers, whose lanes use every other pixel of a line.)
-    constexpr int D = DEPTH ? DEPTH : (MI * NI == 1) ? 2 : 4;
+    constexpr int D = DEPTH ? DEPTH : (MI * NI == 1 || TALL) ? 2 : 4;
     // first: the accumulators hold nothing yet, the first matrix instruction into each takes zero as its addend
     auto compute = [&](const Frag<MI, NI>& f, auto first) {
         const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -678,6 +684,22 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
                     if ((mi * NI + ni) * 16 + e < RPW) mine[(mi * NI + ni) * 16 + e] = acc[mi][ni][e];
+    } else if (TALL) {
+        // One tile after the other through the same 32 KB: with room for both, only two workgroups would fit a compute unit.
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+            if (mi > 0) __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[(wave * 16 + e) * 64 + lane] = acc[mi][0][e];
+            __syncthreads();
+#pragma unroll
+            for (int rr = 0; rr < RPT; ++rr) {
+                float v = red[(wave * RPT + rr) * 64 + lane];
+#pragma unroll
+                for (int w = 1; w < KW; ++w) v += red[(w * 16 + wave * RPT + rr) * 64 + lane];
+                mine[mi * RPT + rr] = v;
+            }
+        }
     } else {
         if (!TAP_MAJOR) __syncthreads();  // every wave is done with the table before the partial tiles overwrite it
 #pragma unroll
@@ -717,7 +739,9 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
         const int tile = tile_m * p.n_tiles_n + tile_n;
         unsigned* const counter = p.ws_counters + tile;
         // the tile's partial tiles, [split][NACC][64 lanes]: one descriptor, a lane's offset is its lane number
-        float* const partials = p.ws_partials + (size_t)tile * nsplits * (NACC * 64);
+        // (a tall workgroup's tiles side by side, those of the rows above it before them, whether it has two or one)
+        float* const partials = TALL ? p.ws_partials + (size_t)(tile_m * 2 * p.n_tiles_n + tile_n * MI) * nsplits * 1024
+                                     : p.ws_partials + (size_t)tile * nsplits * (NACC * 64);
         const unsigned partials_len = (unsigned)nsplits * (NACC * 256u);
         const __amdgpu_buffer_rsrc_t pres = __builtin_amdgcn_make_buffer_rsrc((void*)partials, 0, partials_len, 0x00027000);
         const int lane4 = lane * 4;
@@ -789,7 +813,10 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
             if (lane == 0) before = __hip_atomic_fetch_add(&waves_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             last = __builtin_amdgcn_readfirstlane(before) == (unsigned)KW - 1;
         }
-        if (last && lane == 0) p.notifier->end_from_one_lane(p.job_id & ~PAELLA_JOB_ID_FLAGS, (p.job_id & PAELLA_JOB_ID_TIME_BLOCKS) != 0, hook_blocks);
+        if (last && lane == 0) {
+            if (TALL) p.notifier->end_many_from_one_lane(p.job_id & ~PAELLA_JOB_ID_FLAGS, hook_blocks, MI);
+            else p.notifier->end_from_one_lane(p.job_id & ~PAELLA_JOB_ID_FLAGS, (p.job_id & PAELLA_JOB_ID_TIME_BLOCKS) != 0, hook_blocks);
+        }
     }
 }
 
@@ -806,6 +833,37 @@ __global__ __launch_bounds__(64 * KW, (MI * NI == 1 && KW == 8 && DEPTH == 0) ? 
     const ConvArgs& p = (&args)[idx];
     if (TAP_MAJOR && p.pointwise) conv_tile<MI, NI, KW, TAP_MAJOR, kPreNone, DEPTH, TAP_MAJOR>(p, blockIdx.x);
     else conv_tile<MI, NI, KW, TAP_MAJOR, kPreNone, DEPTH>(p, blockIdx.x);
+}
+
+// Workgroups of two 32 x 32 tiles, one under the other, for launches that fill the device (kTallFrom says which).  What bounds those is a
+// compute unit's vector cache: per 32 reduction steps a wave's sixteen dword loads of inputs and four 16-byte loads of weights take it some
+// 450 cycles, 1800 for the four waves that have the 1024 cycles of a SIMD's matrix instructions to hide them.  Two tiles share the inputs:
+// 560 cycles to twice the matrix instructions.  Two tiles also share a wave's prologue.  The tiles' sums go through LDS one after the other
+// and the pipeline is two chunks deep, so that three workgroups fit a compute unit (75 registers, 32 KB); with room for two only, at a depth
+// of two or three chunks, 4 and 6 % less.  Same bits as two workgroups of one tile.  Four streams of one layer each, one tile -> two per
+// workgroup, TFLOP/s: 64->64 3x3 on 504x56 97 -> 108, 128->128 on 532x28 122 -> 135, 256->256 on 532x14 116 -> 134, 512->512 on 448x7 109 ->
+// 137, 128->256 stride 2 91 -> 124, 1x7 160->160 111 -> 127, pointwise 768->192 106 -> 112, 2048->320 117 -> 133, 64->256 40 -> 50.
+// (Eight tiles per workgroup that read all operands from LDS: 91 to 132, and workgroups too few and too long for a served launch.)
+__device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned bid) {
+    const unsigned gm = (unsigned)(p.n_tiles_m + 1) >> 1, total = (unsigned)p.n_tiles_n * gm * (unsigned)p.splits;
+    if (bid >= total) return;
+    const unsigned xcd = bid & 7u, q = total >> 3, r = total & 7u;
+    const unsigned at = xcd * q + (xcd < r ? xcd : r) + (bid >> 3);
+    const bool slabs = p.slab_major != 0;
+    const unsigned a = quot_fast(at, p.div_w), b = at - a * (slabs ? (unsigned)p.n_tiles_n : gm * (unsigned)p.splits);
+    const unsigned rest = slabs ? a : b;
+    Tile t;
+    t.n = (int)(slabs ? b : a);
+    t.split = (int)quot_fast(rest, p.div_tm);
+    t.m = (int)(rest - (unsigned)t.split * gm);
+    const PreOp none = PreOp{nullptr, nullptr, 0.f};
+    if (t.m * 2 + 1 < p.n_tiles_m) {
+        if (p.pointwise) conv_tile<2, 1, 8, true, kPreNone, 0, true, true>(p, bid, none, t);
+        else conv_tile<2, 1, 8, true, kPreNone, 0, false, true>(p, bid, none, t);
+    } else {
+        if (p.pointwise) conv_tile<1, 1, 8, true, kPreNone, 0, true, true>(p, bid, none, t);
+        else conv_tile<1, 1, 8, true, kPreNone, 0, false, true>(p, bid, none, t);
+    }
 }
 
 #include "conv_small.h"
@@ -907,7 +965,7 @@ union GroupMember {
     __host__ __device__ GroupMember() {}
 };
 
-enum MemberKind : unsigned { kMemberConv = 0, kMemberPool = 1, kMemberDense = 2 };
+enum MemberKind : unsigned { kMemberConv = 0, kMemberPool = 1, kMemberDense = 2, kMemberTall = 3 };
 
 struct ConvGroupArgs {
     unsigned start[kPackMax];  // first workgroup id of each member; 0xFFFFFFFF for unused entries
@@ -946,6 +1004,39 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_group_kern
     }
     if (TAP_MAJOR && g.m[idx].conv.pointwise) conv_tile<1, 1, KW, TAP_MAJOR, false, 0, TAP_MAJOR>(g.m[idx].conv, bid);
     else conv_tile<1, 1, KW, TAP_MAJOR>(g.m[idx].conv, bid);
+}
+
+__global__ __launch_bounds__(512, 6) void conv_tall_kernel(ConvArgs args) {
+    int idx = 0;
+    asm volatile("" : "+s"(idx));
+    conv_tall_tile((&args)[idx], blockIdx.x);
+}
+
+// The group kernel for members in the tall form, others beside them.
+__global__ __launch_bounds__(512, 6) void conv_tall_group_kernel(ConvGroupArgs g) {
+    int idx = 0;
+    unsigned first = g.start[0];
+#pragma unroll
+    for (int i = 1; i < kPackMax; ++i)
+        if (blockIdx.x >= g.start[i]) {
+            idx = i;
+            first = g.start[i];
+        }
+    const unsigned bid = blockIdx.x - first;
+    const unsigned kind = (g.kinds >> (2 * idx)) & 3u;
+    if (kind == kMemberTall) {
+        conv_tall_tile(g.m[idx].conv, bid);
+    } else if (kind == kMemberPool) {
+        const paella::PoolArgs& p = g.m[idx].pool;
+        const unsigned blocks = p.hook_blocks ? p.hook_blocks : gridDim.x;
+        paella::hook_entry(p.notifier, p.job_id, blocks);
+        paella::pool_element(p, (int)(bid * 512 + threadIdx.x));
+        paella::hook_exit(p.notifier, p.job_id, blocks);
+    } else if (g.m[idx].conv.pointwise) {
+        conv_tile<1, 1, 8, true, kPreNone, 0, true>(g.m[idx].conv, bid);
+    } else {
+        conv_tile<1, 1, 8, true>(g.m[idx].conv, bid);
+    }
 }
 
 constexpr int kMaxGroupWithPool = 3;  // convs of one call that also carries a pooling operator
@@ -1589,7 +1680,7 @@ int fill_args(const paella_conv_plan* plan, const float* x, const void* blob_dev
 int small_form(const paella_conv_plan* const* plans, const ConvArgs* const* args, int n) {
     for (int i = 0; i < n; ++i)
         if (!plans[i]->small || args[i]->notifier || !args[i]->fast_div) return 0;
-    if (n == 1 && plans[0]->small > 1) return plans[0]->small - 1;
+    if (n == 1 && plans[0]->small > 1) return plans[0]->small > 3 ? 0 : plans[0]->small - 1;
     return choose_small(plans, n);
 }
 
@@ -1641,6 +1732,27 @@ void add_kernel_resources(const void* fn, paella_launch_dims* dims) {
     }
 }
 
+// Workgroups of one tile from which on a launch takes those of two tiles (conv_tall_tile): three per compute unit.  Below, the device holds
+// all of them at once, and half as many that take twice as long make the launch longer.  One launch alone, one tile -> two: 196 workgroups
+// 5.8 -> 8.3 us, 392 8.3 -> 8.6, 588 11.0 -> 13.1, 676 8.2 -> 8.1, 784 14.1 -> 13.5, 784 (pointwise) 5.0 -> 4.6, 948 17.3 -> 17.4, 1352 13.3 ->
+// 12.5.  Served, several problems per launch, never / from 1280 / 1024 / 768 / 512 / 128 / 2: ResNet-18 216 / 212 / 207 / 206 / 207 / 206 / 205 ms,
+// MobileNetV2 : ResNet-50 188 / 184 / 183 / 182 / 182 / 182 / 181, small CNN : Inception-v3 163 / 162 / 162 / 162 / 165 / 171 / 170.
+constexpr unsigned kTallFrom = 768;
+
+// Workgroups of a conv in the tall form (two tiles of 32 rows each), 0 where it has none; and its arguments, from those of the plan's own kernel.
+unsigned tall_grid(const paella_conv_plan* plan, const ConvArgs& a) {
+    if (!plan->k_order || plan->kw != 8 || plan->mi != 1 || plan->ni != 1 || plan->depth || !a.fast_div || a.n_tiles_m < 2 || a.slab_major > 1) return 0;
+    return (unsigned)(a.n_tiles_n * ((a.n_tiles_m + 1) / 2) * a.splits);
+}
+
+ConvArgs tall_args(const ConvArgs& a) {
+    ConvArgs t = a;
+    const unsigned gm = (unsigned)(a.n_tiles_m + 1) / 2;
+    t.div_w = fast_div(a.slab_major ? (unsigned)a.n_tiles_n : gm * (unsigned)a.splits);
+    t.div_tm = fast_div(gm);
+    return t;
+}
+
 typedef void (*ConvGroupKernel)(ConvGroupArgs);
 
 ConvGroupKernel pick_group_kernel(int kw, int k_order) {
@@ -1685,10 +1797,10 @@ unsigned align_start(unsigned next) { return (next + 7u) & ~7u; }
 
 // One launch of the group kernel over the first n members of g (their start[] and kinds filled; the rest marked
 // unused here).
-int launch_group_args(ConvGroupArgs& g, int n, int kw, int k_order, unsigned grid, unsigned dyn_lds, void* stream) {
+int launch_group_args(ConvGroupArgs& g, int n, int kw, int k_order, unsigned grid, unsigned dyn_lds, void* stream, bool tall = false) {
     for (int i = n; i < kPackMax; ++i) g.start[i] = 0xFFFFFFFFu;
     g.reserved = 0;
-    ConvGroupKernel kern = pick_group_kernel(kw, k_order);
+    ConvGroupKernel kern = tall ? conv_tall_group_kernel : pick_group_kernel(kw, k_order);
     if (!kern) return PAELLA_EINVAL;
     if (int rc = allow_lds(reinterpret_cast<const void*>(kern), dyn_lds)) return rc;
     paella::launch_used(kern, dim3(grid), dim3(64u * (unsigned)kw), dyn_lds, reinterpret_cast<hipStream_t>(stream),
@@ -1710,6 +1822,7 @@ struct PackItem {
     unsigned dyn_lds = 0;
     ConvArgs args[kMaxGroup];
     unsigned grids[kMaxGroup];
+    unsigned tall_grids[kMaxGroup];    // of the tall form, 0 where a conv has none
     paella::PoolArgs pool;
     unsigned pool_grid = 0;
     int members() const { return n + (has_pool ? 1 : 0); }
@@ -1856,6 +1969,8 @@ bool pack_hold(const paella_conv_plan* const* plans, const ConvArgs* args, int n
     for (int i = 0; i < n; ++i) {
         it.args[i] = args[i];
         it.grids[i] = plans[i]->dims.grid;
+        // (its workgroups send no start messages and no time samples)
+        it.tall_grids[i] = (args[i].job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START ? tall_grid(plans[i], args[i]) : 0;
         it.grid += plans[i]->dims.grid;
         it.dyn_lds = std::max(it.dyn_lds, plans[i]->dims.lds_bytes);
     }
@@ -1885,15 +2000,26 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
         unsigned grid = 0, dyn_lds = 0;
         size_t i = done;
         int total = 0;
-        for (; i < list.items.size() && total + list.items[i].members() <= kPackMax; ++i) total += list.items[i].members();
+        unsigned tall_total = 0;
+        for (; i < list.items.size() && total + list.items[i].members() <= kPackMax; ++i) {
+            total += list.items[i].members();
+            for (int c = 0; c < list.items[i].n; ++c) tall_total += list.items[i].tall_grids[c] ? list.items[i].grids[c] : 0;
+        }
+        const bool tall = tall_total >= kTallFrom;
         g.kinds = 0;
         for (size_t k = done; k < i; ++k) {  // the convs of every item first ...
             const PackItem& it = list.items[k];
             for (int c = 0; c < it.n; ++c) {
                 grid = align_start(grid);
-                g.m[n].conv = it.args[c];
                 g.start[n] = grid;
-                grid += it.grids[c];
+                if (tall && it.tall_grids[c]) {
+                    g.m[n].conv = tall_args(it.args[c]);
+                    g.kinds |= kMemberTall << (2 * n);
+                    grid += it.tall_grids[c];
+                } else {
+                    g.m[n].conv = it.args[c];
+                    grid += it.grids[c];
+                }
                 ++n;
             }
             dyn_lds = std::max(dyn_lds, it.dyn_lds);
@@ -1914,15 +2040,14 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
             break;
         }
         if (n == 1) {  // nothing to share the launch with: the plain kernel, whose argument block is a quarter of the group's
-            ConvKernel kern = pick_kernel(1, 1, kw, k_order);
-            g.m[0].conv.hook_blocks = grid;
+            ConvKernel kern = g.kinds ? conv_tall_kernel : pick_kernel(1, 1, kw, k_order);
             rc = allow_lds(reinterpret_cast<const void*>(kern), dyn_lds);
             if (rc == 0) {
                 paella::launch(kern, dim3(grid), dim3(64u * (unsigned)kw), dyn_lds, reinterpret_cast<hipStream_t>(target), g.m[0].conv);
                 rc = (int)hipGetLastError();
             }
         } else {
-            rc = launch_group_args(g, n, kw, k_order, grid, dyn_lds, target);
+            rc = launch_group_args(g, n, kw, k_order, grid, dyn_lds, target, tall);
         }
         if (rc != 0) {
             failed = true;
@@ -2319,6 +2444,10 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         if (plan->mi == 1 && plan->ni == 1 && !plan->depth && pack_hold(&plan, &a, 1, stream)) return 0;
         SmallArgs small;
         unsigned grid = 0;
+        if (!nf && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom)) && (grid = tall_grid(plan, a)) != 0) {
+            paella::launch(conv_tall_kernel, dim3(grid), dim3(512), plan->dims.lds_bytes, st, tall_args(a));
+            return (int)hipGetLastError();
+        }
         const ConvArgs* one = &a;
         const int mi = small_form(&plan, &one, 1);
         if (mi && fill_small(plan, a, mi, small, &grid)) {

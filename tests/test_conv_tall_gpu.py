@@ -1,0 +1,102 @@
+"""Workgroups of two 32 x 32 tiles (conv_tall_tile): the bits of workgroups of one, alone and packed, and each job's notifier sees the
+workgroups that its plan counts."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from test_conv_small_gpu import reference, rnd
+from test_pack_gpu import NO_START, ring  # noqa: F401
+from test_ring_gpu import decode
+
+pytestmark = pytest.mark.gpu
+
+# C, K, H, W, (R, S), stride, pad, tile hint (0: the plan's own choice of waves and splits)
+EDGES = [
+    (64, 33, 1, 1, (1, 1), 1, 0, 0x0113),     # a second tile of one row, one pixel, a chunk per wave
+    (72, 64, 5, 7, (1, 1), 1, 0, 0x0113),     # nine chunks over eight waves of two: three of them without any
+    (64, 65, 4, 8, (3, 3), 1, 1, 0),          # three tiles: the last rows are a single one
+    (64, 96, 11, 3, (3, 3), 1, 1, 0x2113),    # ... with the reduction split four ways; 33 pixels
+    (128, 128, 9, 9, (3, 3), 2, 1, 0x1113),   # paired filter columns, two splits
+    (128, 160, 8, 8, (3, 3), 2, 0, 0),
+    (96, 100, 9, 9, (1, 7), 1, (0, 3), 0),
+    (96, 64, 11, 11, (1, 1), 2, 0, 0),        # pointwise with a stride
+    (512, 128, 7, 7, (3, 3), 1, 1, 0),        # the plan's own eight splits
+]
+
+
+@pytest.mark.parametrize("case", EDGES)
+def test_two_tiles_give_the_bits_of_one(cuda, case):
+    from paella_amd import ops
+    c, k, h, w, (r, s), stride, pad, hint = case
+    rng = np.random.default_rng(c * 1000 + k)
+    wt, b, x = rnd(rng, k, c, r, s), rnd(rng, k), rnd(rng, 1, c, h, w)
+    act = ops.ACT_PRELU if k % 2 else ops.ACT_RELU
+    slope = rnd(rng, k) if act == ops.ACT_PRELU else None
+    conv = ops.Conv2d(wt, b, stride=stride, pad=pad, act=act, slope=slope, in_hw=(h, w), has_residual=True, tile_hint=hint)
+    assert conv.plan.kw == 8
+    res = rnd(rng, 1, k, conv.plan.P, conv.plan.Q)
+    xd, rd = torch.tensor(x, device=cuda), torch.tensor(res, device=cuda)
+    conv.plan.small = 0
+    want = conv(xd, residual=rd)
+    conv.plan.small = 4
+    for _ in range(2):  # the second finds the counters of a split reduction as the first left them
+        out = torch.full_like(want, float("nan"))
+        assert torch.equal(conv(xd, residual=rd, out=out), want)
+    # n products and their sum in fp32, each rounded once: an error of at most n * 2^-24 of the sum of their sizes
+    ref = reference(x, wt, b, stride, pad, res, slope, int(act))
+    size = reference(np.abs(x), np.abs(wt), np.abs(b), stride, pad, np.abs(res), None, 0)
+    assert ((out.cpu().double() - ref).abs() <= (c * r * s + 2) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("k, h", [(64, 97), (96, 91)])  # 592 and 780 workgroups of one tile: below the rule's line and above it
+def test_a_launch_by_itself_takes_two_tiles_where_it_fills_the_device(cuda, k, h):
+    from paella_amd import ops
+    rng = np.random.default_rng(h)
+    conv = ops.Conv2d(rnd(rng, k, 64, 1, 1), rnd(rng, k), act=ops.ACT_RELU, in_hw=(h, h))
+    x = torch.tensor(rnd(rng, 1, 64, h, h), device=cuda)
+    assert (conv.plan.dims.grid >= 768) == (k == 96)
+    got = conv(x)
+    conv.plan.small = 0
+    assert torch.equal(got, conv(x))
+
+
+def test_packed_problems_of_two_tiles_report_the_workgroups_of_their_plans(ring, cuda):  # noqa: F811
+    lib, h = ring
+    from paella_amd import ops
+    rng = np.random.default_rng(5)
+    cases = []
+    for c, k, hw, r in [(64, 64, 56, 3), (64, 96, 41, 3), (128, 160, 28, 1), (64, 32, 50, 3), (256, 256, 14, 3), (64, 192, 33, 1), (96, 65, 40, 1)]:
+        conv = ops.Conv2d(rnd(rng, k, c, r, r), rnd(rng, k), pad=r // 2, act=ops.ACT_RELU, in_hw=(hw, hw))
+        assert conv.plan.kw == 8
+        x = torch.tensor(rnd(rng, 1, c, hw, hw), device=cuda)
+        cases.append((conv, x, conv(x)))
+    assert sum(c.plan.dims.grid for c, _, _ in cases) >= 1000
+    torch.cuda.synchronize()
+    batch = lib.paella_ring_batch_size()
+    with ops.DirectQueue() as q:
+        for flags in (NO_START, 0):  # with start messages: workgroups of one tile
+            assert lib.paella_pack_enable(1) == 0
+            try:
+                outs = []
+                for j, (conv, x, want) in enumerate(cases):
+                    y = torch.zeros_like(want)
+                    conv(x, out=y, stream=q.handle, job_id=(j + 1) | flags, notifier=ctypes.c_void_p(lib.paella_ring_notifier(h, j)))
+                    outs.append(y)
+                assert lib.paella_pack_flush() == 1
+                per = [(c.plan.dims.grid + batch - 1) // batch for c, _, _ in cases]
+                total = sum(per) * (1 if flags else 2)
+                buf = np.zeros(total, np.uint64)
+                assert lib.paella_ring_drain(h, buf.ctypes.data, total, 20.0) == total
+                m = decode(buf)
+                for j, (conv, _, _) in enumerate(cases):
+                    ends = (m["job_id"] == j + 1) & (m["is_start"] == 0)
+                    assert m["num"][ends].sum() == conv.plan.dims.grid and ends.sum() == per[j], j
+                extra = np.zeros(1, np.uint64)
+                assert lib.paella_ring_drain(h, extra.ctypes.data, 1, 0.05) == 0
+            finally:
+                lib.paella_pack_enable(0)
+            torch.cuda.synchronize()
+            for y, (_, _, want) in zip(outs, cases):
+                assert torch.equal(y, want)
