@@ -1745,6 +1745,14 @@ unsigned tall_grid(const paella_conv_plan* plan, const ConvArgs& a) {
     return (unsigned)(a.n_tiles_n * ((a.n_tiles_m + 1) / 2) * a.splits);
 }
 
+// Whether a launch by itself takes that form.  Not where the last rows are a single tile: workgroups of one length and of twice that length end
+// far apart (96->96 3x3 on 91x91, 777 workgroups of one tile: 18.2 -> 24.0 us; 96->208 on 112x112 43.6 -> 49.8).  Not where a few of them are left
+// for another turn of the device, which holds 768 (64->256 3x3 on 80x80, 800 workgroups: 22.2 -> 23.0 us; 64->320, 1000 of them, 24.6 -> 22.7).
+bool tall_alone(const ConvArgs& a, unsigned grid) {
+    const unsigned turns = grid / 768, left = grid % 768;
+    return a.n_tiles_m % 2 == 0 && (turns == 0 || turns >= 4 || left == 0 || left >= 192);
+}
+
 ConvArgs tall_args(const ConvArgs& a) {
     ConvArgs t = a;
     const unsigned gm = (unsigned)(a.n_tiles_m + 1) / 2;
@@ -2444,7 +2452,8 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         if (plan->mi == 1 && plan->ni == 1 && !plan->depth && pack_hold(&plan, &a, 1, stream)) return 0;
         SmallArgs small;
         unsigned grid = 0;
-        if (!nf && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom)) && (grid = tall_grid(plan, a)) != 0) {
+        grid = tall_grid(plan, a);
+        if (!nf && grid != 0 && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom && tall_alone(a, grid)))) {
             paella::launch(conv_tall_kernel, dim3(grid), dim3(512), plan->dims.lds_bytes, st, tall_args(a));
             return (int)hipGetLastError();
         }

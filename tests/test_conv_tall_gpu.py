@@ -50,13 +50,14 @@ def test_two_tiles_give_the_bits_of_one(cuda, case):
     assert ((out.cpu().double() - ref).abs() <= (c * r * s + 2) * 2.0 ** -24 * size).all()
 
 
-@pytest.mark.parametrize("k, h", [(64, 97), (96, 91)])  # 592 and 780 workgroups of one tile: below the rule's line and above it
+# workgroups of one tile: 590 and 784, below the rule's line and above it; 777, an odd number of tiles; 1600 and 2000, an empty and a full last turn
+@pytest.mark.parametrize("k, h", [(64, 97), (64, 112), (96, 91), (256, 80), (320, 80)])
 def test_a_launch_by_itself_takes_two_tiles_where_it_fills_the_device(cuda, k, h):
     from paella_amd import ops
     rng = np.random.default_rng(h)
     conv = ops.Conv2d(rnd(rng, k, 64, 1, 1), rnd(rng, k), act=ops.ACT_RELU, in_hw=(h, h))
     x = torch.tensor(rnd(rng, 1, 64, h, h), device=cuda)
-    assert (conv.plan.dims.grid >= 768) == (k == 96)
+    assert (conv.plan.dims.grid >= 768) == (h != 97)
     got = conv(x)
     conv.plan.small = 0
     assert torch.equal(got, conv(x))
