@@ -1485,14 +1485,15 @@ extern "C" int paella_conv2d_plan(const paella_conv_desc* d, int has_residual, i
             plan->depth = (tile_hint >> 16) & 0xF;
             if (plan->depth && !pick_kernel(mi, ni, kw, d->C % 8 == 0 ? 1 : 0, plan->depth)) return PAELLA_EINVAL;
         } else {
-            // The 32 x 32 tile unless it would make thousands of workgroups: measured on the layers of the model zoo
-            // (one launch at a time) it is the fastest or within 3 % of the fastest everywhere, and up to twice as fast
-            // as the larger tiles on layers with few channels (stems, first pointwise layers).  Waves per workgroup:
-            // the power of two that covers the chunks of the reduction, between 2 and 8 -- a wave with a single chunk
-            // still beats fewer waves with two.
-            if (tiles(1, 1) <= 2048) { mi = 1; ni = 1; }
-            else if (tiles(1, 2) <= 2048 || d->K <= 32) { mi = 1; ni = 2; }
-            else { mi = 2; ni = 2; }
+            // The 32 x 32 tile: measured on the layers of the model zoo (one launch at a time) it is the fastest or within 3 % of
+            // the fastest everywhere, and up to twice as fast as the larger tiles on layers with few channels (stems, first
+            // pointwise layers).  Also where it makes thousands of workgroups, which took the 32 x 64 or the 64 x 64 tile once
+            // (operands of four chunks in flight, 8 to 16 waves per compute unit): 64->160 3x3 on 149x149 47.2 -> 43.8 us, pointwise
+            // 160->160 there 21.0 -> 16.9, 48->100 3x3 on 149x229 50.5 -> 37.2, 3->96 on 300x300 35.2 -> 19.8, 3->32 on 512x512 25.6 -> 18.9,
+            // 64->64 on 512x512 194 -> 159, 256->256 on 160x160 260 -> 229, 128->32 on 400x400 102 -> 101, pointwise 17->160 on 149x149
+            // 12.5 -> 10.0.  Waves per workgroup: the power of two that covers the chunks of the reduction, between 2 and 8 -- a wave
+            // with a single chunk still beats fewer waves with two.
+            mi = 1; ni = 1;
             // The same holds with four passes in flight, where throughput rather than latency might have favoured operand
             // reuse (ResNet-18, thousand passes per second, four queues / one): 32 x 32 everywhere 15.8 / 7.0; 64 x 32 where
             // K is a multiple of 64: 12.1 / 4.9, only from K = 256: 13.2 / 5.6; 32 x 64 on the 56 x 56 layers: 14.4 / 6.4.

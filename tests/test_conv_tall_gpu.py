@@ -101,3 +101,16 @@ def test_packed_problems_of_two_tiles_report_the_workgroups_of_their_plans(ring,
             torch.cuda.synchronize()
             for y, (_, _, want) in zip(outs, cases):
                 assert torch.equal(y, want)
+
+
+# layers of more than 2048 tiles: two, four and eight waves, the offset table, two tiles per workgroup
+@pytest.mark.parametrize("c, k, h, w, r", [(16, 96, 149, 149, 1), (24, 128, 117, 149, 1), (3, 65, 199, 150, 3), (64, 192, 113, 111, 3), (64, 161, 113, 111, 1)])
+def test_thousands_of_tiles_give_the_bits_of_larger_ones(cuda, c, k, h, w, r):
+    from paella_amd import ops
+    rng = np.random.default_rng(k)
+    wt, b = rnd(rng, k, c, r, r), rnd(rng, k)
+    x = torch.tensor(rnd(rng, 1, c, h, w), device=cuda)
+    conv = ops.Conv2d(wt, b, pad=r // 2, act=ops.ACT_RELU, in_hw=(h, w))
+    assert (conv.plan.mi, conv.plan.ni) == (1, 1) and conv.plan.dims.grid > 2048
+    large = ops.Conv2d(wt, b, pad=r // 2, act=ops.ACT_RELU, in_hw=(h, w), tile_hint=0x120 | (conv.plan.kw.bit_length() - 1))
+    assert torch.equal(conv(x), large(x))
