@@ -685,6 +685,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid,
                 for (int e = 0; e < 16; ++e)
                     if ((mi * NI + ni) * 16 + e < RPW) mine[(mi * NI + ni) * 16 + e] = acc[mi][ni][e];
     } else if (TALL) {
+        if (!TAP_MAJOR) __syncthreads();  // every wave is done with the table before the partial tiles overwrite it
         // One tile after the other through the same 32 KB: with room for both, only two workgroups would fit a compute unit.
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
@@ -844,6 +845,9 @@ __global__ __launch_bounds__(64 * KW, (MI * NI == 1 && KW == 8 && DEPTH == 0) ? 
 // workgroup, TFLOP/s: 64->64 3x3 on 504x56 97 -> 108, 128->128 on 532x28 122 -> 135, 256->256 on 532x14 116 -> 134, 512->512 on 448x7 109 ->
 // 137, 128->256 stride 2 91 -> 124, 1x7 160->160 111 -> 127, pointwise 768->192 106 -> 112, 2048->320 117 -> 133, 64->256 40 -> 50.
 // (Eight tiles per workgroup that read all operands from LDS: 91 to 132, and workgroups too few and too long for a served launch.)
+// Where the reduction goes through the offset table (four waves; stems), the input operands cost some thirty vector instructions per chunk
+// besides, half as many per tile for two: 3->64 7x7 stride 2 on 224x224, eight problems per launch 3.74 -> 3.19 us each, one alone 8.1 -> 7.5 us.
+template <int KW, bool TAP_MAJOR>
 __device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned bid) {
     const unsigned gm = (unsigned)(p.n_tiles_m + 1) >> 1, total = (unsigned)p.n_tiles_n * gm * (unsigned)p.splits;
     if (bid >= total) return;
@@ -858,11 +862,11 @@ __device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned
     t.m = (int)(rest - (unsigned)t.split * gm);
     const PreOp none = PreOp{nullptr, nullptr, 0.f};
     if (t.m * 2 + 1 < p.n_tiles_m) {
-        if (p.pointwise) conv_tile<2, 1, 8, true, kPreNone, 0, true, true>(p, bid, none, t);
-        else conv_tile<2, 1, 8, true, kPreNone, 0, false, true>(p, bid, none, t);
+        if (TAP_MAJOR && p.pointwise) conv_tile<2, 1, KW, TAP_MAJOR, kPreNone, 0, TAP_MAJOR, true>(p, bid, none, t);
+        else conv_tile<2, 1, KW, TAP_MAJOR, kPreNone, 0, false, true>(p, bid, none, t);
     } else {
-        if (p.pointwise) conv_tile<1, 1, 8, true, kPreNone, 0, true, true>(p, bid, none, t);
-        else conv_tile<1, 1, 8, true, kPreNone, 0, false, true>(p, bid, none, t);
+        if (TAP_MAJOR && p.pointwise) conv_tile<1, 1, KW, TAP_MAJOR, kPreNone, 0, TAP_MAJOR, true>(p, bid, none, t);
+        else conv_tile<1, 1, KW, TAP_MAJOR, kPreNone, 0, false, true>(p, bid, none, t);
     }
 }
 
@@ -1006,14 +1010,16 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_group_kern
     else conv_tile<1, 1, KW, TAP_MAJOR>(g.m[idx].conv, bid);
 }
 
-__global__ __launch_bounds__(512, 6) void conv_tall_kernel(ConvArgs args) {
+template <int KW, bool TAP_MAJOR>
+__global__ __launch_bounds__(64 * KW, TAP_MAJOR ? 6 : 5) void conv_tall_kernel(ConvArgs args) {
     int idx = 0;
     asm volatile("" : "+s"(idx));
-    conv_tall_tile((&args)[idx], blockIdx.x);
+    conv_tall_tile<KW, TAP_MAJOR>((&args)[idx], blockIdx.x);
 }
 
 // The group kernel for members in the tall form, others beside them.
-__global__ __launch_bounds__(512, 6) void conv_tall_group_kernel(ConvGroupArgs g) {
+template <int KW, bool TAP_MAJOR>
+__global__ __launch_bounds__(64 * KW, TAP_MAJOR ? 6 : 5) void conv_tall_group_kernel(ConvGroupArgs g) {
     int idx = 0;
     unsigned first = g.start[0];
 #pragma unroll
@@ -1025,17 +1031,17 @@ __global__ __launch_bounds__(512, 6) void conv_tall_group_kernel(ConvGroupArgs g
     const unsigned bid = blockIdx.x - first;
     const unsigned kind = (g.kinds >> (2 * idx)) & 3u;
     if (kind == kMemberTall) {
-        conv_tall_tile(g.m[idx].conv, bid);
+        conv_tall_tile<KW, TAP_MAJOR>(g.m[idx].conv, bid);
     } else if (kind == kMemberPool) {
         const paella::PoolArgs& p = g.m[idx].pool;
         const unsigned blocks = p.hook_blocks ? p.hook_blocks : gridDim.x;
         paella::hook_entry(p.notifier, p.job_id, blocks);
-        paella::pool_element(p, (int)(bid * 512 + threadIdx.x));
+        paella::pool_element(p, (int)(bid * (64 * KW) + threadIdx.x));
         paella::hook_exit(p.notifier, p.job_id, blocks);
-    } else if (g.m[idx].conv.pointwise) {
-        conv_tile<1, 1, 8, true, kPreNone, 0, true>(g.m[idx].conv, bid);
+    } else if (TAP_MAJOR && g.m[idx].conv.pointwise) {
+        conv_tile<1, 1, KW, TAP_MAJOR, kPreNone, 0, TAP_MAJOR>(g.m[idx].conv, bid);
     } else {
-        conv_tile<1, 1, 8, true>(g.m[idx].conv, bid);
+        conv_tile<1, 1, KW, TAP_MAJOR>(g.m[idx].conv, bid);
     }
 }
 
@@ -1742,7 +1748,7 @@ constexpr unsigned kTallFrom = 768;
 
 // Workgroups of a conv in the tall form (two tiles of 32 rows each), 0 where it has none; and its arguments, from those of the plan's own kernel.
 unsigned tall_grid(const paella_conv_plan* plan, const ConvArgs& a) {
-    if (!plan->k_order || plan->kw != 8 || plan->mi != 1 || plan->ni != 1 || plan->depth || !a.fast_div || a.n_tiles_m < 2 || a.slab_major > 1) return 0;
+    if (!(plan->k_order ? plan->kw == 8 : plan->kw == 4) || plan->mi != 1 || plan->ni != 1 || plan->depth || !a.fast_div || a.n_tiles_m < 2 || a.slab_major > 1) return 0;
     return (unsigned)(a.n_tiles_n * ((a.n_tiles_m + 1) / 2) * a.splits);
 }
 
@@ -1809,7 +1815,7 @@ unsigned align_start(unsigned next) { return (next + 7u) & ~7u; }
 int launch_group_args(ConvGroupArgs& g, int n, int kw, int k_order, unsigned grid, unsigned dyn_lds, void* stream, bool tall = false) {
     for (int i = n; i < kPackMax; ++i) g.start[i] = 0xFFFFFFFFu;
     g.reserved = 0;
-    ConvGroupKernel kern = tall ? conv_tall_group_kernel : pick_group_kernel(kw, k_order);
+    ConvGroupKernel kern = tall ? (k_order ? conv_tall_group_kernel<8, true> : conv_tall_group_kernel<4, false>) : pick_group_kernel(kw, k_order);
     if (!kern) return PAELLA_EINVAL;
     if (int rc = allow_lds(reinterpret_cast<const void*>(kern), dyn_lds)) return rc;
     paella::launch_used(kern, dim3(grid), dim3(64u * (unsigned)kw), dyn_lds, reinterpret_cast<hipStream_t>(stream),
@@ -2049,7 +2055,7 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
             break;
         }
         if (n == 1) {  // nothing to share the launch with: the plain kernel, whose argument block is a quarter of the group's
-            ConvKernel kern = g.kinds ? conv_tall_kernel : pick_kernel(1, 1, kw, k_order);
+            ConvKernel kern = g.kinds ? (k_order ? conv_tall_kernel<8, true> : conv_tall_kernel<4, false>) : pick_kernel(1, 1, kw, k_order);
             rc = allow_lds(reinterpret_cast<const void*>(kern), dyn_lds);
             if (rc == 0) {
                 paella::launch(kern, dim3(grid), dim3(64u * (unsigned)kw), dyn_lds, reinterpret_cast<hipStream_t>(target), g.m[0].conv);
@@ -2455,7 +2461,7 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         unsigned grid = 0;
         grid = tall_grid(plan, a);
         if (!nf && grid != 0 && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom && tall_alone(a, grid)))) {
-            paella::launch(conv_tall_kernel, dim3(grid), dim3(512), plan->dims.lds_bytes, st, tall_args(a));
+            paella::launch(plan->k_order ? conv_tall_kernel<8, true> : conv_tall_kernel<4, false>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, st, tall_args(a));
             return (int)hipGetLastError();
         }
         const ConvArgs* one = &a;

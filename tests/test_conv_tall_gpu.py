@@ -23,6 +23,9 @@ EDGES = [
     (96, 100, 9, 9, (1, 7), 1, (0, 3), 0),
     (96, 64, 11, 11, (1, 1), 2, 0, 0),        # pointwise with a stride
     (512, 128, 7, 7, (3, 3), 1, 1, 0),        # the plan's own eight splits
+    (3, 64, 31, 33, (7, 7), 2, 3, 0),         # the offset table, four waves
+    (5, 65, 9, 11, (3, 3), 1, 1, 0x0112),     # ... 45 values: six chunks; a last row of tiles by itself
+    (3, 96, 13, 13, (5, 5), 1, 2, 0x1112),    # ... two splits
 ]
 
 
@@ -35,7 +38,7 @@ def test_two_tiles_give_the_bits_of_one(cuda, case):
     act = ops.ACT_PRELU if k % 2 else ops.ACT_RELU
     slope = rnd(rng, k) if act == ops.ACT_PRELU else None
     conv = ops.Conv2d(wt, b, stride=stride, pad=pad, act=act, slope=slope, in_hw=(h, w), has_residual=True, tile_hint=hint)
-    assert conv.plan.kw == 8
+    assert conv.plan.kw == (4 if c % 8 else 8)
     res = rnd(rng, 1, k, conv.plan.P, conv.plan.Q)
     xd, rd = torch.tensor(x, device=cuda), torch.tensor(res, device=cuda)
     conv.plan.small = 0
@@ -63,17 +66,23 @@ def test_a_launch_by_itself_takes_two_tiles_where_it_fills_the_device(cuda, k, h
     assert torch.equal(got, conv(x))
 
 
-def test_packed_problems_of_two_tiles_report_the_workgroups_of_their_plans(ring, cuda):  # noqa: F811
+# C, K, H = W, R, stride: layers that are held together
+WIDE = [(64, 64, 56, 3, 1), (64, 96, 41, 3, 1), (128, 160, 28, 1, 1), (64, 32, 50, 3, 1), (256, 256, 14, 3, 1), (64, 192, 33, 1, 1), (96, 65, 40, 1, 1)]
+TABLE = [(3, 64, 112, 7, 2), (3, 96, 97, 3, 2), (3, 32, 99, 3, 2), (3, 65, 112, 3, 2), (3, 64, 61, 7, 1)]
+
+
+@pytest.mark.parametrize("layers", [WIDE, TABLE])
+def test_packed_problems_of_two_tiles_report_the_workgroups_of_their_plans(ring, cuda, layers):  # noqa: F811
     lib, h = ring
     from paella_amd import ops
     rng = np.random.default_rng(5)
     cases = []
-    for c, k, hw, r in [(64, 64, 56, 3), (64, 96, 41, 3), (128, 160, 28, 1), (64, 32, 50, 3), (256, 256, 14, 3), (64, 192, 33, 1), (96, 65, 40, 1)]:
-        conv = ops.Conv2d(rnd(rng, k, c, r, r), rnd(rng, k), pad=r // 2, act=ops.ACT_RELU, in_hw=(hw, hw))
-        assert conv.plan.kw == 8
+    for c, k, hw, r, stride in layers:
+        conv = ops.Conv2d(rnd(rng, k, c, r, r), rnd(rng, k), stride=stride, pad=r // 2, act=ops.ACT_RELU, in_hw=(hw, hw))
+        assert conv.plan.kw == (8 if layers is WIDE else 4)
         x = torch.tensor(rnd(rng, 1, c, hw, hw), device=cuda)
         cases.append((conv, x, conv(x)))
-    assert sum(c.plan.dims.grid for c, _, _ in cases) >= 1000
+    assert sum(c.plan.dims.grid for c, _, _ in cases if c.plan.d.K > 32) >= 768
     torch.cuda.synchronize()
     batch = lib.paella_ring_batch_size()
     with ops.DirectQueue() as q:
