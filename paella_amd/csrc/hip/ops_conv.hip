@@ -144,7 +144,7 @@ struct Tile {
 };
 template <int MI, int NI, int KW, bool TAP_MAJOR, int PRE = kPreNone, int DEPTH = 0, bool PW = false, bool TALL = false>
 __device__ __forceinline__ void conv_tile(const ConvArgs& p, const unsigned bid, const PreOp pre = PreOp{nullptr, nullptr, 0.f}, const Tile given = Tile{0, 0, 0}) {
-    static_assert(!PRE || (TAP_MAJOR && MI * NI == 1), "the input transform is built for the smallest tile in tap-major order");
+    static_assert(!PRE || (TAP_MAJOR && (MI * NI == 1 || TALL)), "the input transform is built for the smallest tile in tap-major order");
     static_assert(!TALL || NI == 1, "a tall workgroup's tiles lie one under the other");
     static_assert(!PW || TAP_MAJOR, "the pointwise shortcut belongs to the tap-major order");
     // A grouped launch starts every conv at a multiple of eight workgroups (see align_start): the ids between the end of one
@@ -847,8 +847,8 @@ __global__ __launch_bounds__(64 * KW, (MI * NI == 1 && KW == 8 && DEPTH == 0) ? 
 // (Eight tiles per workgroup that read all operands from LDS: 91 to 132, and workgroups too few and too long for a served launch.)
 // Where the reduction goes through the offset table (four waves; stems), the input operands cost some thirty vector instructions per chunk
 // besides, half as many per tile for two: 3->64 7x7 stride 2 on 224x224, eight problems per launch 3.74 -> 3.19 us each, one alone 8.1 -> 7.5 us.
-template <int KW, bool TAP_MAJOR>
-__device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned bid) {
+template <int KW, bool TAP_MAJOR, int PRE = kPreNone>
+__device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned bid, const PreOp pre = PreOp{nullptr, nullptr, 0.f}) {
     const unsigned gm = (unsigned)(p.n_tiles_m + 1) >> 1, total = (unsigned)p.n_tiles_n * gm * (unsigned)p.splits;
     if (bid >= total) return;
     const unsigned xcd = bid & 7u, q = total >> 3, r = total & 7u;
@@ -860,13 +860,12 @@ __device__ __forceinline__ void conv_tall_tile(const ConvArgs& p, const unsigned
     t.n = (int)(slabs ? b : a);
     t.split = (int)quot_fast(rest, p.div_tm);
     t.m = (int)(rest - (unsigned)t.split * gm);
-    const PreOp none = PreOp{nullptr, nullptr, 0.f};
     if (t.m * 2 + 1 < p.n_tiles_m) {
-        if (TAP_MAJOR && p.pointwise) conv_tile<2, 1, KW, TAP_MAJOR, kPreNone, 0, TAP_MAJOR, true>(p, bid, none, t);
-        else conv_tile<2, 1, KW, TAP_MAJOR, kPreNone, 0, false, true>(p, bid, none, t);
+        if (TAP_MAJOR && p.pointwise) conv_tile<2, 1, KW, TAP_MAJOR, PRE, 0, TAP_MAJOR, true>(p, bid, pre, t);
+        else conv_tile<2, 1, KW, TAP_MAJOR, PRE, 0, false, true>(p, bid, pre, t);
     } else {
-        if (TAP_MAJOR && p.pointwise) conv_tile<1, 1, KW, TAP_MAJOR, kPreNone, 0, TAP_MAJOR, true>(p, bid, none, t);
-        else conv_tile<1, 1, KW, TAP_MAJOR, kPreNone, 0, false, true>(p, bid, none, t);
+        if (TAP_MAJOR && p.pointwise) conv_tile<1, 1, KW, TAP_MAJOR, PRE, 0, TAP_MAJOR, true>(p, bid, pre, t);
+        else conv_tile<1, 1, KW, TAP_MAJOR, PRE, 0, false, true>(p, bid, pre, t);
     }
 }
 
@@ -932,6 +931,7 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_pre_kernel
 // The same for up to kPackMax such convs of different requests in one launch (launch packing).
 struct ConvPreGroupArgs {
     unsigned start[PAELLA_CONV_PACK_MAX];  // first workgroup id of each problem; 0xFFFFFFFF for unused entries
+    unsigned tall, reserved;               // one bit per problem: workgroups of two tiles
     ConvPreArgs m[PAELLA_CONV_PACK_MAX];   // only the used entries are written to the argument ring
 };
 
@@ -948,6 +948,26 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_pre_group_
             first = g.start[i];
         }
     conv_pre_tile<KW>(g.m[idx], blockIdx.x - first);
+}
+
+// ... some of them in workgroups of two tiles (conv_tall_tile), which also share the transform of an operand.  Scales and shifts in flight make
+// it 86 registers, two workgroups per compute unit.  Eight problems per launch, one tile -> two, us each: 256->256 3x3 on 14x14 3.24 -> 2.98,
+// 512->512 on 7x7 3.83 -> 3.45, 64->64 on 56x56 2.53 -> 2.38, pointwise 256->128 there 2.70 -> 2.47, 192->128 2.01 -> 2.11, 1024->512 on 14x14 2.56 ->
+// 2.17.  Served, 330 requests of ArcFace-R100 132.6 -> 128.2 ms, 1000 of DenseNet-121 153.5 -> 152.4.
+__global__ __launch_bounds__(512, 4) void conv_pre_tall_group_kernel(ConvPreGroupArgs g) {
+    int idx = 0;
+    unsigned first = g.start[0];
+#pragma unroll
+    for (int i = 1; i < PAELLA_CONV_PACK_MAX; ++i)
+        if (blockIdx.x >= g.start[i]) {
+            idx = i;
+            first = g.start[i];
+        }
+    const ConvPreArgs& a = g.m[idx];
+    const unsigned bid = blockIdx.x - first;
+    if (!((g.tall >> idx) & 1u)) conv_pre_tile<8>(a, bid);
+    else if (a.pre.lo > -__builtin_inff()) conv_tall_tile<8, true, kPreBounded>(a.conv, bid, a.pre);
+    else conv_tall_tile<8, true, kPreUnbounded>(a.conv, bid, a.pre);
 }
 
 // Up to four independent convs in one launch: layers whose own grids would leave most of the 256 CUs idle (the 1x1
@@ -1883,6 +1903,7 @@ struct PackState {
     struct PreItem {
         ConvPreArgs a;
         unsigned grid = 0, dyn_lds = 0;
+        unsigned tall_grid = 0;  // as in PackItem
     };
     std::vector<PreItem> pre_lists[4];  // convs with a fused input transform, by log2(waves per workgroup)
     const void* rec_key = nullptr;  // the sequence being recorded (paella::g_pack_recording says whether one is)
@@ -2632,6 +2653,7 @@ bool pack_hold_pre(const paella_conv_plan* plan, const ConvPreArgs& a, void* str
     it.grid = plan->dims.grid;
     it.dyn_lds = pre_lds_bytes(plan);
     it.a.conv.hook_blocks = it.grid;
+    it.tall_grid = (a.conv.job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START ? tall_grid(plan, a.conv) : 0;
     g_pack.pre_lists[kw_index(plan->kw)].push_back(it);
     if (g_pack.held++ == 0) g_pack.first_held_ns = now_ns();
     return true;
@@ -2647,11 +2669,14 @@ int pre_send_all(bool only_full) {
             const size_t left = list.size() - done;
             if (only_full && left < (size_t)kPackMax) break;
             const int n = (int)std::min<size_t>(left, (size_t)kPackMax);
+            unsigned tall_total = 0;
+            for (int i = 0; i < n; ++i) tall_total += list[done + (size_t)i].tall_grid ? list[done + (size_t)i].grid : 0;
+            const bool tall = kw == 8 && tall_total >= kTallFrom;
             void* target = nullptr;
             unsigned grid = 0, dyn_lds = 0;
             int rc = paella_direct_queue_shared(&target) != 0 ? -1 : 0;
             if (rc != 0) {
-            } else if (n == 1) {
+            } else if (n == 1 && !tall) {
                 ConvPreKernel kern = pick_pre_kernel(kw);
                 ConvPreArgs a = list[done].a;
                 a.conv.hook_blocks = list[done].grid;
@@ -2662,15 +2687,23 @@ int pre_send_all(bool only_full) {
                 }
             } else {
                 ConvPreGroupArgs g;
+                g.tall = g.reserved = 0;
                 for (int i = 0; i < n; ++i) {
+                    const PackState::PreItem& it = list[done + (size_t)i];
                     grid = align_start(grid);
-                    g.m[i] = list[done + (size_t)i].a;
+                    g.m[i] = it.a;
                     g.start[i] = grid;
-                    grid += list[done + (size_t)i].grid;
-                    dyn_lds = std::max(dyn_lds, list[done + (size_t)i].dyn_lds);
+                    if (tall && it.tall_grid) {
+                        g.m[i].conv = tall_args(it.a.conv);
+                        g.tall |= 1u << i;
+                        grid += it.tall_grid;
+                    } else {
+                        grid += it.grid;
+                    }
+                    dyn_lds = std::max(dyn_lds, it.dyn_lds);
                 }
                 for (int i = n; i < kPackMax; ++i) g.start[i] = 0xFFFFFFFFu;
-                ConvPreGroupKernel kern = pick_pre_group_kernel(kw);
+                ConvPreGroupKernel kern = tall ? conv_pre_tall_group_kernel : pick_pre_group_kernel(kw);
                 rc = allow_lds(reinterpret_cast<const void*>(kern), dyn_lds);
                 if (rc == 0) {
                     paella::launch_used(kern, dim3(grid), dim3(64u * (unsigned)kw), dyn_lds, reinterpret_cast<hipStream_t>(target),

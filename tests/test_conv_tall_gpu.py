@@ -123,3 +123,42 @@ def test_thousands_of_tiles_give_the_bits_of_larger_ones(cuda, c, k, h, w, r):
     assert (conv.plan.mi, conv.plan.ni) == (1, 1) and conv.plan.dims.grid > 2048
     large = ops.Conv2d(wt, b, pad=r // 2, act=ops.ACT_RELU, in_hw=(h, w), tile_hint=0x120 | (conv.plan.kw.bit_length() - 1))
     assert torch.equal(conv(x), large(x))
+
+
+def test_packed_problems_with_an_input_transform(ring, cuda):  # noqa: F811
+    lib, h = ring
+    from paella_amd import ops
+    rng = np.random.default_rng(9)
+    cases = []
+    for c, k, hw, r, act in [(64, 64, 56, 3, ops.ACT_NONE), (128, 160, 28, 1, ops.ACT_RELU), (256, 256, 14, 3, ops.ACT_RELU), (64, 32, 50, 3, ops.ACT_NONE),
+                             (64, 65, 41, 1, ops.ACT_RELU), (128, 128, 28, 3, ops.ACT_RELU)]:
+        conv = ops.Conv2d(rnd(rng, k, c, r, r), rnd(rng, k), pad=r // 2, act=ops.ACT_RELU, in_hw=(hw, hw))
+        assert conv.plan.kw == 8
+        x = torch.tensor(rnd(rng, 1, c, hw, hw), device=cuda)
+        t = dict(in_scale=torch.tensor(rnd(rng, c), device=cuda), in_shift=torch.tensor(rnd(rng, c), device=cuda), in_act=act)
+        cases.append((conv, x, t, conv(x, **t)))
+    assert sum(c.plan.dims.grid for c, _, _, _ in cases if c.plan.d.K > 32) >= 768
+    torch.cuda.synchronize()
+    batch = lib.paella_ring_batch_size()
+    with ops.DirectQueue() as q:
+        assert lib.paella_pack_enable(1) == 0
+        try:
+            outs = []
+            for j, (conv, x, t, want) in enumerate(cases):
+                y = torch.zeros_like(want)
+                conv(x, out=y, stream=q.handle, job_id=(j + 1) | NO_START, notifier=ctypes.c_void_p(lib.paella_ring_notifier(h, j)), **t)
+                outs.append(y)
+            assert lib.paella_pack_flush() == 1
+            per = [(c.plan.dims.grid + batch - 1) // batch for c, _, _, _ in cases]
+            buf = np.zeros(sum(per), np.uint64)
+            assert lib.paella_ring_drain(h, buf.ctypes.data, sum(per), 20.0) == sum(per)
+            m = decode(buf)
+            for j, (conv, _, _, _) in enumerate(cases):
+                assert m["num"][m["job_id"] == j + 1].sum() == conv.plan.dims.grid, j
+            extra = np.zeros(1, np.uint64)
+            assert lib.paella_ring_drain(h, extra.ctypes.data, 1, 0.05) == 0
+        finally:
+            lib.paella_pack_enable(0)
+        torch.cuda.synchronize()
+        for y, (_, _, _, want) in zip(outs, cases):
+            assert torch.equal(y, want)
