@@ -2463,6 +2463,17 @@ extern "C" int paella_conv2d_launch_pair(const paella_conv_operands* first, cons
     return paella_conv2d_launch_group(members, 2, stream, job_id, notifier);
 }
 
+// One conv by itself in the tall form; false where that does not apply.  (Out of line: most calls go past it, and its copy of the arguments
+// would be part of their stack frame.)
+__attribute__((noinline)) static bool launch_tall(const paella_conv_plan* plan, const ConvArgs& a, hipStream_t stream) {
+    const unsigned grid = tall_grid(plan, a);
+    if (grid == 0 || (plan->small != 4 && !tall_alone(a, grid))) return false;
+    const ConvArgs t = tall_args(a);
+    if (plan->k_order) paella::launch(conv_tall_kernel<8, true>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, stream, t);
+    else paella::launch(conv_tall_kernel<4, false>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, stream, t);
+    return true;
+}
+
 extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x, const void* blob_dev, const float* bias,
                                     const float* residual, const float* slope, float* y, void* workspace, void* stream,
                                     uint32_t job_id, void* notifier) {
@@ -2480,11 +2491,7 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         if (plan->mi == 1 && plan->ni == 1 && !plan->depth && pack_hold(&plan, &a, 1, stream)) return 0;
         SmallArgs small;
         unsigned grid = 0;
-        grid = tall_grid(plan, a);
-        if (!nf && grid != 0 && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom && tall_alone(a, grid)))) {
-            paella::launch(plan->k_order ? conv_tall_kernel<8, true> : conv_tall_kernel<4, false>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, st, tall_args(a));
-            return (int)hipGetLastError();
-        }
+        if (!nf && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom)) && launch_tall(plan, a, st)) return (int)hipGetLastError();
         const ConvArgs* one = &a;
         const int mi = small_form(&plan, &one, 1);
         if (mi && fill_small(plan, a, mi, small, &grid)) {
