@@ -2463,14 +2463,17 @@ extern "C" int paella_conv2d_launch_pair(const paella_conv_operands* first, cons
     return paella_conv2d_launch_group(members, 2, stream, job_id, notifier);
 }
 
-// One conv by itself in the tall form; false where that does not apply.  (Out of line: most calls go past it, and its copy of the arguments
-// would be part of their stack frame.)
-__attribute__((noinline)) static bool launch_tall(const paella_conv_plan* plan, const ConvArgs& a, hipStream_t stream) {
+// One conv by itself in the tall form; false where that does not apply, else *rc says how it went.  (Out of line: most calls go past it, and
+// its copy of the arguments would be part of their stack frame.)
+__attribute__((noinline)) static bool launch_tall(const paella_conv_plan* plan, const ConvArgs& a, hipStream_t stream, int* rc) {
     const unsigned grid = tall_grid(plan, a);
     if (grid == 0 || (plan->small != 4 && !tall_alone(a, grid))) return false;
     const ConvArgs t = tall_args(a);
-    if (plan->k_order) paella::launch(conv_tall_kernel<8, true>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, stream, t);
-    else paella::launch(conv_tall_kernel<4, false>, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, stream, t);
+    ConvKernel kern = plan->k_order ? conv_tall_kernel<8, true> : conv_tall_kernel<4, false>;
+    *rc = allow_lds(reinterpret_cast<const void*>(kern), plan->dims.lds_bytes);  // a long reduction's offset table is beyond 64 KB
+    if (*rc) return true;
+    paella::launch(kern, dim3(grid), dim3(plan->dims.block), plan->dims.lds_bytes, stream, t);
+    *rc = (int)hipGetLastError();
     return true;
 }
 
@@ -2491,7 +2494,8 @@ extern "C" int paella_conv2d_launch(const paella_conv_plan* plan, const float* x
         if (plan->mi == 1 && plan->ni == 1 && !plan->depth && pack_hold(&plan, &a, 1, stream)) return 0;
         SmallArgs small;
         unsigned grid = 0;
-        if (!nf && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom)) && launch_tall(plan, a, st)) return (int)hipGetLastError();
+        int rc = 0;
+        if (!nf && (plan->small == 4 || (plan->small == 1 && plan->dims.grid >= kTallFrom)) && launch_tall(plan, a, st, &rc)) return rc;
         const ConvArgs* one = &a;
         const int mi = small_form(&plan, &one, 1);
         if (mi && fill_small(plan, a, mi, small, &grid)) {

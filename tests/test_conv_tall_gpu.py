@@ -162,3 +162,21 @@ def test_packed_problems_with_an_input_transform(ring, cuda):  # noqa: F811
         torch.cuda.synchronize()
         for y, (_, _, _, want) in zip(outs, cases):
             assert torch.equal(y, want)
+
+
+# offset tables of 72 128 and 103 232 bytes, in launches that take workgroups of two tiles by themselves
+@pytest.mark.parametrize("c, r", [(1001, 3), (516, 5)])
+def test_an_offset_table_of_more_than_64_kb(cuda, c, r):
+    from paella_amd import ops
+    k, h, w, rows = 64, 100, 128, 3
+    rng = np.random.default_rng(c)
+    wt, b, x = rnd(rng, k, c, r, r), rnd(rng, k), rnd(rng, 1, c, h, w)
+    conv = ops.Conv2d(wt, b, pad=r // 2, act=ops.ACT_RELU, in_hw=(h, w))
+    assert conv.plan.dims.lds_bytes > 65536 and conv.plan.dims.grid == 800
+    xd = torch.tensor(x, device=cuda)
+    got = conv(xd)
+    conv.plan.small = 0
+    assert torch.equal(got, conv(xd))
+    top = x[:, :, :rows + r // 2]  # all that the first rows read; the bound is that of the first test
+    ref, size = (reference(*(f(a) for a in (top, wt, b)), 1, r // 2, None, None, act)[:, :, :rows] for f, act in ((np.asarray, 1), (np.abs, 0)))
+    assert ((got[:, :, :rows].cpu().double() - ref).abs() <= (c * r * r + 1) * 2.0 ** -24 * size).all()
