@@ -1759,11 +1759,13 @@ void add_kernel_resources(const void* fn, paella_launch_dims* dims) {
     }
 }
 
-// Workgroups of one tile from which on a launch takes those of two tiles (conv_tall_tile): three per compute unit.  Below, the device holds
-// all of them at once, and half as many that take twice as long make the launch longer.  One launch alone, one tile -> two: 196 workgroups
-// 5.8 -> 8.3 us, 392 8.3 -> 8.6, 588 11.0 -> 13.1, 676 8.2 -> 8.1, 784 14.1 -> 13.5, 784 (pointwise) 5.0 -> 4.6, 948 17.3 -> 17.4, 1352 13.3 ->
-// 12.5.  Served, several problems per launch, never / from 1280 / 1024 / 768 / 512 / 128 / 2: ResNet-18 216 / 212 / 207 / 206 / 207 / 206 / 205 ms,
-// MobileNetV2 : ResNet-50 188 / 184 / 183 / 182 / 182 / 182 / 181, small CNN : Inception-v3 163 / 162 / 162 / 162 / 165 / 171 / 170.
+// Workgroups of one tile from which on a launch takes those of two tiles (conv_tall_tile): three per compute unit.  Below, half as many that
+// take nearly twice as long leave compute units with one workgroup or none, and nothing to run while it waits.  One launch alone, one tile ->
+// two: 196 workgroups 5.8 -> 8.3 us, 392 8.3 -> 8.6, 588 11.0 -> 13.1; from there on tall_alone says which.  Served, several problems per launch,
+// never / from 1280 / 1024 / 768 / 512 / 128 / 2: ResNet-18 216 / 212 / 207 / 206 / 207 / 206 / 205 ms, MobileNetV2 : ResNet-50 188 / 184 / 183 / 182 /
+// 182 / 182 / 181, small CNN : Inception-v3 163 / 162 / 162 / 162 / 165 / 171 / 170.  The same line for the forms whose workgroups fit a compute unit
+// in other numbers (table: five, a transform of the input: two), us per problem in launches of eight, four streams: 3->64 7x7 stride 2, 784
+// workgroups 3.82 -> 3.25; with a transform 64->64 3x3 on 56x56 at 784 2.29 -> 2.22, 256->256 on 14x14 at 896 2.73 -> 2.55.
 constexpr unsigned kTallFrom = 768;
 
 // Workgroups of a conv in the tall form (two tiles of 32 rows each), 0 where it has none; and its arguments, from those of the plan's own kernel.
@@ -1772,12 +1774,22 @@ unsigned tall_grid(const paella_conv_plan* plan, const ConvArgs& a) {
     return (unsigned)(a.n_tiles_n * ((a.n_tiles_m + 1) / 2) * a.splits);
 }
 
-// Whether a launch by itself takes that form.  Not where the last rows are a single tile: workgroups of one length and of twice that length end
-// far apart (96->96 3x3 on 91x91, 777 workgroups of one tile: 18.2 -> 24.0 us; 96->208 on 112x112 43.6 -> 49.8).  Not where a few of them are left
-// for another turn of the device, which holds 768 (64->256 3x3 on 80x80, 800 workgroups: 22.2 -> 23.0 us; 64->320, 1000 of them, 24.6 -> 22.7).
-bool tall_alone(const ConvArgs& a, unsigned grid) {
-    const unsigned turns = grid / 768, left = grid % 768;
-    return a.n_tiles_m % 2 == 0 && (turns == 0 || turns >= 4 || left == 0 || left >= 192);
+// Whether a launch by itself, `one` workgroups of one tile or `two` in the tall form, takes the latter.  Workgroups go to the 256 compute units in
+// turn, and the launch lasts as long as the unit with the most of them, which in the tall form are fewer and longer: by 1.82 for a reduction that
+// is bound by the matrix instructions (1.78 pointwise), by 1.6 where most of a workgroup's time is its way there and back (one or two chunks per
+// wave) or the inputs' (a stride uses half of every line), by 1.7 through the offset table, by 1.45 where that table is so long that a unit holds
+// fewer than four workgroups and has little to run beside one that waits.  How many the device holds at once does not decide: 3 workgroups per unit
+// fit or 5, the steps are at multiples of 256 in both forms.  One tile -> two per workgroup, us, at 768 / 832 / 1152 / 1408 / 1600 / 2304 / 2816 / 3136
+// workgroups of one tile: 64->64 3x3 11.0 -> 12.7, 13.2 -> 12.7, 15.8 -> 17.3, 18.3 -> 17.2, 20.7 -> 21.8, 26.0 -> 26.6, 30.9 -> 31.2, 35.8 -> 35.5;
+// pointwise 256->64 6.8 -> 7.5, 7.8 -> 7.5, 9.2 -> 9.5, 10.6 -> 9.7, 11.9 -> 12.3, 15.7 -> 15.2, 18.2 -> 17.5, 20.0 -> 19.8; pointwise 64->64 4.8 -> 4.7,
+// 5.4 -> 4.7, 6.2 -> 5.6, 6.9 -> 5.7, 7.6 -> 7.2, 9.3 -> 8.2, 10.7 -> 9.2, 11.8 -> 10.5; 33->64 3x3 by the table 10.2 -> 10.9, 11.5 -> 10.9, 13.3 -> 13.6,
+// 15.2 -> 13.6, 16.9 -> 16.0, 20.7 -> 19.0, 24.2 -> 23.2, 27.6 -> 25.8.  With an odd number of rows the workgroups have two lengths: the rule asks for
+// more than such a launch needs (64->96 3x3 at 1602: 20.9 -> 26.3, 64->160 at 770: 13.2 -> 12.7).  Over 160 drawn layers of 768 to 9000 workgroups
+// (1 to 7 wide filters, strides 1 and 2, 3 to 1024 channels) the time is 1.003 of the faster form's; one tile throughout 1.098, two 1.022.
+bool tall_alone(const ConvArgs& a, unsigned one, unsigned two, bool table, unsigned lds_bytes) {
+    const bool short_way = (a.pointwise && a.nchunks <= 16) || a.sw > 1;
+    const unsigned percent = table ? (lds_bytes * 4 > 160 * 1024 ? 145 : 170) : short_way ? 160 : a.pointwise ? 178 : 182;
+    return (uint64_t)((two + 255) / 256) * percent < (uint64_t)((one + 255) / 256) * 100;
 }
 
 ConvArgs tall_args(const ConvArgs& a) {
@@ -2467,7 +2479,7 @@ extern "C" int paella_conv2d_launch_pair(const paella_conv_operands* first, cons
 // its copy of the arguments would be part of their stack frame.)
 __attribute__((noinline)) static bool launch_tall(const paella_conv_plan* plan, const ConvArgs& a, hipStream_t stream, int* rc) {
     const unsigned grid = tall_grid(plan, a);
-    if (grid == 0 || (plan->small != 4 && !tall_alone(a, grid))) return false;
+    if (grid == 0 || (plan->small != 4 && !tall_alone(a, plan->dims.grid, grid, plan->k_order == 0, plan->dims.lds_bytes))) return false;
     const ConvArgs t = tall_args(a);
     ConvKernel kern = plan->k_order ? conv_tall_kernel<8, true> : conv_tall_kernel<4, false>;
     *rc = allow_lds(reinterpret_cast<const void*>(kern), plan->dims.lds_bytes);  // a long reduction's offset table is beyond 64 KB

@@ -27,3 +27,37 @@ def test_more_than_64_kb_of_lds_are_asked_for(c, k, h, w, r, route, small):
     """An offset table of a long reduction, in every form that a launch takes."""
     [(_, [(_, _, lds, allowed)])] = launches((route, c, k, h, w, r, r, 1, r // 2, 0, small, 0x80000000, 1))
     assert 65536 < lds <= allowed
+
+
+ONE, TWO = 1, 2  # tiles per workgroup
+
+
+def form(launch):
+    return TWO if "tall" in launch[0] else ONE
+
+
+def alone(c, k, h, w, r=1, stride=1):
+    return "alone", c, k, h, w, r, r, stride, r // 2, 0, -1, 0, 1
+
+
+@pytest.mark.parametrize("layer, grid, want", [
+    # a matrix-bound reduction: two of twice the work against three on the fullest compute unit, against four, three against five, ...
+    (alone(64, 64, 192, 64, 3), 768, ONE), (alone(64, 64, 193, 64, 3), 772, TWO), (alone(64, 64, 256, 64, 3), 1024, TWO), (alone(64, 64, 257, 64, 3), 1028, ONE),
+    (alone(64, 64, 320, 64, 3), 1280, ONE), (alone(64, 64, 321, 64, 3), 1284, TWO), (alone(64, 64, 400, 64, 3), 1600, ONE), (alone(64, 64, 576, 64, 3), 2304, ONE),
+    (alone(64, 64, 704, 64, 3), 2816, TWO), (alone(64, 64, 784, 64, 3), 3136, TWO),
+    # pointwise
+    (alone(256, 64, 288, 64), 1152, ONE), (alone(256, 64, 400, 64), 1600, ONE), (alone(256, 64, 576, 64), 2304, TWO),
+    # ... of one or two chunks per wave, and a stride
+    (alone(64, 64, 192, 64), 768, ONE), (alone(64, 64, 288, 64), 1152, TWO), (alone(128, 64, 400, 64), 1600, TWO), (alone(136, 64, 288, 64), 1152, ONE),
+    (alone(64, 64, 576, 128, 3, 2), 1152, TWO),
+    # the offset table, short and long
+    (alone(33, 64, 192, 64, 3), 768, ONE), (alone(33, 64, 288, 64, 3), 1152, ONE), (alone(33, 64, 400, 64, 3), 1600, TWO),
+    (alone(1001, 64, 192, 64, 3), 768, TWO), (alone(516, 64, 288, 64, 5), 1152, TWO),
+    # an odd number of rows
+    (alone(96, 96, 91, 91, 3), 777, ONE), (alone(96, 208, 112, 112, 3), 2744, ONE), (alone(64, 160, 77, 64, 3), 770, TWO), (alone(64, 160, 90, 64, 3), 900, ONE),
+])
+def test_which_launches_take_two_tiles_by_themselves(layer, grid, want):
+    [(got, [launch])] = launches(layer)
+    assert got == grid and form(launch) == want
+    rows = (layer[2] + 31) // 32
+    assert launch[1] == (grid if want == ONE else grid // rows * ((rows + 1) // 2))
