@@ -1792,6 +1792,15 @@ bool tall_alone(const ConvArgs& a, unsigned one, unsigned two, bool table, unsig
     return (uint64_t)((two + 255) / 256) * percent < (uint64_t)((one + 255) / 256) * 100;
 }
 
+// The same for a launch that packing held and that carries this one conv.  Other queues' launches run beside it as a rule, and then the work counts and
+// not the fullest compute unit, so that it takes two tiles also where it would not alone (64->256 3x3 on 80x80, one behind the other on four
+// queues 16.4 -> 15.0 us each, with nothing beside it 0.7 us more) -- but for an odd number of rows, whose workgroups of two lengths end far apart
+// either way: 96->96 3x3 on 91x91 11.6 -> 12.3 us on four queues and 5.3 more alone, 96->208 on 112x112 40.9 -> 41.9 and 4.4 more.  Through the offset
+// table those too are faster (3->160 7x7 stride 2 on 224x224 8.6 -> 7.7 us).
+bool tall_held_alone(const ConvArgs& a, unsigned one, unsigned two, bool table) {
+    return table || a.n_tiles_m % 2 == 0 || tall_alone(a, one, two, false, 0);
+}
+
 ConvArgs tall_args(const ConvArgs& a) {
     ConvArgs t = a;
     const unsigned gm = (unsigned)(a.n_tiles_m + 1) / 2;
@@ -2053,7 +2062,8 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
             total += list.items[i].members();
             for (int c = 0; c < list.items[i].n; ++c) tall_total += list.items[i].tall_grids[c] ? list.items[i].grids[c] : 0;
         }
-        const bool tall = tall_total >= kTallFrom;
+        const PackItem& head = list.items[done];
+        const bool tall = tall_total >= kTallFrom && (total > 1 || tall_held_alone(head.args[0], head.grids[0], head.tall_grids[0], k_order == 0));
         g.kinds = 0;
         for (size_t k = done; k < i; ++k) {  // the convs of every item first ...
             const PackItem& it = list.items[k];
@@ -2694,7 +2704,8 @@ int pre_send_all(bool only_full) {
             const int n = (int)std::min<size_t>(left, (size_t)kPackMax);
             unsigned tall_total = 0;
             for (int i = 0; i < n; ++i) tall_total += list[done + (size_t)i].tall_grid ? list[done + (size_t)i].grid : 0;
-            const bool tall = kw == 8 && tall_total >= kTallFrom;
+            const PackState::PreItem& head = list[done];
+            const bool tall = kw == 8 && tall_total >= kTallFrom && (n > 1 || tall_held_alone(head.a.conv, head.grid, head.tall_grid, false));
             void* target = nullptr;
             unsigned grid = 0, dyn_lds = 0;
             int rc = paella_direct_queue_shared(&target) != 0 ? -1 : 0;

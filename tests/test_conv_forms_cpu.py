@@ -61,3 +61,25 @@ def test_which_launches_take_two_tiles_by_themselves(layer, grid, want):
     assert got == grid and form(launch) == want
     rows = (layer[2] + 31) // 32
     assert launch[1] == (grid if want == ONE else grid // rows * ((rows + 1) // 2))
+
+
+def held(times, c, k, h, r=1, stride=1, route="packed"):
+    return route, c, k, h, h, r, r, stride, r // 2, 0, -1, 0x80000000, times
+
+
+@pytest.mark.parametrize("layer, grid, want", [
+    # an odd number of rows that loses with two tiles, one that gains; even ones, also where the rule for a launch without company says one
+    (held(1, 96, 96, 91, 3), 777, ONE), (held(1, 96, 208, 112, 3), 2744, ONE), (held(1, 64, 288, 56, 3), 882, TWO),
+    (held(1, 64, 64, 112, 3), 784, TWO), (held(1, 64, 256, 80, 3), 1600, TWO), (held(1, 3, 160, 224, 7, 2), 1960, TWO),
+    (held(1, 64, 64, 110, 3), 758, ONE),
+    # the same with an input transform
+    (held(1, 96, 96, 91, 3, route="transformed"), 777, ONE), (held(1, 96, 208, 112, 3, route="transformed"), 2744, ONE),
+    (held(1, 64, 64, 112, 3, route="transformed"), 784, TWO),
+])
+def test_which_held_launches_of_one_conv_take_two_tiles(layer, grid, want):
+    [(got, [launch])] = launches(layer)
+    assert got == grid and form(launch) == want
+
+
+def test_a_held_launch_whose_workgroups_report_their_start_takes_one_tile():
+    assert [form(x) for _, [x] in launches(("packed",) + held(1, 64, 64, 112, 3)[1:11] + (0, 1))] == [ONE]
