@@ -952,8 +952,8 @@ __global__ __launch_bounds__(64 * KW, KW == 8 ? 8 : 1) void conv_mfma_pre_group_
 
 // ... some of them in workgroups of two tiles (conv_tall_tile), which also share the transform of an operand.  Scales and shifts in flight make
 // it 86 registers, two workgroups per compute unit.  Eight problems per launch, one tile -> two, us each: 256->256 3x3 on 14x14 3.24 -> 2.98,
-// 512->512 on 7x7 3.83 -> 3.45, 64->64 on 56x56 2.53 -> 2.38, pointwise 256->128 there 2.70 -> 2.47, 192->128 2.01 -> 2.11, 1024->512 on 14x14 2.56 ->
-// 2.17.  Served, 330 requests of ArcFace-R100 132.6 -> 128.2 ms, 1000 of DenseNet-121 153.5 -> 152.4.
+// 512->512 on 7x7 3.83 -> 3.45, 64->64 on 56x56 2.53 -> 2.38, pointwise 256->128 there 2.70 -> 2.47, 1024->512 on 14x14 2.56 -> 2.17 (and at
+// tall_packed those that do not gain).  Served, 330 requests of ArcFace-R100 132.6 -> 128.2 ms, 1000 of DenseNet-121 153.5 -> 152.4.
 __global__ __launch_bounds__(512, 4) void conv_pre_tall_group_kernel(ConvPreGroupArgs g) {
     int idx = 0;
     unsigned first = g.start[0];
@@ -1792,6 +1792,17 @@ bool tall_alone(const ConvArgs& a, unsigned one, unsigned two, bool table, unsig
     return (uint64_t)((two + 255) / 256) * percent < (uint64_t)((one + 255) / 256) * 100;
 }
 
+// Whether the tall form is taken where several problems share a launch.  Not for three rows of tiles of a filter with several taps: half of the
+// workgroups are of two tiles and half of one, and where they take turns on the compute units the former meet on half of those (launches of eight, four
+// queues, us per problem, one tile -> two: 96->96 3x3 on 35x35 1.75 -> 2.12, 64->96 there 1.28 -> 1.48, on 71x71 5.20 -> 5.83, on 91x91 12.04 -> 12.07,
+// 3->96 3x3 on 149x149 5.68 -> 6.01; five and more rows are level to 11 % faster on average: 64->160 on 56x56 5.17 -> 4.82, 96->160 on 28x28 1.89 -> 2.11,
+// 128->224 on 17x17 1.63 -> 1.46, 3->160 7x7 8.53 -> 7.48; three rows of one tap 64->96 on 56x56 1.07 -> 0.94, 256->96 1.67 -> 1.65).
+// Pointwise convs with an input transform and two or three chunks per wave do not gain by themselves either (two of their workgroups fit a compute
+// unit where four of one tile do; 128 outputs on 56x56 from 64 / 96 / 128 / 160 / 192 / 224 / 256 channels 1.52 -> 1.49, 1.69 -> 1.76, 1.77 -> 1.79, 1.89 ->
+// 2.00, 1.92 -> 2.04, 2.30 -> 2.27, 2.36 -> 2.30), but half as many workgroups leave more of the device to the launches of other queues: served
+// with 48 in flight, 1000 requests of DenseNet-121, which has these layers, take 155.3 ms with them in this form and 156.7 without (six runs each).
+bool tall_packed(const ConvArgs& a) { return a.n_tiles_m != 3 || a.RS == 1; }
+
 // The same for a launch that packing held and that carries this one conv.  Other queues' launches run beside it as a rule, and then the work counts and
 // not the fullest compute unit, so that it takes two tiles also where it would not alone (64->256 3x3 on 80x80, one behind the other on four
 // queues 16.4 -> 15.0 us each, with nothing beside it 0.7 us more) -- but for an odd number of rows, whose workgroups of two lengths end far apart
@@ -2027,7 +2038,7 @@ bool pack_hold(const paella_conv_plan* const* plans, const ConvArgs* args, int n
         it.args[i] = args[i];
         it.grids[i] = plans[i]->dims.grid;
         // (its workgroups send no start messages and no time samples)
-        it.tall_grids[i] = (args[i].job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START ? tall_grid(plans[i], args[i]) : 0;
+        it.tall_grids[i] = (args[i].job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START && tall_packed(args[i]) ? tall_grid(plans[i], args[i]) : 0;
         it.grid += plans[i]->dims.grid;
         it.dyn_lds = std::max(it.dyn_lds, plans[i]->dims.lds_bytes);
     }
@@ -2686,7 +2697,7 @@ bool pack_hold_pre(const paella_conv_plan* plan, const ConvPreArgs& a, void* str
     it.grid = plan->dims.grid;
     it.dyn_lds = pre_lds_bytes(plan);
     it.a.conv.hook_blocks = it.grid;
-    it.tall_grid = (a.conv.job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START ? tall_grid(plan, a.conv) : 0;
+    it.tall_grid = (a.conv.job_id & PAELLA_JOB_ID_FLAGS) == PAELLA_JOB_ID_NO_START && tall_packed(a.conv) ? tall_grid(plan, a.conv) : 0;
     g_pack.pre_lists[kw_index(plan->kw)].push_back(it);
     if (g_pack.held++ == 0) g_pack.first_held_ns = now_ns();
     return true;

@@ -83,3 +83,21 @@ def test_which_held_launches_of_one_conv_take_two_tiles(layer, grid, want):
 
 def test_a_held_launch_whose_workgroups_report_their_start_takes_one_tile():
     assert [form(x) for _, [x] in launches(("packed",) + held(1, 64, 64, 112, 3)[1:11] + (0, 1))] == [ONE]
+
+
+def in_all(n, grid):
+    return grid * n + (-grid % 8) * (n - 1)  # a problem's first workgroup is a multiple of eight
+
+
+@pytest.mark.parametrize("layer, want", [
+    # three rows of tiles with several taps, with one; five
+    (held(8, 96, 96, 35, 3), ONE), (held(8, 64, 96, 71, 3), ONE), (held(1, 3, 96, 149, 3), ONE), (held(8, 64, 96, 56), TWO), (held(8, 64, 160, 56, 3), TWO),
+    (held(8, 64, 96, 56, 3, route="transformed"), ONE), (held(8, 64, 160, 56, 3, route="transformed"), TWO),
+    (held(8, 192, 128, 56, route="transformed"), TWO), (held(8, 64, 64, 56, 3, route="transformed"), TWO),
+    # in all fewer workgroups than 768, and just as many
+    (held(7, 64, 64, 42, 3), TWO), (held(6, 64, 64, 42, 3), ONE),
+])
+def test_which_convs_take_two_tiles_in_a_launch_of_several(layer, want):
+    [(grid, [launch])] = launches(layer)
+    rows, n = (layer[2] + 31) // 32, layer[-1]
+    assert launch[1] == in_all(n, grid if want == ONE else grid // rows * ((rows + 1) // 2))
