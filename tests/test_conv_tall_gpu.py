@@ -53,7 +53,8 @@ def test_two_tiles_give_the_bits_of_one(cuda, case):
     assert ((out.cpu().double() - ref).abs() <= (c * r * s + 2) * 2.0 ** -24 * size).all()
 
 
-# workgroups of one tile: 590 and 784, below the rule's line and above it; 777, an odd number of tiles; 1600 and 2000, an empty and a full last turn
+# workgroups of one tile: 590 and 784, below the rule's line and above it; 777, three rows of tiles; 1600 and 2000, four workgroups of two tiles on the
+# fullest compute unit against seven and eight of one
 @pytest.mark.parametrize("k, h", [(64, 97), (64, 112), (96, 91), (256, 80), (320, 80)])
 def test_a_launch_by_itself_takes_two_tiles_where_it_fills_the_device(cuda, k, h):
     from paella_amd import ops
@@ -68,10 +69,11 @@ def test_a_launch_by_itself_takes_two_tiles_where_it_fills_the_device(cuda, k, h
 
 # C, K, H = W, R, stride: layers that are held together
 WIDE = [(64, 64, 56, 3, 1), (64, 96, 41, 3, 1), (128, 160, 28, 1, 1), (64, 32, 50, 3, 1), (256, 256, 14, 3, 1), (64, 192, 33, 1, 1), (96, 65, 40, 1, 1)]
-TABLE = [(3, 64, 112, 7, 2), (3, 96, 97, 3, 2), (3, 32, 99, 3, 2), (3, 65, 112, 3, 2), (3, 64, 61, 7, 1)]
+TABLE = [(3, 64, 112, 7, 2), (3, 96, 97, 3, 2), (3, 32, 99, 3, 2), (3, 65, 112, 3, 2), (3, 64, 61, 7, 1)]  # three rows of tiles: one per workgroup
+FIVE_ROWS = [(3, 64, 112, 7, 2), (3, 160, 97, 3, 2), (3, 32, 99, 3, 2), (3, 65, 112, 3, 2), (3, 64, 61, 7, 1)]
 
 
-@pytest.mark.parametrize("layers", [WIDE, TABLE])
+@pytest.mark.parametrize("layers", [WIDE, TABLE, FIVE_ROWS])
 def test_packed_problems_of_two_tiles_report_the_workgroups_of_their_plans(ring, cuda, layers):  # noqa: F811
     lib, h = ring
     from paella_amd import ops
@@ -180,3 +182,56 @@ def test_an_offset_table_of_more_than_64_kb(cuda, c, r):
     top = x[:, :, :rows + r // 2]  # all that the first rows read; the bound is that of the first test
     ref, size = (reference(*(f(a) for a in (top, wt, b)), 1, r // 2, None, None, act)[:, :, :rows] for f, act in ((np.asarray, 1), (np.abs, 0)))
     assert ((got[:, :, :rows].cpu().double() - ref).abs() <= (c * r * r + 1) * 2.0 ** -24 * size).all()
+
+
+# one notifier counts a job's workgroups of two tiles (which add two), of one tile and of the pooling operator, in messages of 1, 2, 64 and 128
+@pytest.mark.parametrize("batch", [1, 2, 64, 128])
+def test_one_notifier_for_workgroups_of_two_tiles_of_one_and_of_pooling(cuda, batch):
+    from paella_amd import _abi, ops
+    lib, h = _abi.ops(), ctypes.c_void_p()
+    assert lib.paella_ring_create_batched(8192, 4, batch, ctypes.byref(h)) == 0
+    rng = np.random.default_rng(batch)
+
+    def conv_of(c, k, hw, r):
+        conv = ops.Conv2d(rnd(rng, k, c, r, r), rnd(rng, k), pad=r // 2, act=ops.ACT_RELU, in_hw=(hw, hw))
+        assert conv.plan.kw == 8
+        return conv, torch.tensor(rnd(rng, 1, c, hw, hw), device=cuda)
+
+    jobs = [  # convs, and the map that is pooled
+        ([conv_of(64, 64, 40, 3), conv_of(256, 256, 14, 3), conv_of(64, 96, 40, 3)], None),  # a split reduction; three rows of tiles: one per workgroup
+        ([conv_of(64, 160, 40, 1), conv_of(64, 32, 40, 3)], torch.tensor(rnd(rng, 1, 64, 40, 40), device=cuda)),
+        ([conv_of(64, 128, 56, 3)], torch.tensor(rnd(rng, 1, 64, 39, 40), device=cuda)),
+    ]
+    want = [[conv(x) for conv, x in convs] + ([ops.pool2d(p, 3, 1, pad=1)] if p is not None else []) for convs, p in jobs]
+    grids = [sum(c.plan.dims.grid for c, _ in convs) + (0 if p is None else (p.numel() + 511) // 512) for convs, p in jobs]
+    assert sum(c.plan.dims.grid for convs, _ in jobs for c, _ in convs if c.plan.d.K not in (32, 96)) >= 768
+    torch.cuda.synchronize()
+    try:
+        with ops.DirectQueue() as q:
+            for flags in (NO_START, NO_START, 0):  # the second finds the counters as the first left them; with start messages: workgroups of one tile
+                assert lib.paella_pack_enable(1) == 0
+                got = []
+                for j, (convs, p) in enumerate(jobs):
+                    args = dict(stream=q.handle, job_id=(j + 1) | flags, notifier=ctypes.c_void_p(lib.paella_ring_notifier(h, j)))
+                    cs, xs = [c for c, _ in convs], [x for _, x in convs]
+                    if p is None:
+                        got.append(ops.conv2d_group(cs, xs, **args))
+                    else:
+                        ys, py = ops.conv2d_group_pool(cs, xs, p, 3, 1, pad=1, **args)
+                        got.append(list(ys) + [py])
+                assert lib.paella_pack_flush() == 1
+                ends = [(g + batch - 1) // batch for g in grids]
+                total = sum(ends) * (1 if flags else 2)
+                buf = np.zeros(total + 1, np.uint64)
+                assert lib.paella_ring_drain(h, buf.ctypes.data, total, 20.0) == total
+                assert lib.paella_ring_drain(h, buf.ctypes.data + 8 * total, 1, 0.05) == 0
+                m = decode(buf[:total])
+                for j, g in enumerate(grids):
+                    mine = (m["job_id"] == j + 1) & (m["is_start"] == 0)
+                    assert m["num"][mine].sum() == g and mine.sum() == ends[j], (j, flags)
+                torch.cuda.synchronize()
+                for ys, zs in zip(got, want):
+                    assert len(ys) == len(zs) and all(torch.equal(a, b) for a, b in zip(ys, zs))
+    finally:
+        lib.paella_pack_enable(0)
+        lib.paella_ring_destroy(h)
