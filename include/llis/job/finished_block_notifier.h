@@ -122,10 +122,9 @@ class FinishedBlockNotifier {
         announce<false>(&agg_counter_end_, 0, job_id, num_blocks);
     }
 
-    // For a workgroup that does the work of `count` of the num_blocks workgroups the scheduler counts (not under per-workgroup
+    // For a workgroup that does the work of `count` (at least one) of the num_blocks workgroups the scheduler counts (not under per-workgroup
     // timing): the messages are those that `count` calls of end_from_one_lane would send.
     __device__ __forceinline__ void end_many_from_one_lane(JobId job_id, unsigned num_blocks, unsigned count) {
-        if (count == 0) return;
         const unsigned batch = batch_mask_ + 1;
         const unsigned before = atomicAdd(&agg_counter_end_, count), total = before + count;
         // the last one leaves the counter at zero, ahead of the message that lets the next kernel start
