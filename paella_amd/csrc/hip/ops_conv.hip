@@ -2356,17 +2356,17 @@ extern "C" int paella_pack_stats(uint64_t* launches, uint64_t* members) {
 
 namespace {
 
-// The members of a group call on 16-row tiles, if all of them have that form.  Returns 1 when launched, 0 when not, else an error.
-int launch_small_group(const paella_conv_plan* const* plans, const ConvArgs* args, int n, const paella::PoolArgs* pool, void* stream) {
+// The members of a group call on 16-row tiles, if all of them have that form; false where they have not, else *rc says how it went.
+bool launch_small_group(const paella_conv_plan* const* plans, const ConvArgs* args, int n, const paella::PoolArgs* pool, void* stream, int* rc) {
     const ConvArgs* each[kMaxGroup];
     for (int i = 0; i < n; ++i) each[i] = args + i;
     const int mi = small_form(plans, each, n);
-    if (!mi) return 0;
+    if (!mi) return false;
     SmallGroupArgs g;
     unsigned next = 0, lds = 0;
     for (int i = 0; i < n; ++i) {
         unsigned grid = 0;
-        if (!fill_small(plans[i], args[i], mi, g.m[i], &grid)) return 0;
+        if (!fill_small(plans[i], args[i], mi, g.m[i], &grid)) return false;
         next = align_start(next);
         g.start[i] = next;
         next += grid;
@@ -2381,10 +2381,11 @@ int launch_small_group(const paella_conv_plan* const* plans, const ConvArgs* arg
         next += (unsigned)(((size_t)pool->C * pool->P * pool->Q + block - 1) / block);
     }
     auto kern = mi == 1 ? conv_small_group_kernel<1> : conv_small_group_kernel<2>;
-    if (int rc = allow_lds(reinterpret_cast<const void*>(kern), lds)) return rc;
+    *rc = allow_lds(reinterpret_cast<const void*>(kern), lds);
+    if (*rc) return true;
     paella::launch(kern, dim3(next), dim3(64u * kSmallWaves), lds, reinterpret_cast<hipStream_t>(stream), g);
-    const int rc = (int)hipGetLastError();
-    return rc ? rc : 1;
+    *rc = (int)hipGetLastError();
+    return true;
 }
 
 }  // namespace
@@ -2408,7 +2409,7 @@ extern "C" int paella_conv2d_launch_group(const paella_conv_operands* members, i
         dyn_lds = std::max(dyn_lds, m.plan->dims.lds_bytes);
     }
     if (pack_hold(plans, args, n, stream)) return 0;
-    if (const int rc = launch_small_group(plans, args, n, nullptr, stream)) return rc == 1 ? 0 : rc;
+    if (int rc = 0; launch_small_group(plans, args, n, nullptr, stream, &rc)) return rc;
     for (int i = 0; i < n; ++i) {
         next = align_start(next);
         g.m[i].conv = args[i];
@@ -2468,7 +2469,7 @@ extern "C" int paella_conv2d_launch_group_pool(const paella_conv_operands* membe
     if (!paella::pool_fill_args(pool, pool_x, pool_y, job_id, notifier, &pa)) return PAELLA_EINVAL;
     const unsigned pool_grid = dims.grid - next;
     if (pack_hold(plans, args, n, stream, &pa, pool_grid)) return 0;
-    if (const int rc = launch_small_group(plans, args, n, &pa, stream)) return rc == 1 ? 0 : rc;
+    if (int rc = 0; launch_small_group(plans, args, n, &pa, stream, &rc)) return rc;
     next = 0;
     for (int i = 0; i < n; ++i) {
         next = align_start(next);

@@ -1,7 +1,9 @@
 // Which kernel a conv's launch takes, with how many workgroups and how much LDS, without a device: the runtime's entry points and the direct-dispatch
 // layer are taken by the functions below (an executable's definitions come before a library's).
-// Reads lines "alone|packed|transformed C K H W R S stride pad tile_hint small flags times" (flags: bits of the job id), calls each layer that often and
-// prints a line per call: "kernel grid dynamic_lds allowed_lds" per launch, separated by ';'.  packed: held by launch packing until all are in.
+// Reads lines "alone|packed|transformed|group|refused|refused_group C K H W R S stride pad tile_hint small flags times" (flags: bits of the job id), calls
+// each layer that often and prints a line: the plan's workgroups, then "kernel grid dynamic_lds allowed_lds" per launch, separated by ';'.
+// packed, transformed: held by launch packing until all are in; group: each call has the layer twice.  refused: the runtime refuses the launch
+// (hipErrorInvalidValue); printed is what the call returned.
 
 #include "../../paella_amd/csrc/hip/direct_dispatch.h"
 #include "paella_ops.h"
@@ -23,6 +25,8 @@ std::map<const void*, std::string>& names() {  // filled while the libraries are
 }
 std::map<const void*, int> g_allowed_lds;
 std::string g_out;
+bool g_refuse = false;
+hipError_t g_last_error = hipSuccess;
 char g_queue;  // its address is the one direct queue's handle
 
 struct {
@@ -72,14 +76,18 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 }
 hipError_t hipLaunchKernel(const void* kernel, dim3 grid, dim3, void**, size_t lds, hipStream_t) {
     note(kernel, grid, lds);
-    return hipSuccess;
+    return g_last_error = g_refuse ? hipErrorInvalidValue : hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void* kernel, hipFuncAttribute what, int value) {
     if (what == hipFuncAttributeMaxDynamicSharedMemorySize) g_allowed_lds[kernel] = value;
     return hipSuccess;
 }
 hipError_t hipFuncGetAttributes(hipFuncAttributes*, const void*) { return hipErrorNoDevice; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+    const hipError_t e = g_last_error;
+    g_last_error = hipSuccess;
+    return e;
+}
 
 int paella_direct_queue_shared(void** queue) {
     *queue = &g_queue;
@@ -113,16 +121,21 @@ int main() {
         paella_conv_plan plan;
         if (paella_conv2d_plan(&d, 0, hint, &plan)) return 1;
         if (small >= 0) plan.small = small;
-        const bool packed = route != "alone";
+        g_refuse = route.rfind("refused", 0) == 0;
+        const bool packed = route == "packed" || route == "transformed", group = route.find("group") != std::string::npos;
+        const paella_conv_operands member = {&plan, memory, memory, memory, nullptr, nullptr, memory, memory};
+        const paella_conv_operands members[2] = {member, member};
         void* const stream = packed ? &g_queue : nullptr;
         if (packed && paella_pack_enable(1)) return 1;
         for (int i = 0; i < times; ++i) {
             const uint32_t job = (uint32_t)(i + 1) | flags;
-            const int rc = route == "transformed"
+            const int rc = group ? paella_conv2d_launch_group(members, 2, stream, job, nullptr)
+                           : route == "transformed"
                                ? paella_conv2d_launch_transformed(&plan, memory, memory, memory, PAELLA_ACT_RELU, memory, memory, nullptr, nullptr, memory,
                                                                   memory, stream, job, nullptr)
                                : paella_conv2d_launch(&plan, memory, memory, memory, nullptr, nullptr, memory, memory, stream, job, nullptr);
-            if (rc) return 1;
+            if (g_refuse) g_out = "returned " + std::to_string(rc);
+            else if (rc) return 1;
         }
         if (packed && paella_pack_enable(0)) return 1;
         std::printf("%u %s\n", plan.dims.grid, g_out.c_str());

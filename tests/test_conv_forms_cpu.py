@@ -7,15 +7,19 @@ import pytest
 from _fake import FAKE_LIB, ensure_built
 
 
-def launches(*layers):
-    """Per layer (route, C, K, H, W, R, S, stride, pad, tile hint, small, flags of the job id, calls): the plan's workgroups, and for each launch
-    (kernel, workgroups, dynamic LDS, the most that was asked for)."""
+def check(layers):
+    """A line per layer (route, C, K, H, W, R, S, stride, pad, tile hint, small, flags of the job id, calls)."""
     ensure_built()
     out = subprocess.run([os.path.join(FAKE_LIB, "launch_check")], input="".join(" ".join(map(str, x)) + "\n" for x in layers), capture_output=True,
                          text=True, timeout=60)
     assert out.returncode == 0, out.stderr
+    return out.stdout.splitlines()
+
+
+def launches(*layers):
+    """Per layer the plan's workgroups, and for each launch (kernel, workgroups, dynamic LDS, the most that was asked for)."""
     res = []
-    for line in out.stdout.splitlines():
+    for line in check(layers):
         grid, _, rest = line.partition(" ")
         res.append((int(grid), [(a, int(b), int(c), int(d)) for a, b, c, d in (x.split() for x in rest.split(";"))]))
     return res
@@ -101,3 +105,14 @@ def test_which_convs_take_two_tiles_in_a_launch_of_several(layer, want):
     [(grid, [launch])] = launches(layer)
     rows, n = (layer[2] + 31) // 32, layer[-1]
     assert launch[1] == in_all(n, grid if want == ONE else grid // rows * ((rows + 1) // 2))
+
+
+@pytest.mark.parametrize("layer, kernel", [
+    ((64, 64, 14, 14, 1, 1, 1, 0, 0, -1, 0, 1), "conv_small"), ((64, 64, 56, 56, 3, 3, 1, 1, 0, -1, 0, 1), "conv_mfma"),
+    ((64, 64, 112, 112, 3, 3, 1, 1, 0, -1, 0, 1), "conv_tall"),
+])
+def test_a_launch_that_the_runtime_refuses_is_no_success(layer, kernel):
+    """... by itself and of a group of two (which has no form of two tiles), with the error that is also the number 1."""
+    [(_, [alone]), (_, [group])] = launches(("alone",) + layer, ("group",) + layer)
+    assert alone[0].startswith(kernel) and group[0].startswith(kernel.replace("tall", "mfma") + "_group")
+    assert [x.split()[1:] for x in check([("refused",) + layer, ("refused_group",) + layer])] == [["returned", "1"]] * 2
