@@ -122,11 +122,12 @@ def conv_roofline(models, hip, model, reps, back_to_back=200):
             "by_op": by_op, "direct_rps": direct_rps, "forward_us": sum(per_stage)}
 
 
-def full_device_pass(models, hip, model, images=16, reps=10, timed=True, kw=None, depth=0, only=None, burst=8, transform=False):
+def full_device_pass(models, hip, model, images=16, reps=10, timed=True, kw=None, depth=0, only=None, burst=8, transform=False, one_tile=False):
     """The conv kernel with the device full: every distinct conv layer of the model (groups == 1) over `images` inputs stacked
     along the height, i.e. with `images` times the pixel tiles -- what the compute units see on the serving path, where packed
     launches on four queues keep 16 to 24 problems in flight -- on the 32 x 32 tile with the layer's own waves per workgroup and
-    no split of the reduction over workgroups, one launch at a time on a HIP stream.  timed: durations from the kernel's own
+    no split of the reduction over workgroups, one launch at a time on a HIP stream.  The library chooses the workgroups: of two tiles,
+    as served launches have from 768 on, or of one; one_tile (and kw, depth, transform, which have no other form): of one throughout.  timed: durations from the kernel's own
     begin and end stamps, of the last of `burst` launches enqueued back to back (stream order: they do not overlap; the ones in
     front keep the device's clocks from dropping in the idle gap that a synchronize per launch leaves); otherwise one launch per
     layer with a synchronize after each (for counter collection)."""
@@ -160,7 +161,7 @@ def full_device_pass(models, hip, model, images=16, reps=10, timed=True, kw=None
         # forced shape: waves per workgroup (the layer's own unless given) and chunks of operands in flight per wave (0: default)
         use_kw = kw if kw and c % 8 == 0 else alone.plan.kw
         use_depth = depth if c % 8 == 0 else 0
-        hint = (use_depth << 16) | (1 << 8) | (1 << 4) | (use_kw.bit_length() - 1)
+        hint = (use_depth << 16) | (1 << 8) | (1 << 4) | (use_kw.bit_length() - 1) | (0 if one_tile or kw or depth or transform else 1 << 20)
         conv = ops.Conv2d(wt, np.zeros(k, np.float32), stride=tuple(node["stride"]), pad=tuple(node["pad"]), dil=tuple(node["dil"]), act=ops.ACT_RELU,
                           in_hw=(h * images, w), tile_hint=hint)
         xin = torch.randn((1, c, h * images, w), device="cuda:0")
@@ -198,8 +199,10 @@ def full_device_pass(models, hip, model, images=16, reps=10, timed=True, kw=None
         flops = sum(r["flops"] * r["count"] for r in rows)
         us = sum(r["us"] * r["count"] for r in rows)
         out.update({"achieved": flops / us / 1e6, "frac": flops / us / 1e6 / FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                    "how": "every conv layer of %s over %d inputs stacked along the height (%d times the pixel tiles), 32 x 32 tile, one launch at a time "
-                           "(the last of %d enqueued back to back); layers weighted by their count in a forward pass" % (model, images, images, max(1, burst))})
+                    "how": "every conv layer of %s over %d inputs stacked along the height (%d times the pixel tiles), 32 x 32 tile, workgroups of %s, one launch at a time "
+                           "(the last of %d enqueued back to back); layers weighted by their count in a forward pass" %
+                           (model, images, images, "one tile" if one_tile or kw or depth or transform else "two tiles or one as the library chooses",
+                            max(1, burst))})
     return out
 
 
@@ -430,7 +433,7 @@ def roofline_of(rl, model):
     achieved = rl["conv_flops"] / (rl["conv_us"] * 1e-6) / 1e12
     return {"bound": "mfma", "achieved": achieved, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / FP32_MFMA_PEAK_TFLOPS,
             "traffic": CONV_TRAFFIC_BYTES_PER_LAUNCH.get(model),
-            "kernel": "conv_mfma_kernel, conv_small_kernel and their grouped forms (all %d conv launches of one %s forward pass, one at a time on an idle device)" % (rl["conv_launches"], model),
+            "kernel": "conv_mfma_kernel, conv_small_kernel, conv_tall_kernel and their grouped forms (all %d conv launches of one %s forward pass, one at a time on an idle device)" % (rl["conv_launches"], model),
             "flops_per_launch_avg": rl["conv_flops"] / rl["conv_launches"], "us_per_launch_avg": rl["conv_us"] / rl["conv_launches"],
             "algorithmic_bytes_per_launch_avg": rl["by_op"]["conv"]["bytes"] / rl["conv_launches"]}
 
@@ -468,6 +471,7 @@ def main():
     ap.add_argument("--fd-images", type=int, default=16)
     ap.add_argument("--fd-transform", action="store_true",
                     help="with --full-device: a per-channel scale-shift applied to the input of every layer that can take one (conv_mfma_pre_kernel)")
+    ap.add_argument("--fd-one-tile", action="store_true", help="with --full-device: workgroups of one 32 x 32 tile throughout")
     ap.add_argument("--fd-burst", type=int, default=8, help="with --full-device: launches enqueued back to back per sample; the last one is timed")
     ap.add_argument("--counter-pass", default=None, metavar="MODEL",
                     help="only this: three forward passes of MODEL, one launch at a time with a synchronize after each (the leg to run "
@@ -493,7 +497,8 @@ def main():
         return
     if args.full_device:
         fd = full_device_pass(models, hip, args.full_device, images=args.fd_images, timed=not under_counter_collection(), kw=args.fd_kw, depth=args.fd_depth,
-                              only=args.fd_only.split(",") if args.fd_only else None, burst=args.fd_burst, transform=args.fd_transform)
+                              only=args.fd_only.split(",") if args.fd_only else None, burst=args.fd_burst, transform=args.fd_transform,
+                              one_tile=args.fd_one_tile)
         for r in fd["layers"]:
             log("[bench] %-26s x%d  %5d workgroups x %d waves  %8.1f MFLOP  %s%s" % (r["layer"], r["count"], r["workgroups"], r["waves_per_workgroup"], r["flops"] / 1e6,
                 "%7.2f us  %6.1f TFLOP/s" % (r["us"], r["flops"] / r["us"] / 1e6) if r["us"] else "", "  (input transformed)" if r["input_transformed"] else ""))
@@ -951,7 +956,7 @@ def headline(out):
         if k in out:
             line[k] = out[k]
     r = {k: rf.get(k) for k in ("bound", "achieved", "peak", "unit", "frac", "traffic") if k in rf}
-    r["kernel"] = "conv_mfma_kernel, conv_small_kernel (+ grouped forms), Inception-v3's conv launches one at a time"
+    r["kernel"] = "conv_mfma_kernel, conv_small_kernel, conv_tall_kernel (+ grouped forms), Inception-v3's conv launches one at a time"
     for k in ("flops_per_launch_avg", "us_per_launch_avg", "algorithmic_bytes_per_launch_avg", "peak_measured", "empty_kernel_us"):
         if k in rf:
             r[k] = rf[k]
