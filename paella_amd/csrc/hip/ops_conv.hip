@@ -836,7 +836,7 @@ __global__ __launch_bounds__(64 * KW, (MI * NI == 1 && KW == 8 && DEPTH == 0) ? 
     else conv_tile<MI, NI, KW, TAP_MAJOR, kPreNone, DEPTH>(p, blockIdx.x);
 }
 
-// Workgroups of two 32 x 32 tiles, one under the other, for launches that fill the device (kTallFrom says which).  What bounds those is a
+// Workgroups of two 32 x 32 tiles, one under the other, for launches that fill the device (kTallFrom and tall_alone say which).  What bounds those is a
 // compute unit's vector cache: per 32 reduction steps a wave's sixteen dword loads of inputs and four 16-byte loads of weights take it some
 // 450 cycles, 1800 for the four waves that have the 1024 cycles of a SIMD's matrix instructions to hide them.  Two tiles share the inputs:
 // 560 cycles to twice the matrix instructions.  Two tiles also share a wave's prologue.  The tiles' sums go through LDS one after the other
@@ -1388,6 +1388,8 @@ ConvKernel pick_kw(int kw) {
     }
 }
 
+// Tiles other than 32 x 32 are for callers that ask for them (tile_hint of paella_conv2d_plan, and plans that were stored when thousands of tiles
+// took them): the plan's own rule has none of them any more.
 template <bool TM>
 ConvKernel pick_tile(int mi, int ni, int kw) {
     if (mi == 1 && ni == 1) return pick_kw<1, 1, TM>(kw);
