@@ -116,3 +116,20 @@ def test_a_launch_that_the_runtime_refuses_is_no_success(layer, kernel):
     [(_, [alone]), (_, [group])] = launches(("alone",) + layer, ("group",) + layer)
     assert alone[0].startswith(kernel) and group[0].startswith(kernel.replace("tall", "mfma") + "_group")
     assert [x.split()[1:] for x in check([("refused",) + layer, ("refused_group",) + layer])] == [["returned", "1"]] * 2
+
+
+# The layers of tests/test_conv_tall_gpu.py, whose results and message counts are those of either form: which one they compare.
+EDGES = [(64, 33, 1, 1, 1, 1, 1, 0, 0x0113), (72, 64, 5, 7, 1, 1, 1, 0, 0x0113), (64, 65, 4, 8, 3, 3, 1, 1, 0), (64, 96, 11, 3, 3, 3, 1, 1, 0x2113),
+         (128, 128, 9, 9, 3, 3, 2, 1, 0x1113), (128, 160, 8, 8, 3, 3, 2, 0, 0), (96, 100, 9, 9, 1, 7, 1, 0, 0), (96, 64, 11, 11, 1, 1, 2, 0, 0),
+         (512, 128, 7, 7, 3, 3, 1, 1, 0), (3, 64, 31, 33, 7, 7, 2, 3, 0), (5, 65, 9, 11, 3, 3, 1, 1, 0x0112), (3, 96, 13, 13, 5, 5, 1, 2, 0x1112)]
+
+
+@pytest.mark.parametrize("layer", EDGES)
+def test_a_launch_that_is_asked_for_two_tiles_takes_them(layer):
+    assert [form(launch) for _, [launch] in launches(("alone",) + layer + (4, 0, 1), ("alone",) + layer + (0, 0, 1))] == [TWO, ONE]
+
+
+@pytest.mark.parametrize("k, h, want", [(64, 97, ONE), (64, 112, TWO), (96, 91, ONE), (256, 80, TWO), (320, 80, TWO)])
+def test_which_of_the_layers_on_the_device_take_two_tiles(k, h, want):
+    [(_, [launch])] = launches(alone(64, k, h, h))
+    assert form(launch) == want
