@@ -45,6 +45,9 @@ class Client {
 
     // Sleeps on the wake-up socket, then spins on the completion ring for the finished instance.
     JobInstanceRef* wait();
+    // The same, but nullptr when nothing has finished after `seconds`: for programs that would rather fail than hang when a request
+    // is never answered.  Not in the reference.
+    JobInstanceRef* wait_for(double seconds);
 
     ProfilerClient* get_profiler_client() { return &profiler_client_; }
 
@@ -58,6 +61,7 @@ class Client {
     ipc::ShmChannelCpuWriter c2s_channel_;
     ipc::ShmChannelCpuReader s2c_channel_;
     ipc::UnixDatagramSocket s2c_socket_;
+    bool woken_ = false;  // a wake-up was taken whose request had not completed in time
 
     std::vector<std::unique_ptr<JobInstanceRef>> job_instance_refs_;
     std::vector<JobInstanceRefId> unused_job_instance_refs_;

@@ -62,6 +62,7 @@ class ShmPrimitiveChannelBase {
 
     size_t get_count() const { return count_; }
     T* get_slots() const { return slots_; }
+    unsigned get_read_pos() const { return read_pos_; }  // of this endpoint
     unsigned* get_cursor() const { return cursor_; }
 
     template <typename U>

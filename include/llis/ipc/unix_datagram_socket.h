@@ -33,6 +33,9 @@ class UnixDatagramSocket {
     // sandboxed kernels, the queue is full.
     bool try_write(const void* buf, size_t count, bool* refused = nullptr);
     ssize_t read(void* buf, size_t count);
+    // read() that gives up, with false, after the time set by set_read_timeout (never, unless it was called).
+    void set_read_timeout(unsigned milliseconds);
+    bool try_read(void* buf, size_t count);
 
   private:
     UnixDatagramSocket(int fd, bool owner) : fd_(fd), owner_(owner) {}

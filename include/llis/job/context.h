@@ -62,7 +62,14 @@ class Context {
         for (unsigned i = 0; i < num_poll_hooks_; ++i) poll_hooks_[i]();
     }
 
+    // What a job library adds to the scheduler's report of a stall (see StreamPoolScheduler::report_stall), on the serving thread.
+    static void set_report_hook(PollHook fn) { report_hook_ = fn; }
+    static void run_report_hook() {
+        if (report_hook_) report_hook_();
+    }
+
   private:
+    static PollHook report_hook_;
     static constexpr unsigned kMaxPollHooks = 8;
     static PollHook poll_hooks_[kMaxPollHooks];
     static unsigned num_poll_hooks_;

@@ -136,6 +136,7 @@ class Job {
     bool reports_charged_blocks() const { return reports_charged_; }
 
     bool is_running() const { return is_running_; }
+    unsigned get_num_running_blocks() const { return num_running_blocks_; }  // workgroups of the stage that have not reported their end
     void unset_running() { is_running_ = false; }
 
     // The scheduler is about to resume the job for its next stage on `stream`.

@@ -16,6 +16,7 @@
 #include <llis/job/job.h>
 #include <llis/server/server.h>
 
+#include <chrono>
 #include <functional>
 #include <memory>
 #include <string>
@@ -118,6 +119,11 @@ class StreamPoolScheduler : public Scheduler {
     void post_mem_completion(job::Job* job);
     void spin_sleep() const;
 
+    // Once, when nothing has been reported for 20 s (LLIS_STALL_REPORT_S) with jobs in flight: what the scheduler, the ring and the
+    // jobs' queues hold goes to stderr (a kernel that takes longer makes a harmless line).
+    void look_for_stall();
+    void report_stall() const;
+
     SchedulerOptions options_;
     unsigned num_jobs_ = 0;
     // Compute-unit id of the message being handled (InstrumentInfo.smid): meaningful inside handle_block_start / _finish for
@@ -137,6 +143,11 @@ class StreamPoolScheduler : public Scheduler {
     std::unordered_map<void*, unsigned> stream_index_;
     std::vector<std::unique_ptr<job::Job>> job_id_to_job_map_;
     std::vector<JobId> unused_job_id_;
+
+    uint32_t idle_turns_ = 0;                            // turns of the serving loop since a message came in
+    std::chrono::steady_clock::time_point quiet_since_;  // when that was first looked at
+    bool stall_reported_ = false;
+    double stall_after_s_ = 20;
 };
 
 }  // namespace server

@@ -147,10 +147,20 @@ int main(int argc, char** argv) {
 
     // Warm-up: create every pooled instance and run it once (one at a time in verify mode, which also learns the expected outputs).
     const auto init_start = Clock::now();
-    gen.warm_up(job_refs);
+    try {
+        gen.warm_up(job_refs);
+    } catch (const std::exception& e) {
+        std::fprintf(stderr, "llis_app_client: %s\n", e.what());
+        return 4;
+    }
     const double init_us = std::chrono::duration<double, std::micro>(Clock::now() - init_start).count();
 
-    gen.run();
+    try {
+        gen.run();
+    } catch (const std::exception& e) {
+        std::fprintf(stderr, "llis_app_client: %s\n", e.what());
+        return 4;
+    }
 
     const double elapsed = gen.elapsed_us();
     Stats all = summarize(gen.latencies());

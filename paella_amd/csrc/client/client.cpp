@@ -4,6 +4,7 @@
 
 #include <dlfcn.h>
 
+#include <chrono>
 #include <random>
 #include <stdexcept>
 
@@ -27,6 +28,7 @@ Client::Client(std::string server_name)
     s2c_channel_.disconnect();
     s2c_channel_.connect(ipc::s2c_channel_name(server_name_, client_id_));
     s2c_socket_.bind(ipc::s2c_socket_name(server_name_, client_id_));
+    s2c_socket_.set_read_timeout(200);  // for wait_for
 }
 
 Client::~Client() {}
@@ -70,11 +72,24 @@ void Client::release_job_instance_ref(JobInstanceRef* ref) {
 }
 
 JobInstanceRef* Client::wait() {
-    bool woken;
-    s2c_socket_.read(&woken, sizeof(woken));  // sent when the request's last stage is dispatched
+    bool poke;
+    while (!woken_) woken_ = s2c_socket_.try_read(&poke, sizeof(poke));  // sent when the request's last stage is dispatched
+    woken_ = false;
     JobInstanceRef* done;
     s2c_channel_.read(&done);  // posted when it has completed
     return done;
+}
+
+JobInstanceRef* Client::wait_for(double seconds) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::duration<double>(seconds);
+    bool poke;
+    while (!woken_) {
+        woken_ = s2c_socket_.try_read(&poke, sizeof(poke));
+        if (!woken_ && std::chrono::steady_clock::now() >= until) return nullptr;
+    }
+    for (unsigned turn = 1; !s2c_channel_.can_read(); ++turn)
+        if (turn % 1024 == 0 && std::chrono::steady_clock::now() >= until) return nullptr;
+    return wait();
 }
 
 }  // namespace client

@@ -495,6 +495,18 @@ extern "C" int paella_direct_queue_shared(void** out) {
     return 0;
 }
 
+extern "C" void paella_direct_report_hook(void) {
+    std::lock_guard<std::mutex> lock(paella::g_shared_mutex);
+    for (void* h : paella::g_shared_queues) {
+        DirectQueue* q = static_cast<DirectQueue*>(h);
+        const unsigned long long taken = hsa_queue_load_read_index_scacquire(q->queue);
+        std::fprintf(stderr, "[paella]   direct queue: %llu packets written, %llu taken\n", (unsigned long long)q->write_index, taken);
+    }
+    uint64_t launches = 0, members = 0;
+    const int held = paella_pack_stats(&launches, &members);
+    std::fprintf(stderr, "[paella]   launch packing: %d held, %llu launches of %llu members so far\n", held, (unsigned long long)launches, (unsigned long long)members);
+}
+
 extern "C" int paella_direct_queue_set_ordered(void* queue, int ordered) {
     DirectQueue* q = paella::direct_queue_lookup(queue);
     if (!q) return PAELLA_EINVAL;

@@ -2,6 +2,7 @@
 #include <llis/utils/error.h>
 
 #include <sys/socket.h>
+#include <sys/time.h>
 #include <unistd.h>
 
 #include <cerrno>
@@ -86,6 +87,18 @@ ssize_t UnixDatagramSocket::read(void* buf, size_t count) {
     ssize_t n = ::read(fd_, buf, count);
     LLIS_CHECK_POSIX(n);
     return n;
+}
+
+void UnixDatagramSocket::set_read_timeout(unsigned milliseconds) {
+    const timeval t = {(time_t)(milliseconds / 1000), (suseconds_t)(milliseconds % 1000 * 1000)};
+    LLIS_CHECK_POSIX(::setsockopt(fd_, SOL_SOCKET, SO_RCVTIMEO, &t, sizeof(t)));
+}
+
+bool UnixDatagramSocket::try_read(void* buf, size_t count) {
+    const ssize_t n = ::read(fd_, buf, count);
+    if (n < 0 && (errno == EAGAIN || errno == EWOULDBLOCK || errno == EINTR)) return false;
+    LLIS_CHECK_POSIX(n);
+    return true;
 }
 
 }  // namespace ipc

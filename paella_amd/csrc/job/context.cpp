@@ -11,6 +11,7 @@ ipc::Gpu2SchedChannel Context::gpu2sched_block_time_channel_;
 ipc::ShmChannelCpuWriter Context::mem2sched_channel_;
 Context::PollHook Context::poll_hooks_[Context::kMaxPollHooks] = {};
 unsigned Context::num_poll_hooks_ = 0;
+Context::PollHook Context::report_hook_ = nullptr;
 
 void Context::add_poll_hook(PollHook fn) {
     if (!fn) return;

@@ -137,6 +137,7 @@ class ModelJob : public llis::job::CoroutineJob {
         const char* pack = std::getenv("PAELLA_PACK");
         pack_ = direct_ && !(pack && std::strcmp(pack, "0") == 0);
         if (pack_) llis::job::Context::add_poll_hook(&paella_pack_poll_hook);  // one address for every adapter library: registered once
+        if (direct_) llis::job::Context::set_report_hook(&paella_direct_report_hook);
         // The staging copy of an input too large for zero-copy leaves the serving thread unless PAELLA_STAGE_THREAD=0; only
         // under a scheduler that waits for a stage's completion before it issues the next one.
         const char* st = std::getenv("PAELLA_STAGE_THREAD");

@@ -9,6 +9,9 @@
 //   * latency = completion time - scheduled arrival time; percentiles are sorted[size * q] (truncated).
 // iat == 0 submits as fast as the caps allow (saturation).
 //
+// A request that is never answered ends the run with an exception: with requests outstanding and no completion for
+// LLIS_CLIENT_STALL_S seconds (default 60; 0 waits for ever, as the reference does).
+//
 // Verify mode (Options::verify_variants > 0; the reference's client checks no output at all): every pooled instance carries one
 // of `verify_variants` seeded inputs of its job type (verify_input below), the warm-up runs the instances ONE AT A TIME on the
 // otherwise idle server and keeps the first output of every (type, variant) as that pair's expectation, and from then on every
@@ -27,11 +30,14 @@
 #include <chrono>
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <queue>
 #include <random>
+#include <stdexcept>
 #include <string>
 #include <thread>
 #include <vector>
@@ -42,6 +48,11 @@ namespace loadgen {
 using Clock = std::chrono::steady_clock;
 
 inline double us_since_epoch(Clock::time_point t) { return std::chrono::duration<double, std::micro>(t.time_since_epoch()).count(); }
+
+inline double stall_seconds() {
+    const char* s = std::getenv("LLIS_CLIENT_STALL_S");
+    return s && *s ? std::atof(s) : 60.0;
+}
 
 struct Stats {
     double mean = 0, p50 = 0, p90 = 0, p95 = 0, p99 = 0, max = 0, sd = 0;
@@ -160,7 +171,7 @@ class LoadGenerator {
                 std::memcpy(inst->get_input_ptr(), inputs[v].data(), in_bytes);
                 std::memset(inst->get_output_ptr(), 0xFF, out_size_[t]);
                 inst->launch();
-                if (client_->wait() != inst) throw std::runtime_error("verify warm-up: a completion for another instance");
+                if (next_completion([] { return true; }) != inst) throw std::runtime_error("verify warm-up: a completion for another instance");
                 std::vector<char>& want = expected_[t][v];
                 if (want.empty() && out_size_[t]) {
                     want.assign(static_cast<char*>(inst->get_output_ptr()), static_cast<char*>(inst->get_output_ptr()) + out_size_[t]);
@@ -169,7 +180,7 @@ class LoadGenerator {
                 }
             }
         }
-        for (unsigned i = 0; i < total; ++i) client_->wait();
+        for (unsigned i = 0; i < total; ++i) next_completion([] { return true; });
         if (variants) {
             // ... and once more all at once, as the reference's warm-up does: the server builds a pooled job instance of its own
             // for every request in flight (device arena, workspace, weights on first use), which the one-at-a-time pass above
@@ -182,7 +193,7 @@ class LoadGenerator {
                 it.first->launch();
             }
             for (size_t i = 0; i < all.size(); ++i) {
-                llis::client::JobInstanceRef* inst = client_->wait();
+                llis::client::JobInstanceRef* inst = next_completion([] { return true; });
                 check(inst, type_of_ref_[inst->get_job_ref_id()]);
             }
         }
@@ -244,7 +255,14 @@ class LoadGenerator {
     void phase(unsigned num_jobs, bool record) {
         phase_jobs_ = num_jobs;
         phase_record_ = record;
-        std::thread monitor_thr([this] { monitor(); });
+        std::thread monitor_thr([this] {
+            try {
+                monitor();
+            } catch (...) {
+                failure_ = std::current_exception();
+                failed_.store(true, std::memory_order_release);
+            }
+        });
         std::thread submit_thr([this] { submit(); });
         if (opt_.pin_threads) {
             pin(monitor_thr, 0);
@@ -252,6 +270,17 @@ class LoadGenerator {
         }
         monitor_thr.join();
         submit_thr.join();
+        if (failure_) std::rethrow_exception(failure_);
+    }
+
+    // The next request that has completed; `outstanding` says whether one is due at all.
+    template <typename F>
+    llis::client::JobInstanceRef* next_completion(F outstanding) {
+        if (stall_s_ <= 0) return client_->wait();
+        for (;;) {
+            if (llis::client::JobInstanceRef* inst = client_->wait_for(stall_s_)) return inst;
+            if (outstanding()) throw std::runtime_error("a request was not answered: no completion for " + std::to_string((int)stall_s_) + " s with requests outstanding");
+        }
     }
 
     static void pin(std::thread& thr, int cpu) {
@@ -273,6 +302,7 @@ class LoadGenerator {
         free_instances_[type].pop_back();
         ++outstanding_per_type_[type];
         inst->set_start_time(scheduled_arrival_us);
+        last_launch_ = Clock::now();
         if (opt_.verify_variants && out_size_[type]) std::memset(inst->get_output_ptr(), 0xFF, out_size_[type]);
         inst->launch();
     }
@@ -297,7 +327,13 @@ class LoadGenerator {
     void monitor() {
         const auto very_start = Clock::now();
         for (unsigned done = 0; done < phase_jobs_; ++done) {
-            llis::client::JobInstanceRef* inst = client_->wait();
+            llis::client::JobInstanceRef* inst = next_completion([this] {
+                const auto quiet_since = Clock::now() - std::chrono::duration<double>(stall_s_);
+                std::lock_guard<std::mutex> lk(mtx_);
+                unsigned n = 0;
+                for (unsigned o : outstanding_per_type_) n += o;
+                return n != 0 && last_launch_ <= quiet_since;
+            });
             const auto now = Clock::now();
             const double latency = us_since_epoch(now) - inst->get_start_time();
             const double t = std::chrono::duration<double, std::micro>(now - very_start).count();
@@ -349,13 +385,14 @@ class LoadGenerator {
         const double start_us = us_since_epoch(start_time_);
         unsigned submitted = 0;
 
-        while (submitted < phase_jobs_) {
+        while (submitted < phase_jobs_ && !failed_.load(std::memory_order_acquire)) {
             const double elapsed = std::chrono::duration<double, std::micro>(Clock::now() - start_time_).count();
             if (elapsed < next_submit) continue;
 
             if (num_outstanding_.load(std::memory_order_acquire) >= opt_.concurrency) {
                 ++num_queue_full_;
                 while (num_outstanding_.load(std::memory_order_acquire) >= opt_.concurrency) {
+                    if (failed_.load(std::memory_order_acquire)) return;
                 }
             }
             const unsigned type = replay ? trace_[trace_pos % trace_.size()].first
@@ -395,6 +432,10 @@ class LoadGenerator {
     std::vector<std::queue<double>> due_;
     std::vector<unsigned> outstanding_per_type_;
     std::atomic<int> num_outstanding_{0};
+    const double stall_s_ = stall_seconds();
+    Clock::time_point last_launch_;          // under mtx_
+    std::atomic<bool> failed_{false};        // the monitor has given up: failure_ says why
+    std::exception_ptr failure_;
 
     std::vector<unsigned> type_of_ref_;
     std::vector<std::pair<unsigned, double>> trace_;

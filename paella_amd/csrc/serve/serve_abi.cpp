@@ -195,11 +195,13 @@ int paella_client_single(const char* server_name, const char* job_path, const vo
         llis::client::JobInstanceRef* inst = job.create_instance();
         std::memset(inst->get_input_ptr(), 0, job.get_job()->get_input_size());
         if (input) std::memcpy(inst->get_input_ptr(), input, in_bytes);
+        const double stall_s = llis::loadgen::stall_seconds();
         for (int i = 0; i < n; ++i) {
             const auto t0 = std::chrono::steady_clock::now();
             inst->launch();
-            llis::client::JobInstanceRef* done = client.wait();
+            llis::client::JobInstanceRef* done = stall_s > 0 ? client.wait_for(stall_s) : client.wait();
             const auto t1 = std::chrono::steady_clock::now();
+            if (!done) throw std::runtime_error("a request was not answered for " + std::to_string((int)stall_s) + " s");
             if (done != inst) return -1;
             if (latencies_us) latencies_us[i] = std::chrono::duration<double, std::micro>(t1 - t0).count();
         }

@@ -5,6 +5,8 @@
 
 #include "paella_hip.h"
 
+#include <cstdio>
+#include <cstdlib>
 #include <stdexcept>
 
 namespace llis {
@@ -39,6 +41,7 @@ std::vector<std::string> SchedulerFactory::names() {
 
 StreamPoolScheduler::StreamPoolScheduler(const SchedulerOptions& options, size_t mem2sched_bytes)
     : options_(options), gpu2sched_channel_(options.ring_slots), mem2sched_channel_(mem2sched_bytes) {
+    if (const char* s = std::getenv("LLIS_STALL_REPORT_S")) stall_after_s_ = std::atof(s);
     job::Context::set_gpu2sched_channel(&gpu2sched_channel_);
     job::Context::set_mem2sched_channel(&mem2sched_channel_);
 
@@ -65,6 +68,7 @@ StreamPoolScheduler::~StreamPoolScheduler() {
 void StreamPoolScheduler::try_handle_block_start_finish() {
     if (gpu2sched_channel_.can_read<job::InstrumentInfo>()) {
         LLIS_PHASE(kRing);
+        idle_turns_ = 0;
         const job::InstrumentInfo info = gpu2sched_channel_.read<job::InstrumentInfo>();
         job::Job* job = job_of(info.job_id);
         cur_smid_ = info.smid;
@@ -83,6 +87,7 @@ void StreamPoolScheduler::try_handle_block_start_finish() {
     }
     else {
         LLIS_PHASE(kIdle);
+        if ((++idle_turns_ & ((1u << 20) - 1)) == 0) look_for_stall();  // a tenth of a second
     }
     while (options_.measure_block_time && gpu2sched_block_time_channel_.can_read<job::BlockStartEndTime>()) {
         // unpacking as in reference src/server/scheduler_full3.cpp:113-119
@@ -93,6 +98,7 @@ void StreamPoolScheduler::try_handle_block_start_finish() {
     }
     if (mem2sched_channel_.can_read()) {
         LLIS_PHASE(kRing);
+        idle_turns_ = 0;
         job::Job* job;
         mem2sched_channel_.read(&job);
         log_->add('M', job->get_id());
@@ -142,6 +148,38 @@ void StreamPoolScheduler::post_mem_completion(job::Job* job) {
 void StreamPoolScheduler::mem_notification_callback(void* job) {
     // Runs on a runtime thread; several streams may complete at once, so serialise whole messages.
     job::Context::post_mem_completion(static_cast<job::Job*>(job));
+}
+
+void StreamPoolScheduler::look_for_stall() {
+    const auto now = std::chrono::steady_clock::now();
+    if (idle_turns_ == 1u << 20 || num_jobs_ == 0) {
+        quiet_since_ = now;
+        stall_reported_ = false;
+    } else if (!stall_reported_ && std::chrono::duration<double>(now - quiet_since_).count() >= stall_after_s_) {
+        stall_reported_ = true;
+        report_stall();
+    }
+}
+
+void StreamPoolScheduler::report_stall() const {
+    const unsigned count = (unsigned)gpu2sched_channel_.get_count(), at = gpu2sched_channel_.get_read_pos();
+    unsigned unread = 0;  // messages behind a slot that was claimed and never written
+    for (unsigned i = 0; i < 64; ++i) {
+        const uint64_t bits = __atomic_load_n(gpu2sched_channel_.get_slots() + (at + i) % count, __ATOMIC_ACQUIRE);
+        job::InstrumentInfo info;
+        __builtin_memcpy(static_cast<void*>(&info), &bits, sizeof(bits));
+        unread += info.can_read();
+    }
+    std::fprintf(stderr, "[llis] no message for %.0f s with %u jobs in flight: %zu of %zu streams free, ring at %u with %u messages in the 64 slots from there\n",
+                 stall_after_s_, num_jobs_, free_streams_.size(), streams_.size(), at, unread);
+    unsigned shown = 0;
+    for (const std::unique_ptr<job::Job>& job : job_id_to_job_map_) {
+        if (!job || ++shown > 16) continue;
+        std::fprintf(stderr, "[llis]   job %u of type %u: stage %d (%u), %s, %u of its %u workgroups have not reported%s\n", job->get_id(), job->get_registered_job_id(),
+                     job->get_cur_stage(), job->get_cur_stage_span(), !job->is_running() ? "queued" : "running", job->get_num_running_blocks(),
+                     job->get_cur_num_blocks(), job->is_unfit() ? ", beyond the budget" : "");
+    }
+    job::Context::run_report_hook();
 }
 
 void StreamPoolScheduler::spin_sleep() const {

@@ -7,6 +7,7 @@
 //   FAKE_VARIANT 4  fake_self  : a copy stage that reports its own completion (from a thread of its own after 300 us when
 //                                FAKE_SELF_THREAD=1, else before it returns), copy, kernel of 40, copy(pre-notify); output = input + 1
 //   FAKE_VARIANT 5  fake_flaky : fake_mem3 whose every FAKE_FLAKY_EVERY-th run (counted over the process) answers with one wrong byte
+//   FAKE_VARIANT 7  fake_lost  : a kernel of 40 (pre-notify) that is never issued in every FAKE_LOST_EVERY-th run, so that nobody reports its end
 //   FAKE_VARIANT 6  fake_raw   : kernels of 40 and 300 workgroups with un-aggregated hooks, one of 17 with aggregated hooks, one of 500
 //                                with un-aggregated hooks (pre-notify)
 
@@ -85,6 +86,14 @@ class FakeJob : public llis::job::CoroutineJob {
         set_pre_notify();
         yield();
         llis_hip_memcpy_async(reinterpret_cast<char*>(io_ptr) + 100, buf_, 100, LLIS_HIP_D2H, reinterpret_cast<void*>(get_cuda_stream()));
+#elif FAKE_VARIANT == 7
+        static unsigned runs = 0;
+        const char* every = std::getenv("FAKE_LOST_EVERY");
+        set_num_blocks(40);
+        set_num_threads_per_block(128);
+        set_pre_notify();
+        yield();
+        if (!every || ++runs % (unsigned)std::atoi(every) != 0) fake_hip_kernel_launch(reinterpret_cast<void*>(get_cuda_stream()), get_id(), 40);
 #elif FAKE_VARIANT == 4
         set_is_mem();
         set_completes_itself();

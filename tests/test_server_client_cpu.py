@@ -183,6 +183,34 @@ print(json.dumps({"rps": r["throughput_rps"], "count": r["all"]["count"], "out":
     assert res["count"] == 200 and res["out"] == [6, 6, 6, 6] and res["log_lines"] > 1000
 
 
+@pytest.mark.parametrize("call, want", [
+    ("serve.client_run(s.name, [(JOB, 1.0, 6)], 0.0, 6, 200)", "paella_client_run: a request was not answered"),
+    ("serve.client_run(s.name, [(JOB, 1.0, 6)], 0.0, 6, 200, verify=2)", "paella_client_run: a request was not answered"),
+    ("serve.client_single(s.name, JOB, np.zeros(1, np.float32), 2, n=60)", "paella_client_single: a request was not answered"),
+])
+def test_a_request_that_is_never_answered_ends_the_run(call, want):
+    """The client gives up with an exception, the server says what it waits for, and both can be stopped."""
+    code = r'''
+import ctypes, os, sys
+sys.path.insert(0, %r)
+os.environ.update(FAKE_HIP_AUTORUN="1", FAKE_LOST_EVERY="50", LLIS_CLIENT_STALL_S="1.5", LLIS_STALL_REPORT_S="0.5")
+ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
+from paella_amd import serve, _abi
+_abi._cache["llis_hip"] = True
+import numpy as np
+JOB = %r
+with serve.Server("lost%%d" %% os.getpid(), "full3", num_streams=8) as s:
+    try:
+        %s
+    except RuntimeError as e:
+        print("raised")
+print("stopped")
+''' % (os.path.dirname(os.path.dirname(os.path.abspath(__file__))), os.path.join(FAKE_LIB, "libllis_hip.so"), fake_job("fake_lost"), call)
+    out = subprocess.run(["python3", "-c", code], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout.split() == ["raised", "stopped"], out.stderr
+    assert want in out.stderr and "[llis] no message for" in out.stderr and "40 of its 40 workgroups have not reported" in out.stderr
+
+
 def test_server_outlives_a_client_killed_mid_run(tmp_path):
     """A client that dies with requests in flight leaves wake-ups nobody will ever read: the server writes them off
     after the peer has refused them for two seconds, and a second client is served as if nothing had happened."""
