@@ -1789,6 +1789,12 @@ unsigned tall_grid(const paella_conv_plan* plan, const ConvArgs& a) {
 // more than such a launch needs (64->96 3x3 at 1602: 20.9 -> 26.3, 64->160 at 770: 13.2 -> 12.7).  Over 160 drawn layers of 768 to 9000 workgroups
 // (1 to 7 wide filters, strides 1 and 2, 3 to 1024 channels) the time is 1.003 of the faster form's; one tile throughout 1.098, two 1.022.
 bool tall_alone(const ConvArgs& a, unsigned one, unsigned two, bool table, unsigned lds_bytes) {
+    // The device holds three workgroups of two tiles per compute unit: the fourth has nothing to run beside it, which a pointwise
+    // reduction notices whose inputs are not in the caches of the XCDs (4 MB each).  At 1932 to 1954 workgroups of one tile, one -> two: 512->64
+    // (64 MB) 20.97 -> 23.59 us, 768->128 (47) 28.20 -> 32.34, 1024->256 (32) 37.11 -> 41.32, 256->64 (32) 13.26 -> 14.69, 768->256 (24) 28.59 -> 31.74, 672->256
+    // (21) 24.99 -> 28.95, 640->256 (20) 24.20 -> 26.85; the other way 320->128 (20) 14.89 -> 14.65, 296->128 (18) 14.40 -> 13.58, 512->256 (16) 20.62 -> 19.56.
+    // A reduction with several taps does not: 512->64 3x3 (64) 146.6 -> 141.1.
+    if (a.pointwise && (two + 255) / 256 == 4 && a.x_bytes > (18u << 20)) return false;
     const bool short_way = (a.pointwise && a.nchunks <= 16) || a.sw > 1;
     const unsigned percent = table ? (lds_bytes * 4 > 160 * 1024 ? 145 : 170) : short_way ? 160 : a.pointwise ? 178 : 182;
     return (uint64_t)((two + 255) / 256) * percent < (uint64_t)((one + 255) / 256) * 100;

@@ -54,6 +54,8 @@ def alone(c, k, h, w, r=1, stride=1):
     # ... of one or two chunks per wave, and a stride
     (alone(64, 64, 192, 64), 768, ONE), (alone(64, 64, 288, 64), 1152, TWO), (alone(128, 64, 400, 64), 1600, TWO), (alone(136, 64, 288, 64), 1152, ONE),
     (alone(64, 64, 576, 128, 3, 2), 1152, TWO),
+    # ... whose fourth workgroup per compute unit would run alone, with inputs of 47 and 16 MB; with others beside it; several taps
+    (alone(768, 128, 76, 203), 1932, ONE), (alone(512, 256, 38, 203), 1936, TWO), (alone(768, 128, 101, 203), 2564, TWO), (alone(512, 64, 154, 203, 3), 1954, TWO),
     # the offset table, short and long
     (alone(33, 64, 192, 64, 3), 768, ONE), (alone(33, 64, 288, 64, 3), 1152, ONE), (alone(33, 64, 400, 64, 3), 1600, TWO),
     (alone(1001, 64, 192, 64, 3), 768, TWO), (alone(516, 64, 288, 64, 5), 1152, TWO),
