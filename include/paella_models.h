@@ -104,6 +104,9 @@ int paella_exec_bind_input(paella_exec* e, void* device_visible);
 int paella_exec_bind_output(paella_exec* e, void* device_visible);
 /* Issues stage i on `stream`; notifier may be NULL. */
 int paella_exec_launch_stage(paella_exec* e, int stage, void* stream, uint32_t job_id, void* notifier);
+/* Issues stages first..last in order, the last of which reports to `notifier` (which may be NULL).  `stream` keeps them in order.  A small conv and the
+ * pooling stage behind it may share a launch; the conv's own output is then not written. */
+int paella_exec_launch_stages(paella_exec* e, int first, int last, void* stream, uint32_t job_id, void* notifier);
 /* All stages back to back on one stream, un-instrumented (plain single-stream serving). */
 int paella_exec_forward(paella_exec* e, void* stream);
 

@@ -233,6 +233,13 @@ int paella_pool2d_dims(const paella_pool_desc* d, paella_launch_dims* dims);
 int paella_pool2d_launch(const paella_pool_desc* d, const float* x, float* y,
                          void* stream, uint32_t job_id, void* notifier);
 
+/* A small conv and the maximum pooling behind it as ONE launch that reports to nobody; the conv's own output is not written.  Same bits as the two
+ * operators.  Where paella_conv2d_plan_takes_pool() returns 1: windows side by side (stride = window of at most 4 x 4, no padding, the pool's
+ * input the conv's output), a reduction that is not split and short, few tiles; PAELLA_ENOSUP, with nothing launched, otherwise.  x and y must not overlap. */
+int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* pool);
+int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const paella_pool_desc* pool, const float* x, const void* blob_dev, const float* bias,
+                                const float* slope, float* y, void* stream);
+
 /* Up to three such convs (tap-major plans: C a multiple of 8) and one pooling operator in ONE launch: the conv
  * problems' workgroups followed by the pool's, one output element per thread.  An inception module starts with
  * three 1x1 convs and a 3x3 pool that all read the module's input; alone the pool is a launch shorter than the cost of

@@ -902,6 +902,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void conv_small_pre_kernel(SmallP
     }
 }
 
+#include "conv_pool.h"
+
 // A conv that applies a per-channel transform to its input on the way (smallest tile, tap-major order).
 struct ConvPreArgs {
     ConvArgs conv;
@@ -1911,6 +1913,7 @@ struct PackList {
 // A job's whole ordered launch sequence (a model of small kernels is one scheduler stage), recorded between
 // paella_pack_sequence_begin and _end: the sequences of several requests of one model go out position by position, the
 // k-th launches of all of them in one grid, on one queue with the barrier bit set.
+constexpr unsigned kSeqConvPool = 4;  // beside the kinds of members of a group launch
 struct SeqRecord {
     unsigned kind = kMemberConv;
     int kw = 4, k_order = 1;   // conv: the kernel variant; pool and dense ride in the <4, tap-major> variant, whose 256-thread
@@ -1918,6 +1921,7 @@ struct SeqRecord {
     unsigned dyn_lds = 0;
     unsigned units = 0;        // conv: workgroups; pool: output elements; dense: output rows
     GroupMember m;
+    ConvPoolArgs cp;           // kSeqConvPool
 };
 
 struct Sequence {
@@ -2142,6 +2146,19 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
     return failed ? -1 : launches;
 }
 
+// n problems of one shape as one launch.
+int launch_conv_pool(const ConvPoolGroupArgs& g, int n, int kw, void* stream) {
+    const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const dim3 block(64u * (unsigned)kw);
+    if (n == 1) {
+        paella::launch(kw == 2 ? conv_pool_kernel<2> : kw == 4 ? conv_pool_kernel<4> : conv_pool_kernel<8>, dim3(g.grid), block, 0, st, g.m[0]);
+    } else {
+        paella::launch_used(kw == 2 ? conv_pool_group_kernel<2> : kw == 4 ? conv_pool_group_kernel<4> : conv_pool_group_kernel<8>, dim3(g.grid * (unsigned)n), block, 0, st,
+                            offsetof(ConvPoolGroupArgs, m) + (size_t)n * sizeof(ConvPoolArgs), g);
+    }
+    return (int)hipGetLastError();
+}
+
 unsigned units_to_grid(const SeqRecord& r) {
     if (r.kind == kMemberPool) return (r.units + 255u) / 256u;  // one element per thread
     if (r.kind == kMemberDense) return (r.units + 3u) / 4u;     // one row per wave
@@ -2151,6 +2168,15 @@ unsigned units_to_grid(const SeqRecord& r) {
 // The k-th launches of seqs[first .. first + n) as one grid on `queue`; a member with a notifier reports its own workgroups.
 int seq_launch_position(const std::vector<Sequence>& seqs, size_t first, int n, size_t k, void* queue) {
     const SeqRecord& head = seqs[first].recs[k];
+    if (head.kind == kSeqConvPool) {
+        ConvPoolGroupArgs g;
+        g.grid = head.units;
+        g.div_grid = fast_div(head.units);
+        for (int i = 0; i < n; ++i) g.m[i] = seqs[first + (size_t)i].recs[k].cp;
+        g_pack_launches.fetch_add(1, std::memory_order_relaxed);
+        g_pack_members.fetch_add((uint64_t)n, std::memory_order_relaxed);
+        return launch_conv_pool(g, n, head.kw, queue);
+    }
     ConvGroupArgs g;
     g.kinds = 0;
     unsigned grid = 0, dyn_lds = 0;
@@ -2222,7 +2248,9 @@ int seq_send(SeqList& list, bool only_full) {
 bool same_signature(const Sequence& a, const Sequence& b) {
     if (a.recs.size() != b.recs.size()) return false;
     for (size_t k = 0; k < a.recs.size(); ++k)
-        if (a.recs[k].kind != b.recs[k].kind || a.recs[k].kw != b.recs[k].kw || a.recs[k].k_order != b.recs[k].k_order) return false;
+        if (a.recs[k].kind != b.recs[k].kind || a.recs[k].kw != b.recs[k].kw || a.recs[k].k_order != b.recs[k].k_order ||
+            (a.recs[k].kind == kSeqConvPool && a.recs[k].units != b.recs[k].units))
+            return false;
     return true;
 }
 
@@ -2873,4 +2901,62 @@ extern "C" int paella_conv_kernel_vgprs(int kind, int mi, int ni, int kw, unsign
     if (e != hipSuccess) return (int)e;
     *vgprs = (unsigned)attr.numRegs;
     return 0;
+}
+
+// ---- A conv and its pool (conv_pool.h)
+
+extern "C" int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* d) {
+    if (!plan || !d || plan->kind != 0 || plan->mi != 1 || plan->ni != 1 || plan->depth || plan->pair_taps || plan->splits != 1 || plan->small != 1 || !plan->fast_div) return 0;
+    if (plan->kw != 2 && plan->kw != 4 && plan->kw != 8) return 0;
+    if (d->is_avg || d->pad_h || d->pad_w || d->ceil_mode || d->stride_h != d->R || d->stride_w != d->S || d->C != plan->d.K || d->H != plan->P || d->W != plan->Q) return 0;
+    if (d->R > 4 || d->S > 4) return 0;
+    const int area = d->R * d->S, P = d->H / d->R, Q = d->W / d->S;
+    if (area < 2 || P < 1 || Q < 1) return 0;
+    // Half of the columns at work, one workgroup per compute unit and a short reduction: beyond, the two launches gain from larger tiles what
+    // they lose on the way.
+    const int wins = 16 / area;
+    const long tiles = (((long)P * Q + wins - 1) / wins) * ((plan->d.K + 15) / 16);
+    const int nchunks = plan->k_pad / 8;
+    return wins * area >= 8 && tiles <= 256 && (nchunks + plan->kw - 1) / plan->kw <= 8 ? 1 : 0;
+}
+
+extern "C" int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const paella_pool_desc* d, const float* x, const void* blob_dev, const float* bias,
+                                           const float* slope, float* y, void* stream) {
+    if (!plan || !d || !x || !blob_dev || !y) return PAELLA_EINVAL;
+    if (!paella_conv2d_plan_takes_pool(plan, d)) return PAELLA_ENOSUP;
+    ConvArgs a;
+    if (int rc = fill_args(plan, x, blob_dev, bias, nullptr, slope, y, nullptr, 0, nullptr, a)) return rc;
+    if (!a.fast_div) return PAELLA_ENOSUP;
+    ConvPoolGroupArgs g;
+    ConvPoolArgs& c = g.m[0];
+    c.x = a.x; c.wpk = reinterpret_cast<const float*>(blob_dev); c.bias = bias; c.slope = slope; c.y = y;
+    c.H = a.H; c.W = a.W; c.HW = a.H * a.W;
+    c.K = a.K; c.m_pad = a.m_pad; c.nchunks = a.nchunks; c.kdim = a.kdim; c.k_order = plan->k_order; c.CB = a.CB; c.RS = a.RS; c.S = a.S;
+    c.sh = a.sh; c.sw = a.sw; c.ph = a.ph; c.pw = a.pw; c.dh = a.dh; c.dw = a.dw;
+    c.chunks_per_wave = (a.nchunks + plan->kw - 1) / plan->kw;
+    c.pool_r = d->R; c.pool_s = d->S; c.area = d->R * d->S;
+    c.wins = 16 / c.area;
+    c.out_q = d->W / d->S;
+    c.out_n = d->H / d->R * c.out_q;
+    c.n_tiles_n = (c.out_n + c.wins - 1) / c.wins;
+    c.n_tiles_m = (a.K + 15) / 16;
+    c.x_bytes = a.x_bytes; c.w_bytes = a.w_bytes;
+    c.act = a.act; c.lo = a.lo; c.hi = a.hi;
+    // (dividends: columns below 16, windows and tiles of a launch of 256 tiles at most, reduction indices)
+    c.div_area = fast_div((unsigned)c.area); c.div_pool_s = fast_div((unsigned)c.pool_s); c.div_out_q = fast_div((unsigned)c.out_q);
+    c.div_rs = fast_div((unsigned)c.RS); c.div_s = a.div_s; c.div_cb = a.div_cb; c.div_n = fast_div((unsigned)c.n_tiles_n);
+    if (((uint64_t)c.nchunks * 8 + 64) * (uint64_t)c.RS >= ((uint64_t)1 << 32)) return PAELLA_ENOSUP;
+    g.grid = (unsigned)(c.n_tiles_n * c.n_tiles_m);
+    g.div_grid = fast_div(g.grid);
+    if (paella::g_pack_recording && stream == g_pack.rec_queue) {
+        SeqRecord r;
+        r.kind = kSeqConvPool;
+        r.kw = plan->kw;
+        r.k_order = plan->k_order;
+        r.units = g.grid;
+        r.cp = c;
+        g_pack.rec.recs.push_back(r);
+        return 0;
+    }
+    return launch_conv_pool(g, 1, plan->kw, stream);
 }

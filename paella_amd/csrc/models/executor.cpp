@@ -46,6 +46,7 @@ struct Launch {
     int pre = -1;  // count == 1: the scale-shift node whose work the conv nodes[0] does on its input, if any
     int pool = -1;  // a pooling node that shares the launch with the convs (at most three then), or -1
     paella_launch_dims dims{};
+    bool pooled = false;  // a conv whose output only the next stage reads, a pool: the two may go out as one launch
 };
 
 struct paella_model {
@@ -321,6 +322,29 @@ void pair_up(paella_model* m) {
     }
 }
 
+// Marks the convs that may go out together with the pooling stage behind them (hip/conv_pool.h).  The conv's output is not written then, so that nobody
+// else may read it; and the pool's output is written while other workgroups still read the conv's input.
+void mark_pooled(paella_model* m) {
+    const Graph& g = m->g;
+    auto overlap = [&](const View& a, const View& b) {
+        if (a.buf < 0 || b.buf < 0) return false;
+        const size_t a0 = g.buffers[a.buf].offset + a.off, b0 = g.buffers[b.buf].offset + b.off;
+        return a0 < b0 + b.numel() && b0 < a0 + a.numel();
+    };
+    for (size_t s = 0; m->pairing && s + 1 < m->stages.size(); ++s) {
+        const Launch &lc = m->stages[s], &lp = m->stages[s + 1];
+        if (lc.count != 1 || lc.pool >= 0 || lp.count != 1 || lp.pool >= 0 || m->pre_of[lc.nodes[0]] >= 0) continue;
+        const Node &c = g.nodes[lc.nodes[0]], &p = g.nodes[lp.nodes[0]];
+        if (c.op != Op::Conv || p.op != Op::Pool || c.x2.buf >= 0 || !paella_conv2d_plan_takes_pool(&m->plans[lc.nodes[0]].conv, &p.pool)) continue;
+        const View &v = c.y, &x = p.x;
+        if (v.buf != x.buf || v.off != x.off || v.C != x.C || v.H != x.H || v.W != x.W) continue;
+        bool ok = !overlap(v, g.output) && !overlap(p.y, c.x) && !overlap(p.y, v) && c.x.buf != g.output.buf;
+        for (const Node& n : g.nodes)
+            if (&n != &p && (overlap(n.x, v) || overlap(n.x2, v))) ok = false;
+        m->stages[s].pooled = ok;
+    }
+}
+
 // Plans every node and lays out the weight arena (host arithmetic only).
 int plan_nodes(paella_model* m, std::vector<size_t>& tensor_off, std::vector<size_t>& blob_off, size_t& total) {
     const Graph& g = m->g;
@@ -402,6 +426,7 @@ int build(paella_model* m) {
     if (int rc = plan_nodes(m, tensor_off, blob_off, total)) return rc;
     absorb_scale_shifts(m);
     pair_up(m);
+    mark_pooled(m);
 
     // Generate, pack, upload.
     std::vector<char> host(total, 0);
@@ -751,11 +776,25 @@ int paella_exec_launch_stage(paella_exec* e, int stage, void* stream, uint32_t j
     return PAELLA_EINVAL;
 }
 
-static int launch_all(paella_exec* e, void* stream) {
-    for (size_t i = 0; i < e->m->stages.size(); ++i)
-        if (int rc = paella_exec_launch_stage(e, (int)i, stream, 0, nullptr)) return rc;
+int paella_exec_launch_stages(paella_exec* e, int first, int last, void* stream, uint32_t job_id, void* notifier) {
+    if (!e || first < 0 || last < first || (size_t)last >= e->m->stages.size()) return PAELLA_EINVAL;
+    for (int i = first; i <= last; ++i) {
+        if (e->m->stages[i].pooled && i < last && (i + 1 < last || !notifier)) {
+            const StagePlan& st = e->m->plans[e->m->stages[i].nodes[0]];
+            const Node &c = *st.node, &p = e->m->g.nodes[e->m->stages[i + 1].nodes[0]];
+            const int rc = paella_conv2d_launch_pooled(&st.conv, &p.pool, e->ptr(c.x), st.w, st.bias, st.slope, e->ptr(p.y), stream);
+            if (rc == 0) ++i;
+            if (rc != PAELLA_ENOSUP) {
+                if (rc) return rc;
+                continue;
+            }
+        }
+        if (int rc = paella_exec_launch_stage(e, i, stream, i == last ? job_id : 0, i == last ? notifier : nullptr)) return rc;
+    }
     return 0;
 }
+
+static int launch_all(paella_exec* e, void* stream) { return paella_exec_launch_stages(e, 0, (int)e->m->stages.size() - 1, stream, 0, nullptr); }
 
 int paella_exec_forward(paella_exec* e, void* stream) {
     if (!e) return PAELLA_EINVAL;

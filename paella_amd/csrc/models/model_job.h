@@ -247,10 +247,7 @@ class ModelJob : public llis::job::CoroutineJob {
             if (direct_ && last > s) paella_direct_queue_set_ordered(target, 1);
             // ... and the whole group is recorded, to go out together with the same group of other requests of this model
             const bool recording = pack_ && last > s && !group && paella_pack_sequence_begin(model_, target) == 0;
-            for (int k = s; k <= last; ++k) {
-                if (k < last) check(paella_exec_launch_stage(exec_, k, target, 0, nullptr), "stage launch");
-                else check(paella_exec_launch_stage(exec_, k, target, id, get_finished_block_notifier()), "stage launch");
-            }
+            check(paella_exec_launch_stages(exec_, s, last, target, id, get_finished_block_notifier()), "stage launch");
             if (recording) check(paella_pack_sequence_end(), "end of the recorded launch sequence");
             if (direct_ && last > s) paella_direct_queue_set_ordered(target, 0);
             s = last + 1;
