@@ -8,7 +8,9 @@
 // is taken across a wave's lanes and the conv's output is never written.  The launch is one workgroup per 16 channels and tile of windows, with the waves
 // and the chunks per wave of the conv's own plan: the bits are those of the conv's kernel and the pool's.
 // The small CNN (28x28, 5x5 convs of 8 and 16 channels, pools 2x2 and 3x3), five launches -> three: one request without a server 27.9 -> 24.1 us, a lone
-// client of the server 25.4 -> 19.8 us a request, 9 : 1 beside Inception-v3 under load 163.1 -> 159.7 ms.
+// client of the server 25.4 -> 19.8 us a request, 9 : 1 beside Inception-v3 under load 163.1 -> 159.7 ms.  What such a kernel takes is the chain of trips
+// in it: with the arguments in one round instead of six, bias and slope requested with the operands instead of behind the sum, no address arithmetic for
+// chunks that are not there and the two reduction orders apart 24.1 -> 23.1 and 19.8 -> 18.7 us.
 
 struct ConvPoolArgs {
     const float* x;
@@ -32,6 +34,15 @@ struct ConvPoolArgs {
 
 template <int KW>
 __device__ __forceinline__ void conv_pool_tile(const ConvPoolArgs& p, const unsigned bid) {
+    // The arguments requested together (see conv_tile): read where they are used they are six trips to the scalar cache, one behind the other.
+    {
+        const unsigned long long x = (unsigned long long)p.x, w = (unsigned long long)p.wpk, b = (unsigned long long)p.bias, l = (unsigned long long)p.slope;
+        asm volatile("" ::"s"(x), "s"(w), "s"(b), "s"(l), "s"(p.H), "s"(p.W), "s"(p.HW), "s"(p.K), "s"(p.m_pad), "s"(p.nchunks), "s"(p.kdim), "s"(p.k_order), "s"(p.CB), "s"(p.RS), "s"(p.S),
+                     "s"(p.chunks_per_wave), "s"(p.area), "s"(p.wins), "s"(p.n_tiles_n), "s"(p.n_tiles_m), "s"(p.x_bytes), "s"(p.w_bytes), "s"(p.act));
+        asm volatile("" ::"s"(p.sh), "s"(p.sw), "s"(p.ph), "s"(p.pw), "s"(p.dh), "s"(p.dw), "s"(p.pool_r), "s"(p.pool_s), "s"(p.out_q), "s"(p.out_n), "s"(p.div_area.mul),
+                     "s"(p.div_area.one), "s"(p.div_pool_s.mul), "s"(p.div_pool_s.one), "s"(p.div_out_q.mul), "s"(p.div_out_q.one), "s"(p.div_rs.mul), "s"(p.div_rs.one),
+                     "s"(p.div_s.mul), "s"(p.div_s.one), "s"(p.div_cb.mul), "s"(p.div_cb.one), "s"(p.div_n.mul), "s"(p.div_n.one));
+    }
     if (bid >= (unsigned)(p.n_tiles_n * p.n_tiles_m)) return;
     __shared__ float red[KW][4][64];
     const int lane = threadIdx.x & 63;
@@ -50,22 +61,33 @@ __device__ __forceinline__ void conv_pool_tile(const ConvPoolArgs& p, const unsi
     auto rsrc = [](const void* q, unsigned len) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(q), 0, q ? len : 0u, 0x00027000); };
     auto word = [](const __amdgpu_buffer_rsrc_t r, int off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0)); };
 
+    // What the end needs, requested with the operands.
+    constexpr int PER = KW < 4 ? 4 / KW : 1;
+    float bias_v[PER], slope_v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int chan = m0 + 4 * kk + ((wave + i * KW) & 3);
+        bias_v[i] = word(rsrc(p.bias, (unsigned)p.K * 4u), chan * 4);
+        slope_v[i] = word(rsrc(p.slope, p.act == PAELLA_ACT_PRELU ? (unsigned)p.K * 4u : 0u), chan * 4);
+    }
+
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     const int begin = wave * p.chunks_per_wave, end = min(p.nchunks, begin + p.chunks_per_wave);
-    constexpr int B = 4;  // chunks under way together
-    for (int c0 = begin; c0 < end; c0 += B) {
+    auto batch = [&](auto count, auto tap_major, int c0) {  // chunks under way together
+        constexpr int B = decltype(count)::value;
+        constexpr bool TM = decltype(tap_major)::value;
         float a[B][2], b[B][2];
 #pragma unroll
         for (int u = 0; u < B; ++u) {
             const int c = c0 + u;
             const bool live = c < end;
-            const int tap = p.k_order ? (int)quot_fast((unsigned)c, p.div_cb) : 0;
+            const int tap = TM ? (int)quot_fast((unsigned)c, p.div_cb) : 0;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int kl = 4 * (kk & 1) + (kk >> 1) + 2 * i;  // of the chunk's eight, in the order of the 32 x 32 instruction (conv_small.h)
                 int chan, rs;
                 bool ok = valid & live;
-                if (p.k_order) {
+                if (TM) {
                     chan = (c - tap * p.CB) * 8 + kl;
                     rs = tap;
                 } else {
@@ -86,21 +108,33 @@ __device__ __forceinline__ void conv_pool_tile(const ConvPoolArgs& p, const unsi
             if (c0 + u < end)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[u][i], acc, 0, 0, 0);
-    }
+    };
+    auto chunks = [&](auto tap_major) {
+        if (p.chunks_per_wave == 1) {  // (a first layer: the addresses of chunks that are not there take as long as a trip to memory)
+            if (begin < end) batch(std::integral_constant<int, 1>{}, tap_major, begin);
+        } else {
+            for (int c0 = begin; c0 < end; c0 += 4) batch(std::integral_constant<int, 4>{}, tap_major, c0);
+        }
+    };
+    if (p.k_order) chunks(std::true_type{});
+    else chunks(std::false_type{});
 #pragma unroll
     for (int e = 0; e < 4; ++e) red[wave][e][lane] = acc[e];
     __syncthreads();
     // Register e of the tile holds, in lane (j, kk), channel m0 + 4 * kk + e at column j; a wave finishes one of them, or two of two waves.
-    for (int e = wave; e < 4; e += KW) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = wave + i * KW;
+        if (e >= 4) break;
         float v = red[0][e][lane];  // wave order, as in conv_tile
 #pragma unroll
         for (int w = 1; w < KW; ++w) v += red[w][e][lane];
         const int chan = m0 + 4 * kk + e;
-        v += word(rsrc(p.bias, (unsigned)p.K * 4u), chan * 4);
+        v += bias_v[i];
         float none = 0.f;  // where conv_tile adds a residual that is not there: -0 becomes +0
         asm volatile("" : "+v"(none));
         v += none;
-        v = apply_act(v, p.act, p.act == PAELLA_ACT_PRELU ? word(rsrc(p.slope, (unsigned)p.K * 4u), chan * 4) : 0.f, p.lo, p.hi);
+        v = apply_act(v, p.act, slope_v[i], p.lo, p.hi);
         const int first = (lane & 48) + wi * p.area;
         float m = -FLT_MAX;  // in the order of pool_window
         if (p.area == 4) {
