@@ -2908,6 +2908,8 @@ extern "C" int paella_conv_kernel_vgprs(int kind, int mi, int ni, int kw, unsign
 extern "C" int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* d) {
     if (!plan || !d || plan->kind != 0 || plan->mi != 1 || plan->ni != 1 || plan->depth || plan->pair_taps || plan->splits != 1 || plan->small != 1 || !plan->fast_div) return 0;
     if (plan->kw != 2 && plan->kw != 4 && plan->kw != 8) return 0;
+    paella::PoolArgs pa;  // what the pool's own launch would refuse is refused here too
+    if (!paella::pool_fill_args(d, nullptr, nullptr, 0, nullptr, &pa)) return 0;
     if (d->is_avg || d->pad_h || d->pad_w || d->ceil_mode || d->stride_h != d->R || d->stride_w != d->S || d->C != plan->d.K || d->H != plan->P || d->W != plan->Q) return 0;
     if (d->R > 4 || d->S > 4) return 0;
     const int area = d->R * d->S, P = d->H / d->R, Q = d->W / d->S;
