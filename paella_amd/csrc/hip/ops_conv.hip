@@ -2948,6 +2948,9 @@ extern "C" int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const p
     c.div_area = fast_div((unsigned)c.area); c.div_pool_s = fast_div((unsigned)c.pool_s); c.div_out_q = fast_div((unsigned)c.out_q);
     c.div_rs = fast_div((unsigned)c.RS); c.div_s = a.div_s; c.div_cb = a.div_cb; c.div_n = fast_div((unsigned)c.n_tiles_n);
     if (((uint64_t)c.nchunks * 8 + 64) * (uint64_t)c.RS >= ((uint64_t)1 << 32)) return PAELLA_ENOSUP;
+    // Workgroups that are done write while others still read.
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    if (x0 < y0 + (size_t)a.K * c.out_n * sizeof(float) && y0 < x0 + a.x_bytes) return PAELLA_ENOSUP;
     g.grid = (unsigned)(c.n_tiles_n * c.n_tiles_m);
     g.div_grid = fast_div(g.grid);
     if (paella::g_pack_recording && stream == g_pack.rec_queue) {

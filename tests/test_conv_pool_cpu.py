@@ -48,3 +48,14 @@ def test_a_pool_that_is_none_is_refused(window):
     assert lib.paella_conv2d_plan_takes_pool(ctypes.byref(plan), ctypes.byref(d)) == 0
     assert lib.paella_conv2d_launch_pooled(ctypes.byref(plan), ctypes.byref(d), memory, memory, None, None, ctypes.c_void_p(1 << 20), None) == -2
     assert lib.paella_pool2d_dims(ctypes.byref(d), ctypes.byref(_abi.LaunchDims())) != 0
+
+
+@pytest.mark.parametrize("x, y", [(1 << 20, 1 << 20), (1 << 20, (1 << 20) + 8 * 14 * 14 * 4 - 4), ((1 << 20) + 16 * 4 * 4 * 4 - 4, 1 << 20)])
+def test_an_output_that_lies_in_the_input_is_refused(x, y):
+    """Workgroups that have their windows write while others still read: two launches can do that, one cannot."""
+    from paella_amd import _abi
+    plan = conv_plan(8, 16, 14, 14, 5)
+    d = _abi.PoolDesc(16, 14, 14, 3, 3, 3, 3, 0, 0, 0, 0, 1)
+    ptr = ctypes.c_void_p
+    assert _abi.ops().paella_conv2d_plan_takes_pool(ctypes.byref(plan), ctypes.byref(d)) == 1
+    assert _abi.ops().paella_conv2d_launch_pooled(ctypes.byref(plan), ctypes.byref(d), ptr(x), ptr(4096), None, None, ptr(y), None) == -2

@@ -63,3 +63,31 @@ def test_values_that_are_no_numbers_take_the_way_of_the_two_operators(cuda):
     x = torch.tensor(x, device=cuda)
     got, want = pooled(ops, conv, x, (3, 3)), ops.pool2d(conv(x), 3, 3)
     assert torch.equal(got.view(torch.int32), want.view(torch.int32)) and not torch.isfinite(want).all()
+
+
+def small_file(path):
+    """A conv of 8 channels on 28 x 28 and its pool as a file of their own."""
+    import _onnx_writer as ow
+    b = ow.Builder(np.random.default_rng(3))
+    y = b.op("Relu", [b.op("Conv", ["x", b.const(b.randn(8, 1, 5, 5, scale=0.2)), b.const(b.randn(8))], kernel_shape=[5, 5], pads=[2, 2, 2, 2])])
+    y = b.op("MaxPool", [y], kernel_shape=[2, 2], strides=[2, 2])
+    b.save(str(path), [("x", [1, 1, 28, 28])], [(y, [1, 8, 14, 14])])
+    return "onnx:" + str(path)
+
+
+def test_input_and_output_in_the_same_memory(cuda, tmp_path):
+    """Bound to the same memory the two stay two launches: the pool writes over what the conv has read."""
+    from paella_amd import models
+    ex = models.Exec(small_file(tmp_path / "inplace.onnx"))
+    x = torch.tensor(np.random.default_rng(6).standard_normal(784).astype(np.float32), device=cuda)
+    apart, same = torch.zeros(1568, device=cuda), torch.zeros(1568, device=cuda)
+    ex.bind_io(x.data_ptr(), apart.data_ptr())
+    ex.forward()
+    ex.bind_io(same.data_ptr(), same.data_ptr())
+    for _ in range(3):
+        same[:784] = x
+        torch.cuda.synchronize()
+        ex.forward()
+        torch.cuda.synchronize()
+        assert torch.equal(same, apart)
+    ex.close()
