@@ -74,6 +74,9 @@ int paella_model_num_stages(const paella_model* m);
 int paella_model_stage_nodes(const paella_model* m, int stage, int* nodes, int capacity);
 /* Launch shape of stage i in the scheduler's units (vgprs read from the loaded code object). */
 int paella_model_stage_dims(const paella_model* m, int stage, paella_launch_dims* dims);
+/* Launch shape of stage i, a small conv, and the pooling stage behind it where paella_exec_launch_stages issues the two as one: it has workgroups of
+ * its own, which can be more than either stage's.  PAELLA_ENOSUP where it never does. */
+int paella_model_pooled_dims(const paella_model* m, int stage, paella_launch_dims* dims);
 /* Operator name ("conv", "dwconv", "dense", "pool", "gap", "eltwise", "softmax", "lrn") and algorithmic work of stage i
  * (of both convs for a pair). */
 int paella_model_stage_work(const paella_model* m, int stage, const char** op, double* flops, double* bytes);

@@ -237,6 +237,8 @@ int paella_pool2d_launch(const paella_pool_desc* d, const float* x, float* y,
  * operators.  Where paella_conv2d_plan_takes_pool() returns 1: windows side by side (stride = window of at most 4 x 4, no padding, the pool's
  * input the conv's output), a reduction that is not split and short, few tiles; PAELLA_ENOSUP, with nothing launched, otherwise and where x and y overlap. */
 int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* pool);
+/* Launch shape of the two as one launch, which has workgroups of its own; PAELLA_ENOSUP where they stay two. */
+int paella_conv2d_pooled_dims(const paella_conv_plan* plan, const paella_pool_desc* pool, paella_launch_dims* dims);
 int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const paella_pool_desc* pool, const float* x, const void* blob_dev, const float* bias,
                                 const float* slope, float* y, void* stream);
 

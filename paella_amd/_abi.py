@@ -98,6 +98,7 @@ OPS_SYMBOLS = {
     "paella_dense_launch": (c_int, [c_void_p] * 4 + [c_int] * 3 + _TAIL),
     "paella_pool_out": (c_int, [c_int] * 5),
     "paella_conv2d_plan_takes_pool": (c_int, [ctypes.POINTER(ConvPlan), ctypes.POINTER(PoolDesc)]),
+    "paella_conv2d_pooled_dims": (c_int, [ctypes.POINTER(ConvPlan), ctypes.POINTER(PoolDesc), ctypes.POINTER(LaunchDims)]),
     "paella_conv2d_launch_pooled": (c_int, [ctypes.POINTER(ConvPlan), ctypes.POINTER(PoolDesc)] + [c_void_p] * 6),
     "paella_pool2d_dims": (c_int, [ctypes.POINTER(PoolDesc), ctypes.POINTER(LaunchDims)]),
     "paella_pool2d_launch": (c_int, [ctypes.POINTER(PoolDesc), c_void_p, c_void_p] + _TAIL),

@@ -18,6 +18,7 @@ MODEL_SYMBOLS = {
     "paella_model_num_stages": (c_int, [c_void_p]),
     "paella_model_stage_nodes": (c_int, [c_void_p, c_int, ctypes.POINTER(c_int), c_int]),
     "paella_model_stage_dims": (c_int, [c_void_p, c_int, ctypes.POINTER(LaunchDims)]),
+    "paella_model_pooled_dims": (c_int, [c_void_p, c_int, ctypes.POINTER(LaunchDims)]),
     "paella_model_stage_work": (c_int, [c_void_p, c_int, ctypes.POINTER(c_char_p), _pd, _pd]),
     "paella_exec_create": (c_int, [c_void_p, ctypes.POINTER(c_void_p)]),
     "paella_exec_destroy": (c_int, [c_void_p]),

@@ -2146,12 +2146,15 @@ int pack_send(PackList& list, int kw, int k_order, bool only_full) {
     return failed ? -1 : launches;
 }
 
+typedef void (*ConvPoolKernel)(ConvPoolArgs);
+ConvPoolKernel pick_conv_pool(int kw) { return kw == 2 ? conv_pool_kernel<2> : kw == 4 ? conv_pool_kernel<4> : conv_pool_kernel<8>; }
+
 // n problems of one shape as one launch.
 int launch_conv_pool(const ConvPoolGroupArgs& g, int n, int kw, void* stream) {
     const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const dim3 block(64u * (unsigned)kw);
     if (n == 1) {
-        paella::launch(kw == 2 ? conv_pool_kernel<2> : kw == 4 ? conv_pool_kernel<4> : conv_pool_kernel<8>, dim3(g.grid), block, 0, st, g.m[0]);
+        paella::launch(pick_conv_pool(kw), dim3(g.grid), block, 0, st, g.m[0]);
     } else {
         paella::launch_used(kw == 2 ? conv_pool_group_kernel<2> : kw == 4 ? conv_pool_group_kernel<4> : conv_pool_group_kernel<8>, dim3(g.grid * (unsigned)n), block, 0, st,
                             offsetof(ConvPoolGroupArgs, m) + (size_t)n * sizeof(ConvPoolArgs), g);
@@ -2905,7 +2908,10 @@ extern "C" int paella_conv_kernel_vgprs(int kind, int mi, int ni, int kw, unsign
 
 // ---- A conv and its pool (conv_pool.h)
 
-extern "C" int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* d) {
+namespace {
+
+// Workgroups of the two as one launch, 0 where they stay two.
+unsigned pooled_grid(const paella_conv_plan* plan, const paella_pool_desc* d) {
     if (!plan || !d || plan->kind != 0 || plan->mi != 1 || plan->ni != 1 || plan->depth || plan->pair_taps || plan->splits != 1 || plan->small != 1 || !plan->fast_div) return 0;
     if (plan->kw != 2 && plan->kw != 4 && plan->kw != 8) return 0;
     paella::PoolArgs pa;  // what the pool's own launch would refuse is refused here too
@@ -2919,7 +2925,23 @@ extern "C" int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const
     const int wins = 16 / area;
     const long tiles = (((long)P * Q + wins - 1) / wins) * ((plan->d.K + 15) / 16);
     const int nchunks = plan->k_pad / 8;
-    return wins * area >= 8 && tiles <= 256 && (nchunks + plan->kw - 1) / plan->kw <= 8 ? 1 : 0;
+    return wins * area >= 8 && tiles <= 256 && (nchunks + plan->kw - 1) / plan->kw <= 8 ? (unsigned)tiles : 0u;
+}
+
+}  // namespace
+
+extern "C" int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* d) { return pooled_grid(plan, d) ? 1 : 0; }
+
+extern "C" int paella_conv2d_pooled_dims(const paella_conv_plan* plan, const paella_pool_desc* d, paella_launch_dims* dims) {
+    if (!plan || !d || !dims) return PAELLA_EINVAL;
+    const unsigned grid = pooled_grid(plan, d);
+    if (!grid) return PAELLA_ENOSUP;
+    *dims = {};
+    dims->grid = grid;
+    dims->block = 64u * (unsigned)plan->kw;
+    dims->vgprs = 128;
+    add_kernel_resources(reinterpret_cast<const void*>(pick_conv_pool(plan->kw)), dims);
+    return 0;
 }
 
 extern "C" int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const paella_pool_desc* d, const float* x, const void* blob_dev, const float* bias,

@@ -47,6 +47,7 @@ struct Launch {
     int pool = -1;  // a pooling node that shares the launch with the convs (at most three then), or -1
     paella_launch_dims dims{};
     bool pooled = false;  // a conv whose output only the next stage reads, a pool: the two may go out as one launch
+    paella_launch_dims pooled_dims{};  // ... of these
 };
 
 struct paella_model {
@@ -341,7 +342,7 @@ void mark_pooled(paella_model* m) {
         bool ok = !overlap(v, g.output) && !overlap(p.y, c.x) && !overlap(p.y, v) && c.x.buf != g.output.buf;
         for (const Node& n : g.nodes)
             if (&n != &p && (overlap(n.x, v) || overlap(n.x2, v))) ok = false;
-        m->stages[s].pooled = ok;
+        m->stages[s].pooled = ok && paella_conv2d_pooled_dims(&m->plans[lc.nodes[0]].conv, &p.pool, &m->stages[s].pooled_dims) == 0;
     }
 }
 
@@ -577,6 +578,13 @@ int paella_model_num_stages(const paella_model* m) { return m ? (int)m->stages.s
 int paella_model_stage_dims(const paella_model* m, int stage, paella_launch_dims* dims) {
     if (!m || !dims || stage < 0 || (size_t)stage >= m->stages.size()) return PAELLA_EINVAL;
     *dims = m->stages[stage].dims;
+    return 0;
+}
+
+int paella_model_pooled_dims(const paella_model* m, int stage, paella_launch_dims* dims) {
+    if (!m || !dims || stage < 0 || (size_t)stage >= m->stages.size()) return PAELLA_EINVAL;
+    if (!m->stages[stage].pooled) return PAELLA_ENOSUP;
+    *dims = m->stages[stage].pooled_dims;
     return 0;
 }
 

@@ -14,7 +14,7 @@
 //  * a model whose kernels all have at most PAELLA_GROUP_THREADS work-items (default 65536, an eighth of what the device
 //    holds; 0 = off) is one scheduler stage: its kernels are issued together, in order on one queue, and only the last
 //    one reports to the scheduler.  Scheduling kernel by kernel pays off for kernels that fill the device; for the small
-//    CNN (5 kernels of at most 25 workgroups) each trip through the scheduler costs more than the kernel;
+//    CNN (5 kernels, 3 launches of at most 49 workgroups) each trip through the scheduler costs more than the kernel;
 //  * request buffers in the client's shared-memory pool cannot be registered with the runtime on this
 //    platform, so both copies go through a per-instance pinned staging buffer, unless the host addresses the
 //    device's memory and writes the input there (filled on the server
@@ -93,11 +93,18 @@ class ModelJob : public llis::job::CoroutineJob {
         // because a member that must wait for its predecessor stalls everything behind it in its queue.
         bool all_small = group_limit > 0;
         dims_.resize((size_t)num_stages_);
+        pooled_.resize((size_t)num_stages_);
         for (int s = 0; s < num_stages_; ++s) {
             paella_launch_dims& d = dims_[(size_t)s];
             paella_model_stage_dims(model_, s, &d);
             all_small = all_small && (unsigned long)d.grid * d.block <= group_limit;
+            paella_launch_dims& p = pooled_[(size_t)s];
+            if (paella_model_pooled_dims(model_, s, &p) != 0) p = {};
         }
+        // A conv and its pool as one launch have workgroups of their own (49 for 25 of the small CNN's first conv, up to six times as many
+        // elsewhere), held to the same limit: they go out as two where it does not allow that.
+        apart_.assign((size_t)num_stages_, 0);
+        for (int s = 0; s < num_stages_; ++s) apart_[(size_t)s] = all_small && (unsigned long)pooled_[(size_t)s].grid * pooled_[(size_t)s].block > group_limit;
         group_end_.assign((size_t)num_stages_, 0);
         for (int s = 0; s < num_stages_; ++s) group_end_[(size_t)s] = all_small ? num_stages_ - 1 : s;
         // Kernels go out as AQL packets on the operator library's own queues unless PAELLA_DISPATCH=hip; the
@@ -216,7 +223,7 @@ class ModelJob : public llis::job::CoroutineJob {
             const bool group = uncrowded_stages_ > 1 && last == s && llis::job::Context::is_uncrowded();
             if (group) last = std::min(s + uncrowded_stages_, num_stages_) - 1;
             // Admitted and accounted as its last kernel, or, where no limit bounds the others, as the largest.
-            const paella_launch_dims& d = dims_[(size_t)(group ? largest(s, last) : last)];
+            const paella_launch_dims& d = group ? largest(s, last) : dims_[(size_t)last];
             set_num_blocks(d.grid);
             set_num_threads_per_block(d.block);
             set_smem_size_per_block(d.lds_bytes);
@@ -247,7 +254,10 @@ class ModelJob : public llis::job::CoroutineJob {
             if (direct_ && last > s) paella_direct_queue_set_ordered(target, 1);
             // ... and the whole group is recorded, to go out together with the same group of other requests of this model
             const bool recording = pack_ && last > s && !group && paella_pack_sequence_begin(model_, target) == 0;
-            check(paella_exec_launch_stages(exec_, s, last, target, id, get_finished_block_notifier()), "stage launch");
+            for (int k = s, to; k <= last; k = to + 1) {
+                for (to = k; to < last && !apart_[(size_t)to];) ++to;
+                check(paella_exec_launch_stages(exec_, k, to, target, to == last ? id : 0, to == last ? get_finished_block_notifier() : nullptr), "stage launch");
+            }
             if (recording) check(paella_pack_sequence_end(), "end of the recorded launch sequence");
             if (direct_ && last > s) paella_direct_queue_set_ordered(target, 0);
             s = last + 1;
@@ -283,22 +293,25 @@ class ModelJob : public llis::job::CoroutineJob {
         std::memcpy(staging_, io_ptr, in_bytes_);
     }
 
-    // The kernel of first..last that takes the largest share of the device, by the resource it takes most of.
-    int largest(int first, int last) const {
+    // The launch of first..last that takes the largest share of the device, by the resource it takes most of.
+    const paella_launch_dims& largest(int first, int last) const {
         using R = llis::server::SmResources;
-        int at = last;
+        const paella_launch_dims* at = &dims_[(size_t)last];
         double most = 0;
-        for (int k = first; k <= last; ++k) {
-            const paella_launch_dims& d = dims_[(size_t)k];
+        auto look = [&](const paella_launch_dims& d) {
             const double share = d.grid * std::max({(double)R::wg_threads(d.block) / (R::kSimdsPerCu * R::kMaxWavesPerSimd * R::kWaveLanes),
                                                     (double)R::wg_regs(d.block, d.vgprs) / (R::kSimdsPerCu * R::kVgprsPerSimdLane * R::kWaveLanes),
                                                     (double)R::wg_lds(d.lds_bytes) / (160 * 1024)});
             if (share > most) {
                 most = share;
-                at = k;
+                at = &d;
             }
+        };
+        for (int k = first; k <= last; ++k) {
+            look(dims_[(size_t)k]);
+            if (k + 1 < last) look(pooled_[(size_t)k]);  // (a pool that reports goes out by itself)
         }
-        return at;
+        return *at;
     }
 
     void* stream() { return reinterpret_cast<void*>(get_cuda_stream()); }
@@ -329,6 +342,8 @@ class ModelJob : public llis::job::CoroutineJob {
     void* io_ptr_ = nullptr;
     int num_stages_ = 0;
     std::vector<paella_launch_dims> dims_;  // per kernel
+    std::vector<paella_launch_dims> pooled_;  // per kernel: of it and the pool behind it as one launch, no workgroups where that is never done
+    std::vector<char> apart_;      // per kernel: it goes out by itself in a group, although the pool behind it could be in the same launch
     std::vector<int> group_end_;   // per kernel: index of the last kernel of the group it is issued with
     bool direct_ = true;
     bool whole_job_direct_ = false;

@@ -356,3 +356,13 @@ extern "C" __attribute__((visibility("default"))) int paella_exec_launch_stage(p
     g_needs += " " + std::to_string(d.grid) + "," + std::to_string(d.block) + "," + std::to_string(d.lds_bytes) + "," + std::to_string(d.vgprs);
     return notifier ? fake_hip_kernel_launch(stream, job_id & ~PAELLA_JOB_ID_FLAGS, d.grid) : 0;
 }
+
+// A conv and its pool as one launch: "pooled" in the place of their stages' numbers.
+extern "C" __attribute__((visibility("default"))) int paella_conv2d_launch_pooled(const paella_conv_plan* plan, const paella_pool_desc* pool, const float*, const void*,
+                                                                                  const float*, const float*, float*, void*) {
+    paella_launch_dims d;
+    library<int (*)(const paella_conv_plan*, const paella_pool_desc*, paella_launch_dims*)>("paella_conv2d_pooled_dims")(plan, pool, &d);
+    g_issued += " pooled";
+    g_needs += " " + std::to_string(d.grid) + "," + std::to_string(d.block) + "," + std::to_string(d.lds_bytes) + "," + std::to_string(d.vgprs);
+    return 0;
+}
