@@ -3,6 +3,8 @@
 // prints how often a recording was tried and how many passes were launched kernel by kernel and replayed.
 // `exec_check copies`: host_store, host_settle and host_load (csrc/hip/host_io.h) on host memory, up to the last byte in front of a page that may not
 // be touched; prints the number of lengths checked.
+// `exec_check launches <model> <takes|refuses> [first last notifier]...`: what paella_exec_launch_stages returns and issues for each range: a stage's number, with
+// "*<job id>" where it reports to the notifier, or "pooled" for a conv and its pool as one launch (refuses: as that launch does for operands that overlap).
 
 #include "../../paella_amd/csrc/hip/host_io.h"
 #include "paella_models.h"
@@ -10,12 +12,15 @@
 #include <sys/mman.h>
 
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <string>
 #include <vector>
 
 namespace {
 bool g_refuse = false;
 int g_recorded = 0, g_launches = 0, g_replayed = 0;
+std::string g_issued;
 }  // namespace
 
 namespace paella {
@@ -31,9 +36,32 @@ int forward_graph_replay(void*, void*) {
 void forward_graph_destroy(void*) {}
 }  // namespace paella
 
-extern "C" int paella_exec_launch_stage(paella_exec*, int, void*, uint32_t, void*) {
+extern "C" int paella_exec_launch_stage(paella_exec*, int stage, void*, uint32_t job_id, void* notifier) {
     ++g_launches;
+    g_issued += " " + std::to_string(stage);
+    if (notifier || job_id) g_issued += "*" + std::to_string(job_id);
     return 0;
+}
+
+extern "C" int paella_conv2d_launch_pooled(const paella_conv_plan*, const paella_pool_desc*, const float*, const void*, const float*, const float*, float*, void*) {
+    if (g_refuse) return PAELLA_ENOSUP;
+    g_issued += " pooled";
+    return 0;
+}
+
+static int check_launches(int argc, char** argv) {
+    g_refuse = std::strcmp(argv[3], "refuses") == 0;
+    paella_model* m = nullptr;
+    paella_exec* e = nullptr;
+    if (paella_model_get(argv[2], 1, &m) || paella_exec_create(m, &e)) return 1;
+    char notifier;
+    for (int i = 4; i + 2 < argc; i += 3) {
+        const bool reports = std::atoi(argv[i + 2]) != 0;
+        const int rc = paella_exec_launch_stages(e, std::atoi(argv[i]), std::atoi(argv[i + 1]), nullptr, reports ? 7 : 0, reports ? &notifier : nullptr);
+        std::printf("%d%s\n", rc, g_issued.c_str());
+        g_issued.clear();
+    }
+    return paella_exec_destroy(e);
 }
 
 static int check_copies() {
@@ -64,6 +92,7 @@ static int check_copies() {
 
 int main(int argc, char** argv) {
     if (argc > 1 && std::strcmp(argv[1], "copies") == 0) return check_copies();
+    if (argc > 3 && std::strcmp(argv[1], "launches") == 0) return check_launches(argc, argv);
     g_refuse = argc > 1 && std::strcmp(argv[1], "refuse") == 0;
     paella_model* m = nullptr;
     paella_exec* e[2] = {nullptr, nullptr};
