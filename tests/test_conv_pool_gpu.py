@@ -30,7 +30,7 @@ def make(case, rng, ops, act, bias=True):
     return ops.Conv2d(wt, rng.standard_normal(k).astype(np.float32) if bias else None, stride=stride, pad=pad, dil=dil, act=act, slope=slope, in_hw=(h, w), tile_hint=hint)
 
 
-def pooled(ops, conv, x, window):
+def pooled(ops, conv, x, window, stream=None):
     from paella_amd import _abi
     plan = conv.plan
     d = _abi.PoolDesc(plan.d.K, plan.P, plan.Q, *window, *window, 0, 0, 0, 0, 1)
@@ -38,7 +38,7 @@ def pooled(ops, conv, x, window):
     y = torch.full((1, plan.d.K, plan.P // window[0], plan.Q // window[1]), 7.25, device=x.device)
     ptr = lambda t: None if t is None else t.data_ptr()
     _abi.check(_abi.ops().paella_conv2d_launch_pooled(ctypes.byref(plan), ctypes.byref(d), ptr(x), ptr(conv.blob), ptr(conv.bias), ptr(conv.slope), ptr(y),
-                                                      torch.cuda.current_stream().cuda_stream), "paella_conv2d_launch_pooled")
+                                                      stream or torch.cuda.current_stream().cuda_stream), "paella_conv2d_launch_pooled")
     return y
 
 

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from test_conv_pool_gpu import pooled
 from test_ring_gpu import decode
 
 pytestmark = pytest.mark.gpu
@@ -210,6 +211,65 @@ def test_recorded_sequences_of_several_requests_go_out_together(ring, cuda):
     torch.cuda.synchronize()
     for a, b in zip(alone, outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kw", [2, 4, 8])
+def test_recorded_convs_with_their_pools_go_out_together(ring, cuda, kw):
+    """Eleven requests of a conv with its pool (two tiles of channels, eleven of windows) and a dense layer, eight and three to a launch."""
+    lib, h = ring
+    from paella_amd import ops
+    rng = np.random.default_rng(100 + kw)
+    hint = 1 << 20 | 0x110 | kw.bit_length() - 1
+
+    def net(height):
+        conv = ops.Conv2d(rng.standard_normal((20, 8, 3, 3)).astype(np.float32), rng.standard_normal(20).astype(np.float32), pad=1, act=ops.ACT_RELU,
+                          in_hw=(height, 9), tile_hint=hint)
+        outs = 20 * (height // 2) * 4
+        wd = torch.tensor(rng.standard_normal((10, outs)).astype(np.float32), device=cuda)
+        keep = []
+
+        def run(x, stream=None, job_id=0, notifier=None):
+            keep.append(pooled(ops, conv, x, (2, 2), stream) if stream else ops.pool2d(conv(x), 2, 2))
+            return keep[-1], ops.dense(keep[-1].reshape(1, outs), wd, stream=stream, job_id=job_id, notifier=notifier)
+        return run, [torch.tensor(rng.standard_normal((1, 8, height, 9)).astype(np.float32), device=cuda) for _ in range(11)]
+
+    tall, xs = net(23)
+    low, low_xs = net(8)
+    alone = [tall(x) for x in xs] + [low(x) for x in low_xs[:2]] + [tall(x) for x in xs[:2]]
+    torch.cuda.synchronize()
+    key = ctypes.c_void_p(0x1234)
+    outs = []
+
+    def record(run, x, q):
+        j = len(outs)
+        assert lib.paella_pack_sequence_begin(key, ctypes.c_void_p(q.handle)) == 0
+        outs.append(run(x, stream=q.handle, job_id=(j + 1) | NO_START, notifier=ctypes.c_void_p(lib.paella_ring_notifier(h, j))))
+        assert lib.paella_pack_sequence_end() == 0
+
+    with ops.DirectQueue(ordered=True) as q:
+        assert lib.paella_pack_enable(1) == 0
+        try:
+            before = stats(lib)
+            for x in xs:
+                record(tall, x, q)
+            assert held(lib) == 11 and lib.paella_pack_flush() == 4 and held(lib) == 0
+            after = stats(lib)
+            assert (after[0] - before[0], after[1] - before[1]) == (4, 22)
+            # under one key, but of another grid: they do not share a launch
+            for run, some in ((low, low_xs[:2]), (tall, xs[:2])):
+                for x in some:
+                    record(run, x, q)
+            assert held(lib) == 2 and lib.paella_pack_flush() == 2 and held(lib) == 0
+            assert stats(lib)[0] - after[0] == 4 and stats(lib)[1] - after[1] == 8
+            buf = np.zeros(15, np.uint64)
+            assert lib.paella_ring_drain(h, buf.ctypes.data, 15, 20.0) == 15
+            m = decode(buf)
+            assert sorted(m["job_id"]) == list(range(1, 16)) and np.all(m["num"] == 3) and np.all(m["is_start"] == 0)
+        finally:
+            lib.paella_pack_enable(0)
+    torch.cuda.synchronize()
+    for want, got in zip(alone, outs):
+        assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
 
 
 def test_convs_with_a_fused_input_transform_are_packed_among_themselves(ring, cuda):
