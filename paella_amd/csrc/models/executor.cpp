@@ -337,6 +337,11 @@ void mark_pooled(paella_model* m) {
         if (lc.count != 1 || lc.pool >= 0 || lp.count != 1 || lp.pool >= 0 || m->pre_of[lc.nodes[0]] >= 0) continue;
         const Node &c = g.nodes[lc.nodes[0]], &p = g.nodes[lp.nodes[0]];
         if (c.op != Op::Conv || p.op != Op::Pool || c.x2.buf >= 0 || !paella_conv2d_plan_takes_pool(&m->plans[lc.nodes[0]].conv, &p.pool)) continue;
+        // At most four chunks per wave, eight for windows that fill a tile, so that it is no loss in company either.  Time of the one launch over that of
+        // the two, up to 256 tiles, one pair at a time / four at once: one to four chunks 0.48 to 0.82 / 0.53 to 0.86; five to eight 0.79 to
+        // 1.03 / 1.01 to 1.35, windows of 4 x 4 0.68 to 0.75 / 0.72 to 0.82 (the two multiply on larger tiles, with fewer columns idle).
+        const paella_conv_plan& plan = m->plans[lc.nodes[0]].conv;
+        if ((plan.k_pad / 8 + plan.kw - 1) / plan.kw > (p.pool.R * p.pool.S == 16 ? 8 : 4)) continue;
         const View &v = c.y, &x = p.x;
         if (v.buf != x.buf || v.off != x.off || v.C != x.C || v.H != x.H || v.W != x.W) continue;
         bool ok = !overlap(v, g.output) && !overlap(p.y, c.x) && !overlap(p.y, v) && c.x.buf != g.output.buf;

@@ -160,3 +160,13 @@ def test_which_convs_of_a_graph_leave_their_output_unwritten(tmp_path, graph, pa
     count = len(models.launch_plan(model))
     issued = launches(model, [(0, count - 1, 0)])[0].split()
     assert issued[0] == "0" and issued[1:].count("pooled") == pairs and len(issued) - 1 == count - pairs
+
+
+@pytest.mark.parametrize("channels, window, want", [(24, 2, "pooled"), (32, 2, "0 1"), (24, 3, "pooled"), (56, 3, "0 1"), (32, 4, "pooled"), (56, 4, "pooled"), (64, 4, "0 1")])
+def test_convs_of_more_than_four_chunks_per_wave_keep_a_launch_of_their_own(tmp_path, channels, window, want):
+    """Unless the windows fill the tiles.  (Four, five, eight and nine chunks in each of eight waves.)"""
+    b = ow.Builder(np.random.default_rng(8))
+    y = pool(b, conv(b, "x", 32, channels), window)
+    path = str(tmp_path / "g.onnx")
+    b.save(path, [("x", [1, channels, 30, 30])], [(y, [1, 32, 30 // window, 30 // window])])
+    assert launches("onnx:" + path, [(0, 1, 0)]) == ["0 " + want]
