@@ -235,7 +235,8 @@ int paella_pool2d_launch(const paella_pool_desc* d, const float* x, float* y,
 
 /* A small conv and the maximum pooling behind it as ONE launch that reports to nobody; the conv's own output is not written.  Same bits as the two
  * operators.  Where paella_conv2d_plan_takes_pool() returns 1: windows side by side (stride = window of at most 4 x 4, no padding, the pool's
- * input the conv's output), a reduction that is not split and short, few tiles; PAELLA_ENOSUP, with nothing launched, otherwise and where x and y overlap. */
+ * input the conv's output), a reduction that is not split, of at most eight chunks of 8 per wave, and at most 256 workgroups of 16 channels and
+ * 16 / (R * S) windows each; PAELLA_ENOSUP, with nothing launched, otherwise and where x and y overlap. */
 int paella_conv2d_plan_takes_pool(const paella_conv_plan* plan, const paella_pool_desc* pool);
 /* Launch shape of the two as one launch, which has workgroups of its own; PAELLA_ENOSUP where they stay two. */
 int paella_conv2d_pooled_dims(const paella_conv_plan* plan, const paella_pool_desc* pool, paella_launch_dims* dims);

@@ -2920,12 +2920,13 @@ unsigned pooled_grid(const paella_conv_plan* plan, const paella_pool_desc* d) {
     if (d->R > 4 || d->S > 4) return 0;
     const int area = d->R * d->S, P = d->H / d->R, Q = d->W / d->S;
     if (area < 2 || P < 1 || Q < 1) return 0;
-    // Half of the columns at work, one workgroup per compute unit and a short reduction: beyond, the two launches gain from larger tiles what
-    // they lose on the way.
+    // One workgroup per compute unit and a short reduction: beyond, the two launches gain from larger tiles what they lose on the way.  Time of
+    // the one over that of the two, one pair at a time, windows of 2 x 2, 3 x 3 and 4 x 4: 144 to 256 tiles of eight chunks per wave 0.87, 1.03, 0.75, of nine 0.97,
+    // 1.08, 0.79, of fourteen 1.11, 1.26, 0.93; 288 tiles of seven chunks 1.09, 1.22, 0.85 (of four 0.77, 0.89, 0.64).
     const int wins = 16 / area;
     const long tiles = (((long)P * Q + wins - 1) / wins) * ((plan->d.K + 15) / 16);
     const int nchunks = plan->k_pad / 8;
-    return wins * area >= 8 && tiles <= 256 && (nchunks + plan->kw - 1) / plan->kw <= 8 ? (unsigned)tiles : 0u;
+    return tiles <= 256 && (nchunks + plan->kw - 1) / plan->kw <= 8 ? (unsigned)tiles : 0u;
 }
 
 }  // namespace
