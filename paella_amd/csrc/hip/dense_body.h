@@ -35,7 +35,6 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const int o, const
     const int I = a.I;
     const float* __restrict__ x = a.x;
     const float* __restrict__ wr = a.w + (size_t)o * I;
-    const float bias = a.bias ? a.bias[o] : 0.f;  // travels with the row: requested behind the sum it is a trip to memory of its own
     float acc = 0.f;
     if ((I & 3) == 0) {
         const float4* w4 = reinterpret_cast<const float4*>(wr);
@@ -62,7 +61,7 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const int o, const
     }
     acc = dense_wave_sum(acc);
     if (lane == 0) {
-        float v = acc + bias;
+        float v = acc + (a.bias ? a.bias[o] : 0.f);
         if (a.act == PAELLA_ACT_RELU) v = fmaxf(v, 0.f);
         else if (a.act == PAELLA_ACT_RELU6) v = fminf(fmaxf(v, 0.f), 6.f);
         store_out(a.y + o, v);

@@ -65,7 +65,6 @@ __global__ __launch_bounds__(512) void dense_long_kernel(const float* __restrict
     const int wave = threadIdx.x >> 6;
     const int o0 = blockIdx.x * 2;
     const int o1 = min(o0 + 1, O - 1);  // an odd O: the last workgroup reads its only row twice and stores it once
-    const float row_bias = bias && threadIdx.x < 2 && o0 + (int)threadIdx.x < O ? bias[o0 + threadIdx.x] : 0.f;  // travels with the rows
     const int I4 = I >> 2;
     const int per = (I4 + 7) >> 3;
     const int begin = wave * per;
@@ -101,7 +100,7 @@ __global__ __launch_bounds__(512) void dense_long_kernel(const float* __restrict
             float v = 0.f;
 #pragma unroll
             for (int k = 0; k < 8; ++k) v += part[threadIdx.x][k];
-            store_out(y + o, act_apply(v + row_bias, act, 0.f, 0.f, 0.f));
+            store_out(y + o, act_apply(v + (bias ? bias[o] : 0.f), act, 0.f, 0.f, 0.f));
         }
     }
     paella::hook_exit(notifier, job_id);
