@@ -7,10 +7,11 @@
 // (v_mfma_f32_16x16x4_f32, see conv_small.h) are not neighbouring pixels but whole windows -- four of 2x2, one of 3x3 and seven columns idle -- so the maximum
 // is taken across a wave's lanes and the conv's output is never written.  The launch is one workgroup per 16 channels and tile of windows, with the waves
 // and the chunks per wave of the conv's own plan: the bits are those of the conv's kernel and the pool's.
-// The small CNN (28x28, 5x5 convs of 8 and 16 channels, pools 2x2 and 3x3), five launches -> three: one request without a server 27.9 -> 24.1 us, a lone
-// client of the server 25.4 -> 19.8 us a request, 9 : 1 beside Inception-v3 under load 163.1 -> 159.7 ms.  What such a kernel takes is the chain of trips
-// in it: with the arguments in one round instead of six, bias and slope requested with the operands instead of behind the sum, no address arithmetic for
-// chunks that are not there and the two reduction orders apart 24.1 -> 23.1 and 19.8 -> 18.7 us.
+// The small CNN (28x28, 5x5 convs of 8 and 16 channels, pools 2x2 and 3x3), five launches -> three: one request without a server 27.9 -> 23.1 us, a lone
+// client of the server 25.4 -> 18.7 us a request.  What such a kernel takes is the chain of trips in it.  us a launch for its two convs, 2.51 and 4.04
+// now, and, in brackets, for a 1x1 8->16 on 48x48 with 2x2, 2.69: the arguments where they are used, six trips, 2.58 and 4.14 (2.75); bias
+// and slope behind the sum 2.54 and 4.07 (3.01); four chunks' addresses where there is one chunk 3.17 and 4.01 (3.01); one loop for both
+// reduction orders 2.50 and 4.15 (2.74); the maximum in a loop for windows of four and nine too 2.61 and 4.26 (2.91).
 
 struct ConvPoolArgs {
     const float* x;
