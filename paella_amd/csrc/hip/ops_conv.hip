@@ -2914,10 +2914,8 @@ namespace {
 unsigned pooled_grid(const paella_conv_plan* plan, const paella_pool_desc* d) {
     if (!plan || !d || plan->kind != 0 || plan->mi != 1 || plan->ni != 1 || plan->depth || plan->pair_taps || plan->splits != 1 || plan->small != 1 || !plan->fast_div) return 0;
     if (plan->kw != 2 && plan->kw != 4 && plan->kw != 8) return 0;
-    paella::PoolArgs pa;  // what the pool's own launch would refuse is refused here too
-    if (!paella::pool_fill_args(d, nullptr, nullptr, 0, nullptr, &pa)) return 0;
     if (d->is_avg || d->pad_h || d->pad_w || d->ceil_mode || d->stride_h != d->R || d->stride_w != d->S || d->C != plan->d.K || d->H != plan->P || d->W != plan->Q) return 0;
-    if (d->R > 4 || d->S > 4) return 0;
+    if (d->R < 1 || d->S < 1 || d->R > 4 || d->S > 4) return 0;
     const int area = d->R * d->S, P = d->H / d->R, Q = d->W / d->S;
     if (area < 2 || P < 1 || Q < 1) return 0;
     // One workgroup per compute unit and a short reduction: beyond, the two launches gain from larger tiles what they lose on the way.  Time of
