@@ -812,7 +812,7 @@ static int launch_all(paella_exec* e, void* stream) { return paella_exec_launch_
 int paella_exec_forward(paella_exec* e, void* stream) {
     if (!e) return PAELLA_EINVAL;
     // From the fourth pass on, in company, a graph of at least kMinGraph kernels is replayed (to record it costs as
-    // much as three passes' launches; a pass of five kernels is slower as a graph, 49 against 26 us).
+    // much as three passes' launches; the small CNN's pass, of five kernels then, was slower as a graph, 49 against 26 us).
     bool replay = false;
     constexpr size_t kMinGraph = 16;
     constexpr unsigned kPlainPasses = 3;
