@@ -91,3 +91,52 @@ def test_input_and_output_in_the_same_memory(cuda, tmp_path):
         torch.cuda.synchronize()
         assert torch.equal(same, apart)
     ex.close()
+
+
+def test_pairs_in_replayed_passes(cuda, tmp_path):
+    """Two pairs in a pass that is long enough for a graph: recorded and replayed on several streams, the bits of the stages one by one."""
+    import _onnx_writer as ow
+    from paella_amd import models
+    from test_exec_io_gpu import plain
+    b = ow.Builder(np.random.default_rng(9))
+
+    def conv(x, k, c, r):
+        return b.op("Relu", [b.op("Conv", [x, b.const(b.randn(k, c, r, r, scale=1.0 / np.sqrt(c) / r)), b.const(b.randn(k))], kernel_shape=[r, r], pads=[r // 2] * 4)])
+    y = b.op("MaxPool", [conv("x", 8, 1, 5)], kernel_shape=[2, 2], strides=[2, 2])
+    y = b.op("MaxPool", [conv(y, 16, 8, 5)], kernel_shape=[3, 3], strides=[3, 3])
+    for _ in range(14):
+        y = conv(y, 16, 16, 1)
+    b.save(str(tmp_path / "chain.onnx"), [("x", [1, 1, 28, 28])], [(y, [1, 16, 4, 4])])
+    name = "onnx:" + str(tmp_path / "chain.onnx")
+    assert len(models.launch_plan(name)) == 18
+    rng = np.random.default_rng(10)
+    xs = [rng.standard_normal(784).astype(np.float32) for _ in range(2)]
+    want = [plain(name, x) for x in xs]
+    assert not np.array_equal(*want)
+    execs, streams = [models.Exec(name) for _ in range(4)], [torch.cuda.Stream() for _ in range(2)]
+    other = torch.zeros(1 << 16, device=cuda)
+    for turn in range(8):
+        for i, ex in enumerate(execs):
+            ex.set_input(xs[(i + turn) % 2])
+            ex.forward(streams[i % 2].cuda_stream)
+        other += 1
+        for s in streams:
+            s.synchronize()
+        for i, ex in enumerate(execs):
+            np.testing.assert_array_equal(ex.get_output(), want[(i + turn) % 2])
+    for ex in execs:
+        ex.close()
+
+
+@pytest.mark.parametrize("limit", ["6400", "8192", "65536"])
+def test_served_with_pairs_within_the_limit_of_small_kernels_and_beyond(cuda, monkeypatch, limit):
+    """The small CNN under load with none, one and both of its pairs as one launch: every answer as that of the idle server, and that the oracle's."""
+    from paella_amd import models, serve
+    from test_verify_gpu import expectations_match_the_oracle, run_verified, server_name
+    monkeypatch.setenv("LLIS_MODEL_SEED", "1")
+    monkeypatch.setenv("PAELLA_GROUP_THREADS", limit)
+    types = [("mnist", "tvm_mnist", 1.0, 48)]
+    with serve.Server(server_name("pairs"), "full3", num_streams=32, extra_kernels=32) as srv:
+        r, out_bytes = run_verified(serve, models, srv, types, 0.0, 3000, seed=5)
+    assert r["mismatches"] == 0
+    expectations_match_the_oracle(models, types, r, out_bytes, 5)
